@@ -23,10 +23,13 @@
 //     XOR-swizzled with row & 3, read with ds_read_b64_tr_b16);
 //   * each wave owns a 128 x 64 (or 64 x 64) sub-tile as 32 x 32 v_mfma_f32_32x32x16_bf16 tiles
 //     with fp32 accumulation;
-//   * the epilogue moves tiles between the "lane owns a column" accumulator layout and the
-//     "lane owns a row" layout with two MFMAs against a permuted identity, so that the addend is
-//     read and the outputs are written with wide, coalesced accesses staged through wave-private
-//     LDS.
+//   * the MFMAs take the second operand first, so a lane's accumulators are columns of one row of the
+//     tile: the epilogue's arithmetic is lane-local, results are staged once in wave-private LDS and
+//     leave it as whole rows (C) and, through transposing reads, as whole columns (the mirror image
+//     CT), with wide coalesced stores.  Against accumulators that are rows of one column (moved
+//     between the two layouts with MFMAs against an identity) the kernels need 220 instead of 256
+//     vector registers and: GPT-2-124M step 2.14 -> 2.11 ms, 24 x (768 x 3072) products with one rounding
+//     0.239 -> 0.222 ms.
 #include <stdlib.h>
 
 #include "common.h"
@@ -54,9 +57,9 @@ __device__ __forceinline__ u32x2 gload8(const uint16_t* p) {
 // the operand panels measured +0.5 % on the Llama step (and a loss for GPT-2-size matrices, whose
 // outputs the next launch does find in L2, so the small class stores normally).
 template <bool STREAM>
-__device__ __forceinline__ void gstore16(uint16_t* p, u32x4 v) {
-    if constexpr (STREAM) __builtin_nontemporal_store(v, (__attribute__((address_space(1))) u32x4*)(p));
-    else *(__attribute__((address_space(1))) u32x4*)(p) = v;
+__device__ __forceinline__ void bstore16(const uint16_t* base, uint32_t voff, uint32_t soff, u32x4 v) {
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, 0xffffffff, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, static_cast<int>(voff), static_cast<int>(soff), STREAM ? 2 : 0);
 }
 
 constexpr int BK = 64;   // k extent of one ring stage (128 bytes per LDS row)
@@ -148,48 +151,40 @@ __device__ __forceinline__ void wait_frags_tr(u32x4 (&a)[TM], u32x2 (&b)[TN2]) {
 // ---------------------------------------------------------------------------------------------
 // Epilogue helpers
 // ---------------------------------------------------------------------------------------------
-// out = V^T for a 32 x 32 tile of bf16-representable values held in accumulator layout (lane =
-// column l%32, register 4q+e = row 8q + 4(l/32) + e).  V goes in as the A operand; id0/id1 are the
-// B operands with B[slot][j] = (row(slot) == j), where slot (g, t) of k-block h carries tile row
-// 16h + 8(t/4) + 4g + t%4 -- exactly the rows registers 8h .. 8h+7 hold.  bf16 x 1.0 products and
-// sums of a single non-zero term are exact in the fp32 accumulator.
-__device__ __forceinline__ f32x16 tile_transpose_bf16(const float (&v)[16], bf16x8 id0, bf16x8 id1) {
-    bf16x8 f0, f1;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        f0[t] = static_cast<__bf16>(v[t]);
-        f1[t] = static_cast<__bf16>(v[8 + t]);
-    }
-    f32x16 z;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = 0.f;
-    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0, id0, z, 0, 0, 0);
-    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1, id1, z, 0, 0, 0);
-    return z;
+// Result strips go through wave-private LDS, 32 rows of WN bf16 columns at a time, as 16-byte chunks;
+// chunk c of row r sits at position c ^ f(r).  f spreads both the 16-byte accesses of 8 consecutive
+// rows and the transposing reads of 4 rows x 16 columns over all banks.
+template <int WN>
+__device__ __forceinline__ uint32_t strip_pos(int r, int c) {
+    static_assert(WN == 64 || WN == 32, "strip_pos: rows of 8 or 4 chunks");
+    const int f = WN == 64 ? (((r & 3) << 1) | ((r >> 2) & 1)) : ((r & 2) | ((r >> 2) & 1));
+    return static_cast<uint32_t>(r * WN * 2 + ((c ^ f) << 4));
 }
 
-// The same for a tile already packed two bf16 per register (p[k] = values 2k, 2k+1).
-__device__ __forceinline__ f32x16 tile_transpose_packed(const uint32_t (&p)[8], bf16x8 id0, bf16x8 id1) {
-    const bf16x8 f0 = __builtin_bit_cast(bf16x8, u32x4{p[0], p[1], p[2], p[3]});
-    const bf16x8 f1 = __builtin_bit_cast(bf16x8, u32x4{p[4], p[5], p[6], p[7]});
-    f32x16 z;
+// One 32 x 32 tile of packed bf16 pairs (lane = row l % 32, pair 2q + i = columns 8q + 4 (l / 32) + 2i) into
+// columns 32b .. of the strip: the halves of two neighbouring 8-column chunks are exchanged between
+// lanes l and l + 32, so that every lane holds 8 consecutive columns and writes them at once.
+template <int WN>
+__device__ __forceinline__ void strip_write(char* stage, int lr, int g, int b, const uint32_t (&po)[8]) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = 0.f;
-    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0, id0, z, 0, 0, 0);
-    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1, id1, z, 0, 0, 0);
-    return z;
+    for (int q = 0; q < 4; q += 2) {
+        const auto x = __builtin_amdgcn_permlane32_swap(po[2 * q], po[2 * q + 2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(po[2 * q + 1], po[2 * q + 3], false, false);
+        *reinterpret_cast<u32x4*>(stage + strip_pos<WN>(lr, b * 4 + q + g)) = u32x4{x[0], y[0], x[1], y[1]};
+    }
 }
 
-// bf16(gamma * x) for 8 packed bf16 values.
-__device__ __forceinline__ u32x4 scale_bf16x8(u32x4 v, float gamma) {
-    u32x4 r;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float lo = gamma * __uint_as_float(v[k] << 16);
-        const float hi = gamma * __uint_as_float(v[k] & 0xffff0000u);
-        r[k] = pack2bf(lo, hi);
-    }
-    return r;
+// 8 consecutive rows of one column of the strip: lane l takes column s * 16 + l % 16, rows 8 (l / 16) .. + 7,
+// by two transposing reads of 4 rows x 16 columns each (see FragLoadTr for what a lane addresses).
+template <int WN>
+__device__ __forceinline__ u32x4 strip_read_transposed(const char* stage, int lane, int s) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const int r = (lane >> 4) * 8 + ((lane & 15) >> 2), c = s * 2 + ((lane & 3) >> 1), half = (lane & 1) * 8;
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const auto lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(stage + strip_pos<WN>(r, c) + half));
+    const auto hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(stage + strip_pos<WN>(r + 4, c) + half));
+    const u32x2 l = __builtin_bit_cast(u32x2, lo), h = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l.x, l.y, h.x, h.y};
 }
 
 // The parameter step fused into the epilogue of the last update product (muon.py:14, 98-99):
@@ -303,29 +298,27 @@ __device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const
     }
 }
 
-// Wave-private staging bytes of the result strips: one 32-row strip in the direct orientation, then
-// (in the same place) the strip's WN rows of 32 columns in the transposed one; rows padded by 16 B.
-constexpr int strip_stage_bytes(int WN) {
-    return 32 * (WN * 2 + 16) > WN * (32 * 2 + 16) ? 32 * (WN * 2 + 16) : WN * (32 * 2 + 16);
-}
+// Wave-private staging bytes of the result strips: 32 rows of WN columns, twice (the scaled copy, or
+// the strip after).
+constexpr int strip_stage_bytes(int WN) { return 2 * 32 * WN * 2; }
 
-// Per 32-row strip of the wave's sub-tile, per 32 x 32 tile of it: t1 = alpha*acc -> row-owning
-// layout -> + beta*D -> o (bf16) -> staged row-major in LDS -> 16-byte coalesced stores of C (and
-// gamma*o to C2); o moved back to the column-owning layout -> staged -> 16-byte coalesced stores
-// of CT (and C2T).  With APPLY, the orientation of the parameter goes through the fused parameter
-// step instead of a store, and the other orientation is not produced.  `stage` is this wave's
-// strip_stage_bytes(WN) of LDS.
+// Per 32-row strip of the wave's sub-tile: the accumulators hold rows (lane l: 16 columns of row l % 32 per
+// 32 x 32 tile), so t1 = alpha*acc, + beta*D -> o (bf16) is lane-local; o is staged row-major in LDS and
+// read back as whole rows (16-byte coalesced stores of C) and, through transposing LDS reads, as whole
+// columns (16-byte stores of CT); gamma*o likewise to C2 / C2T.  With APPLY, the orientation of the
+// parameter goes through the fused parameter step instead of a store, and the other orientation is
+// not produced.  `stage` is this wave's strip_stage_bytes(WN) of LDS.
 // ROWSUM (a mirrored product without addend): per row of the result, the sum of |o| over the
-// wave's 64 columns goes to d.rowsum[row][col0 / 64]; for a mirrored tile the column sums over the
-// wave's WM rows go to the rows of the mirror image, d.rowsum[col][row0 / 64] (and zero to the other
+// wave's WN columns goes to d.rowsum[row][col0 / WN]; for a mirrored tile the column sums over the
+// wave's WM rows go to the rows of the mirror image, d.rowsum[col][row0 / WN] (and zero to the other
 // slots of those WM rows), so that every slot of every row is written exactly once per launch.
-template <bool HAS_D, bool STREAM, bool APPLY, bool ROWSUM, int WGN, int WM, int WN, int TM, int TN>
+template <bool HAS_D, bool STREAM, bool APPLY, bool ROUND, bool ROWSUM, int WGN, int WM, int WN, int TM, int TN>
 __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const u32x2 (&dv)[TM][TN][4],
                                                    const MuonGemmDesc& d, const MuonTileJob& job, float alpha,
-                                                   float beta, float gamma, bool round_terms, char* stage,
-                                                   const ApplyArgs& ap) {
-    constexpr int DROW = WN * 2 + 16;   // staged row pitch in bytes, direct orientation (32 rows)
-    constexpr int TROW = 32 * 2 + 16;   // transposed orientation (WN rows of one strip's 32 columns)
+                                                   float beta, float gamma, char* stage, const ApplyArgs& ap) {
+    constexpr int SBYTES = 32 * WN * 2;
+    constexpr int CPR = WN / 8, RPI = 64 / CPR;       // direct: chunks per row, rows per wave-wide access
+    constexpr int CB = WN / 16;                       // transposed: blocks of 16 columns
     // The thread index goes through an opaque move here: everything the epilogue derives from it
     // is then computed after the main loop instead of being hoisted above it, where it would sit
     // in registers the loop needs (and be spilled to scratch memory by every wave).
@@ -339,177 +332,118 @@ __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const 
     const bool apply_t = APPLY && ap.mat->rows > ap.mat->cols;
     const bool do_d = APPLY ? !apply_t : d.C != nullptr;
     const bool do_t = APPLY ? apply_t : (d.CT != nullptr && !(job.diag && d.CT == d.C));
+    const bool do_2 = !APPLY && (d.C2 != nullptr || d.C2T != nullptr);
+    // Stores go through buffer resources based at the sub-tile's corner: the lane's offset is the same
+    // for every access of an orientation, rows are stepped in the scalar offset.
+    const uint32_t voff_d = static_cast<uint32_t>(lane / CPR) * static_cast<uint32_t>(d.ldc) * 2u + (lane % CPR) * 16u;
+    const uint32_t voff_t = static_cast<uint32_t>(lane & 15) * static_cast<uint32_t>(d.ldct) * 2u + (lane >> 4) * 16u;
+    const size_t base_d = static_cast<size_t>(row0) * d.ldc + col0, base_t = static_cast<size_t>(col0) * d.ldct + row0;
 
-    bf16x8 id0, id1;
+    float colsum[CB];          // ROWSUM: |o| summed down this lane's rows of every strip, per block of 16 columns
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const int rho = 8 * (t >> 2) + 4 * g + (t & 3);
-        id0[t] = static_cast<__bf16>(rho == lr ? 1.0f : 0.0f);
-        id1[t] = static_cast<__bf16>(16 + rho == lr ? 1.0f : 0.0f);
-    }
-
-    float colsum[TN];          // ROWSUM: |o| summed down this lane's 16 rows of every strip, per column tile
-#pragma unroll
-    for (int b = 0; b < TN; ++b) colsum[b] = 0.f;
+    for (int s = 0; s < CB; ++s) colsum[s] = 0.f;
 #pragma unroll
     for (int a = 0; a < TM; ++a) {
-        uint32_t ot[TN][8];   // this strip's results moved back to accumulator layout, packed bf16 pairs
-        float rowpart = 0.f;  // ROWSUM: |o| summed along this lane's 32 of the strip's 64 columns
+        // a strip with a scaled copy fills both halves of the staging space; else strips alternate
+        char* const st = stage + ((!do_2 && (a & 1)) ? SBYTES : 0);
+        char* const st2 = stage + SBYTES;
+        float rowpart = 0.f;  // ROWSUM: |o| summed along this lane's half of the strip's columns
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            if (round_terms) {
-                // Every term rounded to bf16 as the reference's tensor expressions round.  Values
-                // stay packed two bf16 per register from the conversion that rounds them: the pairs
-                // are what the transposing MFMAs, the staging stores and the next conversion take.
-                uint32_t p1[8];       // bf16(alpha * acc), accumulator layout
+            uint32_t po[8];
+            if constexpr (ROUND || !HAS_D) {
+                // bf16(alpha * acc).  alpha is 1 in every product of the iteration: not multiplying
+                // then saves one of about six vector instructions per element
+                if (alpha == 1.f) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) p1[k] = pack2bf(alpha * acc[a][b][2 * k], alpha * acc[a][b][2 * k + 1]);
-                const f32x16 u = tile_transpose_packed(p1, id0, id1);
-                uint32_t po[8];       // o = bf16(u + bf16(beta * D)), row-owning layout
+                    for (int k = 0; k < 8; ++k) po[k] = pack2bf(acc[a][b][2 * k], acc[a][b][2 * k + 1]);
+                } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (HAS_D) {
-                        const uint32_t t01 = pack2bf(beta * bf_lo(dv[a][b][q].x), beta * bf_hi(dv[a][b][q].x));
-                        const uint32_t t23 = pack2bf(beta * bf_lo(dv[a][b][q].y), beta * bf_hi(dv[a][b][q].y));
-                        po[2 * q] = pack2bf(u[4 * q] + bf_lo(t01), u[4 * q + 1] + bf_hi(t01));
-                        po[2 * q + 1] = pack2bf(u[4 * q + 2] + bf_lo(t23), u[4 * q + 3] + bf_hi(t23));
-                    } else {          // u holds bf16 values: exact
-                        po[2 * q] = pack2bf(u[4 * q], u[4 * q + 1]);
-                        po[2 * q + 1] = pack2bf(u[4 * q + 2], u[4 * q + 3]);
-                    }
-                    if constexpr (ROWSUM) {       // one term after the other, in column order
-                        rowpart += fabsf(bf_lo(po[2 * q]));
-                        rowpart += fabsf(bf_hi(po[2 * q]));
-                        rowpart += fabsf(bf_lo(po[2 * q + 1]));
-                        rowpart += fabsf(bf_hi(po[2 * q + 1]));
-                    }
-                    if (do_d)
-                        *reinterpret_cast<u32x2*>(stage + lr * DROW + (b * 32 + 8 * q + 4 * g) * 2) =
-                            u32x2{po[2 * q], po[2 * q + 1]};
+                    for (int k = 0; k < 8; ++k) po[k] = pack2bf(alpha * acc[a][b][2 * k], alpha * acc[a][b][2 * k + 1]);
                 }
-                if (do_t) {
-                    if (HAS_D) {
-                        const f32x16 w = tile_transpose_packed(po, id0, id1);
+            }
+            if constexpr (HAS_D) {
 #pragma unroll
-                        for (int k = 0; k < 8; ++k) ot[b][k] = pack2bf(w[2 * k], w[2 * k + 1]);
-                    } else {
-                        // without an addend o is the transposed t1, and its transpose is t1 again
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) ot[b][k] = p1[k];
-                        if constexpr (ROWSUM) {
-#pragma unroll
-                            for (int k = 0; k < 8; ++k) {
-                                colsum[b] += fabsf(bf_lo(p1[k]));
-                                colsum[b] += fabsf(bf_hi(p1[k]));
-                            }
-                        }
+                for (int k = 0; k < 8; ++k) {
+                    const uint32_t dk = (k & 1) ? dv[a][b][k / 2].y : dv[a][b][k / 2].x;
+                    if constexpr (ROUND) {       // every term rounded to bf16 as the reference's tensor expressions round
+                        const uint32_t t2 = pack2bf(beta * bf_lo(dk), beta * bf_hi(dk));
+                        po[k] = pack2bf(bf_lo(po[k]) + bf_lo(t2), bf_hi(po[k]) + bf_hi(t2));
+                    } else {                     // one rounding of the finished expression
+                        po[k] = pack2bf(fmaf(alpha, acc[a][b][2 * k], beta * bf_lo(dk)),
+                                        fmaf(alpha, acc[a][b][2 * k + 1], beta * bf_hi(dk)));
                     }
                 }
-                continue;
             }
-            // One rounding per output: keep ~16 mantissa bits of alpha * acc through the transpose by
-            // moving a bf16 head and a bf16 tail and adding them.
-            f32x16 u;
-            {
-                float hi[16], lo[16];
+            if constexpr (ROWSUM) {       // one term after the other, in column order
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float v = alpha * acc[a][b][i];
-                    hi[i] = round_bf(v);
-                    lo[i] = round_bf(v - hi[i]);
-                }
-                const f32x16 uh = tile_transpose_bf16(hi, id0, id1);
-                const f32x16 ul = tile_transpose_bf16(lo, id0, id1);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) u[i] = uh[i] + ul[i];
-            }
-            float o[16];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float dd[4] = {0.f, 0.f, 0.f, 0.f};
-                if (HAS_D) {
-                    dd[0] = bf_lo(dv[a][b][q].x);
-                    dd[1] = bf_hi(dv[a][b][q].x);
-                    dd[2] = bf_lo(dv[a][b][q].y);
-                    dd[3] = bf_hi(dv[a][b][q].y);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    o[4 * q + e] = round_bf(u[4 * q + e] + (HAS_D ? beta * dd[e] : 0.f));
-                    if constexpr (ROWSUM) rowpart += fabsf(o[4 * q + e]);
-                }
-                if (do_d) {
-                    u32x2 pk;
-                    pk.x = pack2bf(o[4 * q], o[4 * q + 1]);
-                    pk.y = pack2bf(o[4 * q + 2], o[4 * q + 3]);
-                    *reinterpret_cast<u32x2*>(stage + lr * DROW + (b * 32 + 8 * q + 4 * g) * 2) = pk;
+                for (int k = 0; k < 8; ++k) {
+                    rowpart += fabsf(bf_lo(po[k]));
+                    rowpart += fabsf(bf_hi(po[k]));
                 }
             }
-            if (do_t) {
-                const f32x16 w = tile_transpose_bf16(o, id0, id1);
+            strip_write<WN>(st, lr, g, b, po);
+            if (do_2) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) ot[b][k] = pack2bf(w[2 * k], w[2 * k + 1]);
-                if constexpr (ROWSUM) {
-#pragma unroll
-                    for (int k = 0; k < 16; ++k) colsum[b] += fabsf(w[k]);
-                }
+                for (int k = 0; k < 8; ++k) po[k] = pack2bf(gamma * bf_lo(po[k]), gamma * bf_hi(po[k]));
+                strip_write<WN>(st2, lr, g, b, po);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (ROWSUM) {
-            // the partner lane (l ^ 32) owns the other 32 columns of the same row
+            // the partner lane (l ^ 32) owns the other columns of the same row
             const float total = rowpart + __shfl_xor(rowpart, 32, 64);
-            if (g == 0)
-                d.rowsum[static_cast<size_t>(row0 + a * 32 + lr) * d.ld_rowsum + col0 / 64] = total;
+            if (g == 0 && d.rowsum)
+                d.rowsum[static_cast<size_t>(row0 + a * 32 + lr) * d.ld_rowsum + col0 / WN] = total;
         }
         if (do_d) {
-            // 16-byte chunks per row, whole rows per wave-wide store
-            constexpr int CPR = WN / 8, RPI = 64 / CPR;
-            const int r = lane / CPR, ch = lane % CPR;
             if constexpr (APPLY) {
 #pragma unroll 1
                 for (int it = 0; it < 32 / RPI; ++it) {
-                    const int row = it * RPI + r;
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * DROW + ch * 16);
-                    apply_chunk8(ap, row0 + a * 32 + row, col0 + ch * 8, v);
+                    const int row = it * RPI + lane / CPR;
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(st + strip_pos<WN>(row, lane % CPR));
+                    apply_chunk8(ap, row0 + a * 32 + row, col0 + (lane % CPR) * 8, v);
                 }
             } else {
 #pragma unroll
                 for (int it = 0; it < 32 / RPI; ++it) {
-                    const int row = it * RPI + r;
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * DROW + ch * 16);
-                    const size_t off = static_cast<size_t>(row0 + a * 32 + row) * d.ldc + col0 + ch * 8;
-                    gstore16<STREAM>(d.C + off, v);
-                    if (d.C2) gstore16<STREAM>(d.C2 + off, scale_bf16x8(v, gamma));
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(st + strip_pos<WN>(it * RPI + lane / CPR, lane % CPR));
+                    bstore16<STREAM>(d.C + base_d, voff_d, (a * 32 + it * RPI) * static_cast<uint32_t>(d.ldc) * 2u, v);
+                }
+                if (d.C2) {
+#pragma unroll
+                    for (int it = 0; it < 32 / RPI; ++it) {
+                        const u32x4 v = *reinterpret_cast<const u32x4*>(st2 + strip_pos<WN>(it * RPI + lane / CPR, lane % CPR));
+                        bstore16<STREAM>(d.C2 + base_d, voff_d, (a * 32 + it * RPI) * static_cast<uint32_t>(d.ldc) * 2u, v);
+                    }
                 }
             }
         }
         if (do_t) {
-#pragma unroll
-            for (int b = 0; b < TN; ++b)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    u32x2 pk;
-                    pk.x = ot[b][2 * q];
-                    pk.y = ot[b][2 * q + 1];
-                    *reinterpret_cast<u32x2*>(stage + (b * 32 + lr) * TROW + (8 * q + 4 * g) * 2) = pk;
-                }
-            constexpr int CPR = 32 / 8, RPI = 64 / CPR;
-            const int r = lane / CPR, ch = lane % CPR;
             if constexpr (APPLY) {
 #pragma unroll 1
-                for (int it = 0; it < WN / RPI; ++it) {
-                    const int row = it * RPI + r;
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * TROW + ch * 16);
-                    apply_chunk8(ap, col0 + row, row0 + a * 32 + ch * 8, v);
+                for (int s = 0; s < CB; ++s) {
+                    const u32x4 v = strip_read_transposed<WN>(st, lane, s);
+                    apply_chunk8(ap, col0 + s * 16 + (lane & 15), row0 + a * 32 + (lane >> 4) * 8, v);
                 }
             } else {
 #pragma unroll
-                for (int it = 0; it < WN / RPI; ++it) {
-                    const int row = it * RPI + r;
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * TROW + ch * 16);
-                    const size_t off = static_cast<size_t>(col0 + row) * d.ldct + row0 + a * 32 + ch * 8;
-                    gstore16<STREAM>(d.CT + off, v);
-                    if (d.C2T) gstore16<STREAM>(d.C2T + off, scale_bf16x8(v, gamma));
+                for (int s = 0; s < CB; ++s) {
+                    const u32x4 v = strip_read_transposed<WN>(st, lane, s);
+                    if constexpr (ROWSUM) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            colsum[s] += fabsf(bf_lo(v[k]));
+                            colsum[s] += fabsf(bf_hi(v[k]));
+                        }
+                    }
+                    bstore16<STREAM>(d.CT + base_t, voff_t, s * 16 * static_cast<uint32_t>(d.ldct) * 2u + a * 64, v);
+                }
+                if (d.C2T) {
+#pragma unroll
+                    for (int s = 0; s < CB; ++s)
+                        bstore16<STREAM>(d.C2T + base_t, voff_t, s * 16 * static_cast<uint32_t>(d.ldct) * 2u + a * 64,
+                                         strip_read_transposed<WN>(st2, lane, s));
                 }
             }
         }
@@ -517,14 +451,15 @@ __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const 
     if constexpr (ROWSUM) {
         if (do_t) {
 #pragma unroll
-            for (int b = 0; b < TN; ++b) {
-                // the partner lane owns the other 16 rows of every strip of the same column
-                const float total = colsum[b] + __shfl_xor(colsum[b], 32, 64);
-                if (g == 0) {
-                    float* const dst = d.rowsum + static_cast<size_t>(col0 + b * 32 + lr) * d.ld_rowsum + row0 / 64;
+            for (int s = 0; s < CB; ++s) {
+                // lanes l, l + 16, l + 32, l + 48 own 8 rows each of every strip of the same column
+                float total = colsum[s] + __shfl_xor(colsum[s], 16, 64);
+                total += __shfl_xor(total, 32, 64);
+                if (lane < 16 && d.rowsum) {
+                    float* const dst = d.rowsum + static_cast<size_t>(col0 + s * 16 + lane) * d.ld_rowsum + row0 / WN;
                     dst[0] = total;
 #pragma unroll
-                    for (int z = 1; z < WM / 64; ++z) dst[z] = 0.f;
+                    for (int z = 1; z < WM / WN; ++z) dst[z] = 0.f;
                 }
             }
         }
@@ -590,10 +525,11 @@ struct GemmCfg {
 // QK: the second operand is given k-major, Q[k][j] with leading dimension ldq (acc[i][j] = sum_k
 // P[i][k] Q[k][j]: the update a X + B X reads X itself, no transposed copy of it exists); its
 // half-stage is then BK rows of BN columns, fetched in the same 1 KiB pieces.
-template <typename Cfg, bool APPLY, bool QK>
+// ROUND: MUON_AMD_ROUND_REFERENCE; ROWSUM: MUON_AMD_GEMM_ROWSUM.
+template <typename Cfg, bool APPLY, bool QK, bool ROUND, bool ROWSUM>
 __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     const MuonGemmDesc* __restrict__ descs, const MuonTileJob* __restrict__ jobs, int njobs, float alpha,
-    float beta, float gamma, int flags, float* __restrict__ split_partials,
+    float beta, float gamma, float* __restrict__ split_partials,
     int32_t* __restrict__ split_counters, const MuonMatDesc* __restrict__ mats, float neg_lr,
     float wd_factor, const float* __restrict__ sc) {
     constexpr int NW = Cfg::NW, WGN = Cfg::WGN, WM = Cfg::WM, WN = Cfg::WN;
@@ -601,6 +537,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     constexpr int NHALF = Cfg::NHALF, NPRE = Cfg::NPRE;
     constexpr int ROWQ = Cfg::BN * 2;           // bytes of one k-row of a k-major Q half-stage
     static_assert(!APPLY || QK, "the parameter step rides the update product, whose second operand is k-major");
+    static_assert(!ROWSUM || !QK, "row sums belong to X X^T");
     extern __shared__ __align__(16) uint16_t lds[];
     const int tid = threadIdx.x;
     const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
@@ -669,7 +606,6 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     static_assert(KSTEPS % 2 == 0, "the fragments read at a block's last k-step land in buffer 0");
     static_assert(DPK <= TM, "one DMA instruction per row of MFMAs");
 
-    const bool round_terms = (flags & MUON_AMD_ROUND_REFERENCE) != 0;
     if constexpr (APPLY) {
         if (sc) {
             neg_lr = -sc[0];
@@ -816,8 +752,9 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
                     u32x4 qv;                                                                  \
                     if constexpr (QK) qv = u32x4{btr[cur][2 * b].x, btr[cur][2 * b].y, btr[cur][2 * b + 1].x, btr[cur][2 * b + 1].y}; \
                     else qv = bfr[cur][b];                                                     \
+                    /* Q first: a lane then holds 16 columns of one row of the tile */         \
                     acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                       \
-                        __builtin_bit_cast(bf16x8, af[cur][a]), __builtin_bit_cast(bf16x8, qv), acc[a][b], 0, 0, 0); \
+                        __builtin_bit_cast(bf16x8, qv), __builtin_bit_cast(bf16x8, af[cur][a]), acc[a][b], 0, 0, 0); \
                 }                                                                              \
                 if (a < DPK) {                                                                 \
                     /* instruction jj of the current pair: the last k-step starts a pair */    \
@@ -933,7 +870,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         }
 
         // ---- epilogue, first part: the addend into registers (staged at the start of the ring) ----
-        const bool has_d = APPLY || d.D != nullptr;
+        const bool has_d = APPLY || (!ROWSUM && d.D != nullptr);
         u32x2 dv[TM][TN][4];
         if (write_tile && has_d) {
             ns_epilogue_addend<WGN, WM, WN, TM, TN>(dv, d, job, reinterpret_cast<const char*>(lds) + wave * (WM * 128));
@@ -974,11 +911,12 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
                 ap.wd_factor = wd_factor;
                 ap.vec_ok = (ap.mat->cols % 8 == 0) && ((reinterpret_cast<uintptr_t>(ap.mat->param) & 15) == 0) &&
                             ((reinterpret_cast<uintptr_t>(ap.mat->out) & 15) == 0);
-                ns_epilogue_strips<true, Cfg::STREAM_STORES, true, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, round_terms, stage, ap);
+                ns_epilogue_strips<true, Cfg::STREAM_STORES, true, ROUND, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, stage, ap);
+            } else if constexpr (ROWSUM) {
+                ns_epilogue_strips<false, Cfg::STREAM_STORES, false, false, true, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, stage, ap);
             } else {
-                if (has_d) ns_epilogue_strips<true, Cfg::STREAM_STORES, false, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, round_terms, stage, ap);
-                else if ((flags & MUON_AMD_GEMM_ROWSUM) && d.rowsum) ns_epilogue_strips<false, Cfg::STREAM_STORES, false, true, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, round_terms, stage, ap);
-                else ns_epilogue_strips<false, Cfg::STREAM_STORES, false, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, round_terms, stage, ap);
+                if (has_d) ns_epilogue_strips<true, Cfg::STREAM_STORES, false, ROUND, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, stage, ap);
+                else ns_epilogue_strips<false, Cfg::STREAM_STORES, false, false, false, WGN, WM, WN, TM, TN>(acc, dv, d, job, alpha, beta, gamma, stage, ap);
             }
         }
         if (!has_next) break;
@@ -1059,9 +997,9 @@ struct DeviceState {
 static DeviceState g_devices[kMaxDevices];
 static std::mutex g_devices_mutex;
 
-template <typename Cfg, bool APPLY, bool QK>
+template <typename Cfg, bool APPLY, bool QK, bool ROUND, bool ROWSUM>
 static int raise_lds_limit() {
-    auto kern = ns_gemm_kernel<Cfg, APPLY, QK>;
+    auto kern = ns_gemm_kernel<Cfg, APPLY, QK, ROUND, ROWSUM>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(Cfg::LDS_BYTES)) != hipSuccess) {
         (void)hipGetLastError();
@@ -1069,6 +1007,18 @@ static int raise_lds_limit() {
         return MUON_AMD_ELAUNCH;
     }
     return MUON_AMD_OK;
+}
+
+template <typename Cfg>
+static int raise_lds_limits() {
+    int rc = raise_lds_limit<Cfg, false, false, true, false>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, false, false, false>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, false, false, true>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, true, true, false>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, true, false, false>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, true, true, true, false>();
+    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, true, true, false, false>();
+    return rc;
 }
 
 static int device_setup(const DeviceState** out) {
@@ -1095,12 +1045,8 @@ static int device_setup(const DeviceState** out) {
             set_error("device %d is %s: this library holds gfx950 (MI355X) code only", dev, prop.gcnArchName);
             return MUON_AMD_EDEVICE;
         }
-        int rc = raise_lds_limit<Cfg0, false, false>();
-        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg0, false, true>();
-        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg0, true, true>();
-        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg1, false, false>();
-        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg1, false, true>();
-        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg1, true, true>();
+        int rc = raise_lds_limits<Cfg0>();
+        if (rc == MUON_AMD_OK) rc = raise_lds_limits<Cfg1>();
         if (rc != MUON_AMD_OK) return rc;
         void* ptr = nullptr;
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || ptr == nullptr) {
@@ -1129,18 +1075,23 @@ static int launch_gemm(const DeviceState& st, const MuonGemmDesc* descs, const M
     // as many workgroups as the GPU holds at once; each walks its share of the job list
     const int resident = st.num_cus * Cfg::MINB;
     const int grid = njobs < resident ? njobs : resident;
-    if (ap.mats)
-        hipLaunchKernelGGL((ns_gemm_kernel<Cfg, true, true>), dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, s, descs, jobs,
-                           njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap.mats, ap.neg_lr,
-                           ap.wd_factor, ap.scalars);
-    else if (flags & MUON_AMD_GEMM_Q_KMAJOR)
-        hipLaunchKernelGGL((ns_gemm_kernel<Cfg, false, true>), dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, s, descs, jobs,
-                           njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap.mats, ap.neg_lr,
-                           ap.wd_factor, ap.scalars);
-    else
-        hipLaunchKernelGGL((ns_gemm_kernel<Cfg, false, false>), dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, s, descs, jobs,
-                           njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap.mats, ap.neg_lr,
-                           ap.wd_factor, ap.scalars);
+    const bool round = (flags & MUON_AMD_ROUND_REFERENCE) != 0;
+    const auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::NT), Cfg::LDS_BYTES, s, descs, jobs, njobs, alpha, beta, gamma,
+                           split_partials, split_counters, ap.mats, ap.neg_lr, ap.wd_factor, ap.scalars);
+    };
+    if (ap.mats) {
+        if (round) go(ns_gemm_kernel<Cfg, true, true, true, false>);
+        else go(ns_gemm_kernel<Cfg, true, true, false, false>);
+    } else if (flags & MUON_AMD_GEMM_Q_KMAJOR) {
+        if (round) go(ns_gemm_kernel<Cfg, false, true, true, false>);
+        else go(ns_gemm_kernel<Cfg, false, true, false, false>);
+    } else if (flags & MUON_AMD_GEMM_ROWSUM) {
+        go(ns_gemm_kernel<Cfg, false, false, false, true>);
+    } else {
+        if (round) go(ns_gemm_kernel<Cfg, false, false, true, false>);
+        else go(ns_gemm_kernel<Cfg, false, false, false, false>);
+    }
     return check_launch("ns_gemm");
 }
 
