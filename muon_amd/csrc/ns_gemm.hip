@@ -85,19 +85,6 @@ __device__ __forceinline__ void dma16(u32x4 rsrc, uint32_t voff, uint32_t soff, 
 // s_waitcnt vmcnt(n) only (expcnt / lgkmcnt left unconstrained); n < 64 (bits 3:0 and 15:14).
 #define NS_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 
-// Wait until at most min(n, H) half-stages (DPH DMA instructions each) of this wave are pending.
-template <int DPH, int H>
-struct WaitHalves {
-    static __device__ __forceinline__ void run(int n) {
-        if (n >= H) NS_WAIT_VMCNT(H * DPH);
-        else WaitHalves<DPH, H - 1>::run(n);
-    }
-};
-template <int DPH>
-struct WaitHalves<DPH, 0> {
-    static __device__ __forceinline__ void run(int) { NS_WAIT_VMCNT(0); }
-};
-
 // Fragment reads of the main loop: N ds_read_b128 from LDS byte address addr + i * 32 rows, issued
 // through inline assembly so that the waits for them can be placed by hand (wait_frags).
 template <int N, int I = 0>
@@ -485,9 +472,6 @@ template <int BT_, int WGM_, int WGN_, int MINB_, int NHALF_, bool SPLIT_K_>
 struct GemmCfg {
     static constexpr bool SPLIT_K = SPLIT_K_;     // jobs may share a tile's reduction
     static constexpr bool STREAM_STORES = BT_ >= 256;   // see gstore16
-    // A second copy of the k-block without the tests of the first and last blocks (see NS_KBLOCK).
-    // The 256 x 256 class has no registers to spare for the moves between two copies of its loop.
-    static constexpr bool STEADY_LOOP = BT_ < 256;
     static constexpr int BM = BT_, BN = BT_, WGM = WGM_, WGN = WGN_, MINB = MINB_, NHALF = NHALF_;
     static constexpr int NW = WGM * WGN, NT = NW * 64;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
@@ -657,7 +641,8 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         // Block 0 has landed once only the younger first halves are pending (for a job after the
         // first, halves 0 .. NPRE-1 landed long ago and at most NHALF - NPRE are pending).
-        WaitHalves<DPH, NHALF - 2>::run((2 * nk < NHALF ? 2 * nk : NHALF) - 2);
+        if (2 * nk >= NHALF) NS_WAIT_VMCNT((NHALF - 2) * DPH);
+        else NS_WAIT_VMCNT(0);
         __syncthreads();
 
         // Fragments are double buffered over k-steps ACROSS blocks: the ds_reads of the next k-step
@@ -701,96 +686,100 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         uint32_t ddst[2] = {0, 0};
         uint32_t dk[2] = {0, 0};           // byte offset of the k-block being fetched, per half of the pair
         const uint32_t dstep[2] = {(NHALF & 1) ? qstep : static_cast<uint32_t>(BK * 2), (NHALF & 1) ? static_cast<uint32_t>(BK * 2) : qstep};
-        bool dgo[2] = {false, false};
 
-        // One k-block.  STEADY_: a block in the middle of a long reduction -- both halves of the pair
-        // created at the previous barrier and the first half of the pair created at this one exist
-        // (1 <= kb <= nk - 3), so every DMA instruction is issued without a test and the wait before
-        // the barrier is a constant; the first block and the last two take the general form.
-#define NS_KBLOCK(STEADY_)                                                                      \
+        // One k-block, MORE_ = how many follow it (2 stands for two or more).  With two or more to follow every
+        // half of the pairs created at this barrier and at the one before exists, so no transfer sits
+        // behind a test and the wait before the barrier is a constant; with one to follow only the first
+        // half of the older pair exists, and the last block fetches nothing.
+        // The barrier stands in the middle of the last k-step's MFMAs: all fragments of the block are in
+        // registers by then, and the matrix pipe works on the first rows while the waves meet.
+        // What bounds the loop is the matrix pipe (2048 clocks per block of a 256 x 256 tile).  With tests at
+        // every transfer and the barrier ahead of the k-step a block took 2630-2700 clocks; in this form
+        // 2230-2290 (32 x 4096^2 Newton-Schulz 41.0 -> 38.5 ms, one 768 x 3072 matrix 326 -> 293 us).
+        // (Transfers of half-stages beyond the end must not be issued, not even against an empty
+        // resource: they corrupted the ring now and then.)
+#define NS_MFMA_ROW(a_, cur_)                                                                   \
+    do {                                                                                       \
+        _Pragma("unroll") for (int b = 0; b < TN; ++b) {                                       \
+            u32x4 qv;                                                                          \
+            if constexpr (QK) qv = u32x4{btr[cur_][2 * b].x, btr[cur_][2 * b].y, btr[cur_][2 * b + 1].x, btr[cur_][2 * b + 1].y}; \
+            else qv = bfr[cur_][b];                                                            \
+            /* Q first: a lane then holds 16 columns of one row of the tile */                 \
+            acc[a_][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                              \
+                __builtin_bit_cast(bf16x8, qv), __builtin_bit_cast(bf16x8, af[cur_][a_]), acc[a_][b], 0, 0, 0); \
+        }                                                                                      \
+    } while (0)
+        /* instruction jj_ of the current pair */
+#define NS_PAIR_DMA(jj_)                                                                        \
+    do {                                                                                       \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+        dma16(drsrc[(jj_) / DPH], dsrc[(jj_) / DPH][(jj_) % DPH], dk[(jj_) / DPH], ddst[(jj_) / DPH] + ((jj_) % DPH) * NW * 1024); \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+    } while (0)
+#define NS_KBLOCK(MORE_)                                                                        \
     do {                                                                                       \
         int spn = sp + 2; spn = spn >= NHALF ? spn - NHALF : spn;                              \
         int sqn = sq + 2; sqn = sqn >= NHALF ? sqn - NHALF : sqn;                              \
-        _Pragma("unroll") for (int ks = 0; ks < KSTEPS; ++ks) {                                \
+        _Pragma("unroll") for (int ks = 0; ks + 1 < KSTEPS; ++ks) {                            \
             const int cur = ks & 1, nxt = cur ^ 1;                                             \
-            if (ks + 1 < KSTEPS) {                                                             \
-                NS_LOAD_FRAGS(nxt, sp, sq, ks + 1);                                            \
-                NS_WAIT_FRAGS(NFRAG, cur);                                                     \
-            } else {                                                                           \
-                /* Every fragment of block kb is in registers.  Block kb+1 has landed once only   \
-                   the younger halves are pending; after the barrier it is visible to all waves   \
-                   and the two slots of block kb are free for the next pair of halves,            \
-                   2kb+NHALF and 2kb+NHALF+1. */                                                  \
-                NS_WAIT_FRAGS(0, cur);                                                         \
-                if (STEADY_ || kb + 1 < nk) {                                                  \
-                    if (STEADY_) {                                                             \
-                        NS_WAIT_VMCNT((NHALF - 4) * DPH);                                      \
-                    } else {                                                                   \
-                        const int issued = 2 * nk < 2 * kb + NHALF ? 2 * nk : 2 * kb + NHALF;  \
-                        WaitHalves<DPH, NHALF - 2>::run(issued - (2 * kb + 4));                \
-                    }                                                                          \
-                    __builtin_amdgcn_s_barrier();                                              \
-                    const int h0 = 2 * kb + NHALF;                                             \
-                    ddst[0] = dst0 + sp * HALF_BYTES;            /* h0 % NHALF == 2kb % NHALF */  \
-                    ddst[1] = dst0 + sq * HALF_BYTES;                                          \
-                    dk[0] = static_cast<uint32_t>(h0 >> 1) * dstep[0];                         \
-                    dk[1] = static_cast<uint32_t>((h0 + 1) >> 1) * dstep[1];                   \
-                    dgo[0] = h0 < 2 * nk;                                                      \
-                    dgo[1] = h0 + 1 < 2 * nk;                                                  \
-                } else {                                                                       \
-                    dgo[0] = dgo[1] = false;     /* last block: nothing left to fetch */       \
-                }                                                                              \
-                /* The first fragments of block kb+1, read under the last MFMAs of block kb.      \
-                   After the last block the same reads go out and their result is not used: the   \
-                   fragment registers then have one definition on every path, so the compiler has \
-                   no reason to copy them while the reads are in flight. */                       \
-                NS_LOAD_FRAGS(nxt, spn, sqn, 0);                                               \
-            }                                                                                  \
+            NS_LOAD_FRAGS(nxt, sp, sq, ks + 1);                                                \
+            NS_WAIT_FRAGS(NFRAG, cur);                                                         \
             __builtin_amdgcn_sched_barrier(0);   /* keep these reads ahead of the MFMAs below */  \
             _Pragma("unroll") for (int a = 0; a < TM; ++a) {                                   \
-                _Pragma("unroll") for (int b = 0; b < TN; ++b) {                               \
-                    u32x4 qv;                                                                  \
-                    if constexpr (QK) qv = u32x4{btr[cur][2 * b].x, btr[cur][2 * b].y, btr[cur][2 * b + 1].x, btr[cur][2 * b + 1].y}; \
-                    else qv = bfr[cur][b];                                                     \
-                    /* Q first: a lane then holds 16 columns of one row of the tile */         \
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                       \
-                        __builtin_bit_cast(bf16x8, qv), __builtin_bit_cast(bf16x8, af[cur][a]), acc[a][b], 0, 0, 0); \
-                }                                                                              \
-                if (a < DPK) {                                                                 \
-                    /* instruction jj of the current pair: the last k-step starts a pair */    \
-                    const int jj = (ks + 1 < KSTEPS ? (ks + 1) * DPK : 0) + a;                 \
-                    const int h = jj / DPH, j = jj % DPH;                                      \
-                    __builtin_amdgcn_sched_barrier(0);                                         \
-                    if (STEADY_ || dgo[h]) dma16(drsrc[h], dsrc[h][j], dk[h], ddst[h] + j * NW * 1024); \
-                    __builtin_amdgcn_sched_barrier(0);                                         \
-                }                                                                              \
+                NS_MFMA_ROW(a, cur);                                                           \
+                if (a < DPK && kb > 0 && ((MORE_) == 2 || ((MORE_) == 1 && (ks + 1) * DPK + a < DPH))) \
+                    NS_PAIR_DMA((ks + 1) * DPK + a);                                           \
             }                                                                                  \
             __builtin_amdgcn_sched_barrier(0);                                                 \
         }                                                                                      \
+        constexpr int cur = (KSTEPS - 1) & 1, nxt = cur ^ 1;                                   \
+        NS_WAIT_FRAGS(0, cur);                                                                 \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+        _Pragma("unroll") for (int a = 0; a < TM / 2; ++a) NS_MFMA_ROW(a, cur);                \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+        if ((MORE_) > 0) {                                                                     \
+            /* Block kb+1 has landed once only the younger halves are pending; after the barrier  \
+               it is visible to all waves and the two slots of block kb are free for the next     \
+               pair of halves, 2kb+NHALF and 2kb+NHALF+1.  (With one block to follow nothing      \
+               younger than it was issued.) */                                                    \
+            NS_WAIT_VMCNT((MORE_) == 2 ? (NHALF - 4) * DPH : 0);                               \
+            __builtin_amdgcn_s_barrier();                                                      \
+            const int h0 = 2 * kb + NHALF;                                                     \
+            ddst[0] = dst0 + sp * HALF_BYTES;            /* h0 % NHALF == 2kb % NHALF */          \
+            ddst[1] = dst0 + sq * HALF_BYTES;                                                  \
+            dk[0] = static_cast<uint32_t>(h0 >> 1) * dstep[0];                                 \
+            dk[1] = static_cast<uint32_t>((h0 + 1) >> 1) * dstep[1];                           \
+            NS_LOAD_FRAGS(nxt, spn, sqn, 0);   /* the first fragments of block kb+1 */         \
+            __builtin_amdgcn_sched_barrier(0);                                                 \
+        }                                                                                      \
+        _Pragma("unroll") for (int a = TM / 2; a < TM; ++a) {                                  \
+            NS_MFMA_ROW(a, cur);                                                               \
+            if ((MORE_) == 2) {                                                                \
+                _Pragma("unroll") for (int jj = 0; jj < DPK; ++jj)                             \
+                    if (jj * (TM - TM / 2) / DPK == a - TM / 2) NS_PAIR_DMA(jj);               \
+            }                                                                                  \
+        }                                                                                      \
         /* Nothing is in flight across the end of a k-block: the reads issued before the last     \
-           row of MFMAs have long arrived, and waiting for them here keeps every pending          \
+           rows of MFMAs have long arrived, and waiting for them here keeps every pending         \
            fragment inside one copy of this code (a register the compiler moved at a loop edge    \
-           or between the two copies would be moved before its data is there). */                 \
-        NS_WAIT_FRAGS(0, 0);                                                                   \
+           would be moved before its data is there). */                                        \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+        if ((MORE_) > 0) NS_WAIT_FRAGS(0, 0);                                                  \
         sp = spn;                                                                              \
         sq = sqn;                                                                              \
     } while (0)
 
         int sp = 0, sq = 1;                 // ring slots of the P and Q halves of block kb
-        for (int kb = 0; kb < nk;) {
-            if constexpr (Cfg::STEADY_LOOP) {
-                if (kb >= 1 && kb <= nk - 3) {
-                    do {
-                        NS_KBLOCK(true);
-                        ++kb;
-                    } while (kb <= nk - 3);
-                    continue;
-                }
-            }
-            NS_KBLOCK(false);
+        int kb = 0;
+        for (; kb < nk - 2; ++kb) NS_KBLOCK(2);
+        if (nk > 1) {
+            NS_KBLOCK(1);
             ++kb;
         }
+        NS_KBLOCK(0);
 #undef NS_KBLOCK
+#undef NS_PAIR_DMA
+#undef NS_MFMA_ROW
 #undef NS_WAIT_FRAGS
 #undef NS_LOAD_FRAGS
         __syncthreads();            // every wave is done reading the ring: LDS becomes staging space
