@@ -128,7 +128,9 @@ typedef struct MuonTileJob {
     int32_t desc;      /* index into the MuonGemmDesc table of the launch */
     int32_t i0;        /* first output row  (multiple of the tile rows)   */
     int32_t j0;        /* first output col  (multiple of the tile cols)   */
-    int32_t diag;      /* 1 when a mirrored (symmetric) GEMM's tile lies in a diagonal block */
+    int32_t diag;      /* mirrored (symmetric) GEMM: 1 when the tile lies in a diagonal block, 2 for
+                          another tile that is stored but not mirrored (the job list then also holds
+                          the tile of its mirror image); 0 otherwise                           */
     int32_t k0, k1;    /* reduction range of this job, multiples of 64; 0 and K when unsplit */
     int32_t part_base; /* first slot of the tile's split group (also its counter); unused when unsplit */
     int32_t split;     /* 0 when unsplit, else index | (count << 16) */

@@ -101,7 +101,7 @@ struct FragLoad {
 // on rows 8..11, two such reads (rows +0 and +4) leave lane l with k = 8 (l / 32) .. + 7 of column
 // l % 32: exactly the second operand of v_mfma_f32_32x32x16_bf16 (checked on the device).
 // f[2 i], f[2 i + 1]: the two halves of fragment i; addr[i]: its per-lane LDS byte address (the
-// 64-byte column blocks of a row are XOR-swizzled with row & 3, so it depends on i).
+// column blocks of a row are XOR-swizzled with row & 3, so it depends on i).
 template <int N, int ROWQ, int I = 0>
 struct FragLoadTr {
     static __device__ __forceinline__ void run(u32x2 (&f)[2 * N], const uint32_t (&addr)[N], uint32_t base) {
@@ -120,6 +120,8 @@ __device__ __forceinline__ void wait_frags(u32x4 (&a)[TM], u32x4 (&b)[TN]) {
         asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]) : "n"(CNT));
     else if constexpr (TM == 2 && TN == 2)
         asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]) : "n"(CNT));
+    else if constexpr (TM == 1 && TN == 1)
+        asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a[0]), "+v"(b[0]) : "n"(CNT));
     else
         static_assert(TM == 2 && TN == 2, "wait_frags: add the operand list of this wave tile");
 }
@@ -131,6 +133,8 @@ __device__ __forceinline__ void wait_frags_tr(u32x4 (&a)[TM], u32x2 (&b)[TN2]) {
                      "+v"(b[2]), "+v"(b[3]) : "n"(CNT));
     else if constexpr (TM == 2 && TN2 == 4)
         asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]) : "n"(CNT));
+    else if constexpr (TM == 1 && TN2 == 2)
+        asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(a[0]), "+v"(b[0]), "+v"(b[1]) : "n"(CNT));
     else
         static_assert(TM == 2 && TN2 == 4, "wait_frags_tr: add the operand list of this wave tile");
 }
@@ -247,14 +251,15 @@ __device__ __forceinline__ void apply_chunk8(const ApplyArgs& ap, int prow, int 
 // The addend: the lane that owns row (a*32 + lr) needs columns b*32 + 8q + 4g .. +4 of it.  Fetched
 // that way from global memory, every load instruction would touch 32 different rows for 16 bytes
 // each and the address pipe would take longer than the whole rest of the epilogue.  So the wave's
-// WM x 64 piece of D is first streamed into its staging area `stage_d` (WM rows of 128 bytes) by
-// the DMA path, one instruction per 8 full rows (chunks XOR-swizzled as in the operand ring), and
+// WM x WN piece of D is first streamed into its staging area `stage_d` (WM rows of 2 WN bytes) by
+// the DMA path, one instruction per 1 KiB of full rows (chunks XOR-swizzled as in the operand ring), and
 // the row-owning 8-byte pieces are read from LDS.  All of them are in registers when this returns:
 // before any store of the sub-tile (D may alias C: in-place a*X + B*X).
 template <int WGN, int WM, int WN, int TM, int TN>
 __device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const MuonGemmDesc& d,
                                                    const MuonTileJob& job, const char* stage_d) {
-    static_assert(WN == 64, "the addend staging assumes 128-byte rows");
+    constexpr int CPR = WN / 8, RPI = 64 / CPR;         // chunks per row, rows per instruction
+    static_assert(WM % RPI == 0, "addend staging in whole instructions");
     int tid_e = threadIdx.x;
     asm volatile("" : "+v"(tid_e));            // see ns_epilogue_strips
     const int lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
@@ -263,12 +268,11 @@ __device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const
     const int row0 = job.i0 + wm * WM, col0 = job.j0 + wn * WN;
     const uint32_t stage_lds = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
         reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)stage_d)));
-    const int drow = lane >> 3;                         // row within the 8 rows of one instruction
     const u32x4 rsrc_d = dma_resource(d.D);
 #pragma unroll
-    for (int j = 0; j < WM / 8; ++j) {
-        const int rr = j * 8 + drow;
-        const int lc = (lane & 7) ^ ((rr >> 1) & 7);    // logical 16-byte chunk this lane fetches
+    for (int j = 0; j < WM / RPI; ++j) {
+        const int rr = j * RPI + lane / CPR;
+        const int lc = (lane % CPR) ^ ((rr >> 1) & (CPR - 1));    // logical 16-byte chunk this lane fetches
         dma16(rsrc_d, static_cast<uint32_t>((static_cast<size_t>(row0 + rr) * d.ldd + col0 + lc * 8) * 2), 0u,
               stage_lds + j * 1024);
     }
@@ -281,7 +285,7 @@ __device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 dv[a][b][q] = *reinterpret_cast<const u32x2*>(
-                    stage_d + rr * 128 + (((b * 4 + q) ^ ((rr >> 1) & 7)) * 16) + g * 8);
+                    stage_d + rr * WN * 2 + (((b * 4 + q) ^ ((rr >> 1) & (CPR - 1))) * 16) + g * 8);
     }
 }
 
@@ -428,9 +432,10 @@ __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const 
                 }
                 if (d.C2T) {
 #pragma unroll
-                    for (int s = 0; s < CB; ++s)
-                        bstore16<STREAM>(d.C2T + base_t, voff_t, s * 16 * static_cast<uint32_t>(d.ldct) * 2u + a * 64,
+                    for (int s = 0; s < CB; ++s) {
+                            bstore16<STREAM>(d.C2T + base_t, voff_t, s * 16 * static_cast<uint32_t>(d.ldct) * 2u + a * 64,
                                          strip_read_transposed<WN>(st2, lane, s));
+                    }
                 }
             }
         }
@@ -484,7 +489,7 @@ struct GemmCfg {
     // workgroup's next job are fetched into slots 0 .. NPRE-1 while the result strips are staged
     // behind them.
     static constexpr int NPRE = 3;
-    static constexpr size_t ADDEND_BYTES = static_cast<size_t>(NW) * WM * 128;
+    static constexpr size_t ADDEND_BYTES = static_cast<size_t>(NW) * WM * WN * 2;
     static constexpr size_t STRIP_OFFSET = static_cast<size_t>(NPRE) * HALF_BYTES;
     static constexpr size_t STRIP_BYTES = strip_stage_bytes(WN);
     static_assert(ADDEND_BYTES <= RING_BYTES, "addend staging");
@@ -520,6 +525,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     constexpr int TM = Cfg::TM, TN = Cfg::TN, HALF_BYTES = Cfg::HALF_BYTES, DPH = Cfg::DPH;
     constexpr int NHALF = Cfg::NHALF, NPRE = Cfg::NPRE;
     constexpr int ROWQ = Cfg::BN * 2;           // bytes of one k-row of a k-major Q half-stage
+    constexpr int QBLK = ROWQ >= 256 ? 64 : 32; // bytes of its swizzled blocks
     static_assert(!APPLY || QK, "the parameter step rides the update product, whose second operand is k-major");
     static_assert(!ROWSUM || !QK, "row sums belong to X X^T");
     extern __shared__ __align__(16) uint16_t lds[];
@@ -541,8 +547,9 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     const int gchunk = (lane & 7) ^ (((wave & 1) << 2) | (lane >> 4));                         \
     const uint32_t dst0 = lds_base + wave * 1024
     // k-major Q: piece (j*NW + wave) of the half-stage is 1024 / ROWQ whole k-rows; lane -> k-row
-    // and 16-byte position in it; the 64-byte block at position pb of row k holds the row's block
-    // pb ^ (k & 3) (the transposing fragment reads of four consecutive k then hit different banks).
+    // and 16-byte position in it; the block at position pb of row k holds the row's block pb ^ (k & 3)
+    // (the transposing fragment reads of four consecutive k then hit different banks): blocks of 64
+    // bytes, or of 32 in a row of four of those.
     uint32_t srcp[DPH];                         // per-lane byte offsets of this wave's pieces in P and Q
     uint32_t srcq[DPH];
     u32x4 rsrc_p, rsrc_q;                       // (wave-uniform: they live in scalar registers)
@@ -555,7 +562,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             if constexpr (QK) {                                                                \
                 const int o_ = (j_ * NW + wave) * 1024 + lane * 16;                            \
                 const int k_ = o_ / ROWQ, w_ = o_ % ROWQ;                                      \
-                const int col_ = (((w_ >> 6) ^ (k_ & 3)) << 5) + ((w_ & 63) >> 1);             \
+                const int col_ = (((w_ / QBLK) ^ (k_ & 3)) * (QBLK / 2)) + ((w_ % QBLK) >> 1);  \
                 srcq[j_] = static_cast<uint32_t>((static_cast<size_t>((job_).k0 + k_) * (d_).ldq + (job_).j0 + col_) * 2); \
             } else {                                                                           \
                 srcq[j_] = static_cast<uint32_t>((static_cast<size_t>((job_).j0 + r_) * (d_).ldq + (job_).k0 + gchunk * 8) * 2); \
@@ -623,8 +630,9 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             const int r4 = (lane & 15) >> 2;
 #pragma unroll
             for (int b = 0; b < TN; ++b)
-                qtr_off[b] = ((lane >> 5) * 8 + r4) * ROWQ + (((wn * (WN / 32) + b) ^ r4) << 6) +
-                             ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+                qtr_off[b] = ((lane >> 5) * 8 + r4) * ROWQ + (lane & 3) * 8 +
+                             (QBLK == 64 ? (((wn * (WN / 32) + b) ^ r4) * 64 + ((lane >> 4) & 1) * 32)
+                                         : (((wn * (WN / 32) + b) * 2 + ((lane >> 4) & 1)) ^ r4) * 32);
         }
         const int koff[4] = {c0 * 16, (c0 ^ 2) * 16, (c0 ^ 4) * 16, (c0 ^ 6) * 16};
         // the sources of the halves beyond the first ones (set again: the copies made when the
@@ -680,17 +688,19 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         // 2*DPH DMA instructions are spread over that k-step and the first KSTEPS-1 of block kb+1,
         // one after each of the first DPK rows of MFMAs -- a burst right after the barrier would hold
         // every wave in the memory-issue queue while the matrix pipe sits idle.
-        // NHALF odd: the first half of a pair is a Q half (needed one block earlier), the second P.
-        const uint32_t* const dsrc[2] = {(NHALF & 1) ? srcq : srcp, (NHALF & 1) ? srcp : srcq};
-        const u32x4 drsrc[2] = {(NHALF & 1) ? rsrc_q : rsrc_p, (NHALF & 1) ? rsrc_p : rsrc_q};
+        // The first half of a pair is a Q half (needed one block earlier), the second P.
+        const uint32_t* const dsrc[2] = {srcq, srcp};
+        const u32x4 drsrc[2] = {rsrc_q, rsrc_p};
         uint32_t ddst[2] = {0, 0};
+        constexpr int RING = (NHALF - 1) / 2;   // whole k-blocks in the ring beside the one that is multiplied
+        static_assert(NHALF % 2 == 1, "the first half of a pair is a Q half");
         uint32_t dk[2] = {0, 0};           // byte offset of the k-block being fetched, per half of the pair
-        const uint32_t dstep[2] = {(NHALF & 1) ? qstep : static_cast<uint32_t>(BK * 2), (NHALF & 1) ? static_cast<uint32_t>(BK * 2) : qstep};
+        const uint32_t dstep[2] = {qstep, static_cast<uint32_t>(BK * 2)};
 
-        // One k-block, MORE_ = how many follow it (2 stands for two or more).  With two or more to follow every
-        // half of the pairs created at this barrier and at the one before exists, so no transfer sits
-        // behind a test and the wait before the barrier is a constant; with one to follow only the first
-        // half of the older pair exists, and the last block fetches nothing.
+        // One k-block, MORE_ = how many follow it (RING stands for RING or more).  With RING or more to follow,
+        // every half of the pairs created at this barrier and at the one before exists, so no transfer sits
+        // behind a test and the wait before the barrier is a constant; with one fewer only the first half of
+        // the older pair exists, and the blocks after that fetch nothing.
         // The barrier stands in the middle of the last k-step's MFMAs: all fragments of the block are in
         // registers by then, and the matrix pipe works on the first rows while the waves meet.
         // What bounds the loop is the matrix pipe (2048 clocks per block of a 256 x 256 tile).  With tests at
@@ -727,7 +737,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             __builtin_amdgcn_sched_barrier(0);   /* keep these reads ahead of the MFMAs below */  \
             _Pragma("unroll") for (int a = 0; a < TM; ++a) {                                   \
                 NS_MFMA_ROW(a, cur);                                                           \
-                if (a < DPK && kb > 0 && ((MORE_) == 2 || ((MORE_) == 1 && (ks + 1) * DPK + a < DPH))) \
+                if (a < DPK && kb > 0 && ((MORE_) == RING || ((MORE_) == RING - 1 && (ks + 1) * DPK + a < DPH))) \
                     NS_PAIR_DMA((ks + 1) * DPK + a);                                           \
             }                                                                                  \
             __builtin_amdgcn_sched_barrier(0);                                                 \
@@ -740,9 +750,8 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         if ((MORE_) > 0) {                                                                     \
             /* Block kb+1 has landed once only the younger halves are pending; after the barrier  \
                it is visible to all waves and the two slots of block kb are free for the next     \
-               pair of halves, 2kb+NHALF and 2kb+NHALF+1.  (With one block to follow nothing      \
-               younger than it was issued.) */                                                    \
-            NS_WAIT_VMCNT((MORE_) == 2 ? (NHALF - 4) * DPH : 0);                               \
+               pair of halves, 2kb+NHALF and 2kb+NHALF+1. */                                      \
+            NS_WAIT_VMCNT(((MORE_) == RING ? NHALF - 4 : (MORE_) > 0 ? 2 * (MORE_) - 2 : 0) * DPH); \
             __builtin_amdgcn_s_barrier();                                                      \
             const int h0 = 2 * kb + NHALF;                                                     \
             ddst[0] = dst0 + sp * HALF_BYTES;            /* h0 % NHALF == 2kb % NHALF */          \
@@ -754,7 +763,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         }                                                                                      \
         _Pragma("unroll") for (int a = TM / 2; a < TM; ++a) {                                  \
             NS_MFMA_ROW(a, cur);                                                               \
-            if ((MORE_) == 2) {                                                                \
+            if ((MORE_) == RING) {                                                             \
                 _Pragma("unroll") for (int jj = 0; jj < DPK; ++jj)                             \
                     if (jj * (TM - TM / 2) / DPK == a - TM / 2) NS_PAIR_DMA(jj);               \
             }                                                                                  \
@@ -771,12 +780,16 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         int sp = 0, sq = 1;                 // ring slots of the P and Q halves of block kb
         int kb = 0;
-        for (; kb < nk - 2; ++kb) NS_KBLOCK(2);
-        if (nk > 1) {
-            NS_KBLOCK(1);
-            ++kb;
+        for (; kb < nk - RING; ++kb) NS_KBLOCK(RING);
+        if constexpr (RING > 3) {
+            if (nk - kb == 4) { NS_KBLOCK(3); ++kb; }
         }
+        if constexpr (RING > 2) {
+            if (nk - kb == 3) { NS_KBLOCK(2); ++kb; }
+        }
+        if (nk - kb == 2) { NS_KBLOCK(1); ++kb; }
         NS_KBLOCK(0);
+        static_assert(RING >= 2 && RING <= 4, "one copy of the block for each of the last RING");
 #undef NS_KBLOCK
 #undef NS_PAIR_DMA
 #undef NS_MFMA_ROW
@@ -787,7 +800,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         const int next_idx = job_idx + static_cast<int>(gridDim.x);
         const bool has_next = next_idx < njobs;
 
-        // ---- split reduction (small tile class only): a tile whose K range is shared by `count`
+        // ---- split reduction (not the 256 x 256 class): a tile whose K range is shared by `count`
         //      jobs.  Each job parks its fp32 accumulators in its own slot; the job that arrives last
         //      adds the slots in slot order (so the sum does not depend on which job that is) and
         //      writes the tile.  Nobody waits for anybody: the other jobs go on to their next job.
@@ -862,7 +875,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         const bool has_d = APPLY || (!ROWSUM && d.D != nullptr);
         u32x2 dv[TM][TN][4];
         if (write_tile && has_d) {
-            ns_epilogue_addend<WGN, WM, WN, TM, TN>(dv, d, job, reinterpret_cast<const char*>(lds) + wave * (WM * 128));
+            ns_epilogue_addend<WGN, WM, WN, TM, TN>(dv, d, job, reinterpret_cast<const char*>(lds) + wave * (WM * WN * 2));
         } else {
             // defined on every path, so that nothing of it is carried around the job loop in registers
 #pragma unroll
@@ -943,13 +956,19 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 // Tile classes: square output tile, waves, workgroups per CU.
 //   0: 128 x 128, 4 waves of 64 x 64, two workgroups per CU   (short side below 1024)
 //   1: 256 x 256, 8 waves of 128 x 64, one workgroup per CU   (large matrices)
+//   2: 64 x 64, 4 waves of 32 x 32, two workgroups per CU     (launches whose larger tiles leave CUs idle)
 #ifndef NS_CFG0_MINB
 #define NS_CFG0_MINB 2
 #define NS_CFG0_NHALF 5
 #endif
 typedef GemmCfg<128, 2, 2, NS_CFG0_MINB, NS_CFG0_NHALF, true> Cfg0;
 typedef GemmCfg<256, 2, 4, 1, 5, false> Cfg1;
-constexpr int kNumTileClasses = 2;
+#ifndef NS_CFG2_MINB
+#define NS_CFG2_MINB 2
+#define NS_CFG2_NHALF 9
+#endif
+typedef GemmCfg<64, 2, 2, NS_CFG2_MINB, NS_CFG2_NHALF, true> Cfg2;
+constexpr int kNumTileClasses = 3;
 
 struct TileClass {
     int bm, bn, threads;
@@ -959,6 +978,7 @@ struct TileClass {
 static const TileClass kTileClasses[kNumTileClasses] = {
     {Cfg0::BM, Cfg0::BN, Cfg0::NT, Cfg0::LDS_BYTES, Cfg0::SPLIT_K},
     {Cfg1::BM, Cfg1::BN, Cfg1::NT, Cfg1::LDS_BYTES, Cfg1::SPLIT_K},
+    {Cfg2::BM, Cfg2::BN, Cfg2::NT, Cfg2::LDS_BYTES, Cfg2::SPLIT_K},
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -1036,6 +1056,7 @@ static int device_setup(const DeviceState** out) {
         }
         int rc = raise_lds_limits<Cfg0>();
         if (rc == MUON_AMD_OK) rc = raise_lds_limits<Cfg1>();
+        if (rc == MUON_AMD_OK) rc = raise_lds_limits<Cfg2>();
         if (rc != MUON_AMD_OK) return rc;
         void* ptr = nullptr;
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || ptr == nullptr) {
@@ -1090,6 +1111,8 @@ static int launch_gemm_class(const DeviceState& st, int tile_class, const MuonGe
                              hipStream_t s) {
     if (tile_class == 0)
         return launch_gemm<Cfg0>(st, descs, jobs, njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap, s);
+    if (tile_class == 2)
+        return launch_gemm<Cfg2>(st, descs, jobs, njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap, s);
     return launch_gemm<Cfg1>(st, descs, jobs, njobs, alpha, beta, gamma, flags, split_partials, split_counters, ap, s);
 }
 
@@ -1172,7 +1195,7 @@ int muon_amd_validate_gemm(const MuonGemmDesc* descs, int ndesc, const MuonTileJ
         MUON_REQUIRE(t.i0 >= 0 && t.j0 >= 0 && t.i0 % TR == 0 && t.j0 % TC == 0 && t.i0 + TR <= d.rows &&
                          t.j0 + TC <= d.colsn,
                      "job %d: tile (%d,%d) outside %dx%d", j, t.i0, t.j0, d.rows, d.colsn);
-        MUON_REQUIRE(t.diag == 0 || t.diag == 1, "job %d: diag=%d", j, t.diag);
+        MUON_REQUIRE(t.diag >= 0 && t.diag <= 2, "job %d: diag=%d", j, t.diag);
         MUON_REQUIRE(t.k0 >= 0 && t.k0 < t.k1 && t.k1 <= d.K && t.k0 % BK == 0 && t.k1 % BK == 0,
                      "job %d: K range %d..%d of %d", j, t.k0, t.k1, d.K);
         const int count = t.split >> 16, idx = t.split & 0xffff;
@@ -1190,9 +1213,10 @@ int muon_amd_validate_gemm(const MuonGemmDesc* descs, int ndesc, const MuonTileJ
             MUON_REQUIRE(seen[t.part_base] <= count, "job %d: split group at slot %d has too many jobs", j, t.part_base);
         }
         // mirrored GEMM: only tiles whose column block is on or above the row block, and tiles
-        // inside a diagonal TR x TR block (stored directly, never mirrored) are flagged
+        // inside a diagonal TR x TR block (stored directly, never mirrored) are flagged; a tile that
+        // is flagged 2 is stored directly wherever it lies
         const int cblk = t.j0 / TR * TR;
-        MUON_REQUIRE(!(d.CT == d.C && d.C) || (cblk >= t.i0 && t.diag == (cblk == t.i0)),
+        MUON_REQUIRE(!(d.CT == d.C && d.C) || t.diag == 2 || (cblk >= t.i0 && t.diag == (cblk == t.i0)),
                      "job %d: mirrored GEMM needs its column block >= row block and diag set on the diagonal block", j);
     }
     for (int g = 0; g < split_slots; ++g)

@@ -83,24 +83,19 @@ class _ChunkRuntime:
         self.chunk = chunk
         self.device = device
         gemm = chunk.gemm_descs(base)
-        for ph in range(_plan.N_PHASES):
-            if ph == _plan.PH_POLY_FULL and chunk.poly_full_jobs is None:
-                continue
-            jobs = (chunk.syrk_jobs if ph in (_plan.PH_SYRK, _plan.PH_SYRK_ODD) else
-                    chunk.sym_jobs if ph == _plan.PH_POLY else
-                    chunk.poly_full_jobs if ph == _plan.PH_POLY_FULL else chunk.full_jobs)
-            full = ph in (_plan.PH_UPD_EVEN, _plan.PH_UPD_ODD, _plan.PH_UPD_LAST)
-            _lib.check(lib.muon_amd_validate_gemm(_lib.host_ptr(gemm[ph]), chunk.nmat,
-                                                  _lib.host_ptr(jobs), len(jobs),
-                                                  chunk.update_class if full else chunk.tile_class,
-                                                  chunk.split_slots if ph in (_plan.PH_SYRK, _plan.PH_SYRK_ODD) else 0),
-                       "validate_gemm")
+        phases = {"gram": (_plan.PH_SYRK, _plan.PH_SYRK_ODD), "gram_rowsum": (_plan.PH_SYRK,), "poly": (_plan.PH_POLY,),
+                  "poly_full": (_plan.PH_POLY_FULL,),
+                  "update": (_plan.PH_UPD_EVEN, _plan.PH_UPD_ODD, _plan.PH_UPD_LAST)}
+        for kind, ln in chunk.launches.items():
+            for ph in phases[kind]:
+                _lib.check(lib.muon_amd_validate_gemm(_lib.host_ptr(gemm[ph]), chunk.nmat, _lib.host_ptr(ln.jobs),
+                                                      len(ln.jobs), ln.tile_class, ln.split_slots), "validate_gemm")
         self.mat_template = chunk.mat_descs(base)
-        # one static device blob: gemm descs | sym jobs | full jobs | block prefix | tile prefix |
-        # syrk jobs (| AOL descs | AOL row prefix | AOL segment prefix), each part 256-byte aligned
-        parts = [gemm.reshape(-1).view(np.uint8), chunk.sym_jobs.view(np.uint8),
-                 chunk.full_jobs.view(np.uint8), chunk.block_prefix.view(np.uint8),
-                 chunk.tile_prefix.view(np.uint8), chunk.syrk_jobs.view(np.uint8)]
+        # one static device blob: gemm descs | block prefix | tile prefix | the job list of every kind of
+        # launch (| AOL descs | AOL row prefix | AOL segment prefix), each part 256-byte aligned
+        kinds = list(chunk.launches)
+        parts = [gemm.reshape(-1).view(np.uint8), chunk.block_prefix.view(np.uint8), chunk.tile_prefix.view(np.uint8)]
+        parts += [chunk.launches[kind].jobs.view(np.uint8) for kind in kinds]
         if chunk.aol:
             aol = chunk.aol_descs(base)
             _lib.check(lib.muon_amd_validate_aol(_lib.host_ptr(aol), chunk.nmat,
@@ -108,8 +103,6 @@ class _ChunkRuntime:
                                                  _lib.host_ptr(chunk.aol_seg_prefix)), "validate_aol")
             parts += [aol.view(np.uint8), chunk.aol_row_prefix.view(np.uint8),
                       chunk.aol_seg_prefix.view(np.uint8)]
-            if chunk.poly_full_jobs is not None:
-                parts.append(chunk.poly_full_jobs.view(np.uint8))
         # {0, blocks of matrix k} for every k: the prefix table of a momentum launch over matrix k alone
         single = np.zeros((chunk.nmat, 2), dtype=np.int32)
         single[:, 1] = np.diff(chunk.block_prefix)
@@ -125,18 +118,16 @@ class _ChunkRuntime:
         self.static = _upload(np.concatenate(blob), device)
         b = self.static.data_ptr()
         self.gemm_ptr = [b + offs[0] + ph * chunk.nmat * _lib.GEMM_DESC.itemsize for ph in range(_plan.N_PHASES)]
-        self.sym_jobs_ptr = b + offs[1]
-        self.full_jobs_ptr = b + offs[2]
-        self.block_prefix_ptr = b + offs[3]
-        self.tile_prefix_ptr = b + offs[4]
-        self.syrk_jobs_ptr = b + offs[5]
+        self.block_prefix_ptr = b + offs[1]
+        self.tile_prefix_ptr = b + offs[2]
+        self.jobs_ptr = {kind: b + offs[3 + i] for i, kind in enumerate(kinds)}
         # counters of the split groups: zero now, and every launch that uses them leaves them zero
-        self.split_counters = torch.zeros(max(chunk.split_slots, 1), dtype=torch.int32, device=device)
-        self.split_partials_ptr = base + chunk.off_split_partials if chunk.split_slots else None
-        self.split_counters_ptr = self.split_counters.data_ptr() if chunk.split_slots else None
+        self.split_slots = max(ln.split_slots for ln in chunk.launches.values())
+        self.split_counters = torch.zeros(max(self.split_slots, 1), dtype=torch.int32, device=device)
+        self.split_partials_ptr = base + chunk.off_split_partials if self.split_slots else None
+        self.split_counters_ptr = self.split_counters.data_ptr() if self.split_slots else None
         if chunk.aol:
-            self.aol_ptr, self.aol_row_prefix_ptr, self.aol_seg_prefix_ptr = (b + o for o in offs[6:9])
-            self.poly_full_jobs_ptr = b + offs[9] if chunk.poly_full_jobs is not None else None
+            self.aol_ptr, self.aol_row_prefix_ptr, self.aol_seg_prefix_ptr = (b + o for o in offs[3 + len(kinds):6 + len(kinds)])
         self.single_prefix_ptr = b + offs[-1]
         self.single_blocks = single[:, 1].tolist()
         self.mat_dev = None
@@ -226,7 +217,7 @@ class _ChunkRuntime:
                         for lay, sz, (has_m, _, _) in zip(c.layouts, store, self.present))
         apply_bytes = sum(lay.numel * (2 + (2 * sz if has_p else 0) + (2 if has_o else 0))
                           for lay, sz, (_, has_p, has_o) in zip(c.layouts, store, self.present))
-        if c.split_slots:
+        if self.split_slots:
             # every launch leaves the counters of the split groups zero; clearing them here as well
             # (a fill kernel, recordable into a graph) keeps a launch that died half way from
             # poisoning every later step
@@ -250,19 +241,18 @@ class _ChunkRuntime:
         }
         f_upd = sum(2 * lay.m * lay.m * lay.n for lay in c.layouts)
 
-        def gemm(name, ph, it, jobs_ptr, njobs, work, extra_flags=0):
+        def gemm(name, ph, it, kind, work, extra_flags=0):
             al, be, ga = c.phase_scalars(ph, it)
-            split = ph in (_plan.PH_SYRK, _plan.PH_SYRK_ODD)
-            tile_class = c.update_class if jobs_ptr == self.full_jobs_ptr else c.tile_class
+            ln = c.launches[kind]
             _launch(name, work, lambda: _lib.check(lib.muon_amd_ns_gemm(
-                self.gemm_ptr[ph], jobs_ptr, njobs, tile_class, al, be, ga, flags | extra_flags,
-                self.split_partials_ptr if split else None, self.split_counters_ptr if split else None, s),
-                "ns_gemm"))
+                self.gemm_ptr[ph], self.jobs_ptr[kind], len(ln.jobs), ln.tile_class, al, be, ga, flags | extra_flags,
+                self.split_partials_ptr if ln.split_slots else None, self.split_counters_ptr if ln.split_slots else None,
+                s), "ns_gemm"))
 
         for it in range(c.steps):
             first_aol = c.aol and it == 0
-            gemm("ns_gemm/syrk", _plan.PH_SYRK if it % 2 == 0 else _plan.PH_SYRK_ODD, it, self.syrk_jobs_ptr,
-                 len(c.syrk_jobs), flops[_plan.PH_SYRK], _lib.GEMM_ROWSUM if first_aol else 0)
+            gemm("ns_gemm/syrk", _plan.PH_SYRK if it % 2 == 0 else _plan.PH_SYRK_ODD, it,
+                 "gram_rowsum" if first_aol else "gram", flops[_plan.PH_SYRK], _lib.GEMM_ROWSUM if first_aol else 0)
             if first_aol:
                 # muon.py:776-785: the row sums of |A| come out of the product's epilogue as partial
                 # sums (one small launch adds them up), then X and A are rescaled in place (A becomes
@@ -278,19 +268,19 @@ class _ChunkRuntime:
                     "aol_rescale"))
             if first_aol and c.variant == "aol4_rows":
                 # A / s is not symmetric: c * A A^T + b * A over every tile, no mirrored store
-                gemm("ns_gemm/poly", _plan.PH_POLY_FULL, it, self.poly_full_jobs_ptr, len(c.poly_full_jobs),
-                     2 * flops[_plan.PH_POLY])
+                gemm("ns_gemm/poly", _plan.PH_POLY_FULL, it, "poly_full", 2 * flops[_plan.PH_POLY])
             else:
-                gemm("ns_gemm/poly", _plan.PH_POLY, it, self.sym_jobs_ptr, len(c.sym_jobs), flops[_plan.PH_POLY])
+                gemm("ns_gemm/poly", _plan.PH_POLY, it, "poly", flops[_plan.PH_POLY])
             if it == c.steps - 1:
                 # the last update product takes the parameter step in its epilogue (muon.py:14, 98-99)
                 al, be, _ = c.phase_scalars(_plan.PH_UPD_LAST, it)
                 _launch("ns_gemm/update_apply", f_upd, lambda: _lib.check(lib.muon_amd_ns_gemm_apply(
-                    self.gemm_ptr[_plan.PH_UPD_LAST], self.full_jobs_ptr, len(c.full_jobs), c.update_class, al, be,
+                    self.gemm_ptr[_plan.PH_UPD_LAST], self.jobs_ptr["update"], len(c.launches["update"].jobs),
+                    c.launches["update"].tile_class, al, be,
                     flags, mats, lr, wd_factor, sc_apply, s), "ns_gemm_apply"))
                 return
-            gemm("ns_gemm/update", _plan.PH_UPD_EVEN if it % 2 == 0 else _plan.PH_UPD_ODD, it, self.full_jobs_ptr,
-                 len(c.full_jobs), f_upd, _lib.GEMM_Q_KMAJOR)
+            gemm("ns_gemm/update", _plan.PH_UPD_EVEN if it % 2 == 0 else _plan.PH_UPD_ODD, it, "update", f_upd,
+                 _lib.GEMM_Q_KMAJOR)
         # no iteration (steps == 0): the parameter step is a launch of its own
         _launch("apply", apply_bytes, lambda: _lib.check(lib.muon_amd_apply(
             mats, self.block_prefix_ptr, c.nmat, c.nblocks, lr, wd_factor, sc_apply, s), "apply"))

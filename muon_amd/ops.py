@@ -10,7 +10,7 @@ Arithmetic: bf16 operands, fp32 accumulation, one rounding to bf16 of the finish
 the reference's kernels do (muon.py:399-400, 531-536, 675-696).  The two symmetric products compute
 the tiles on and above the diagonal and store each with its mirror image (muon.py:402-413): for a
 symmetric A, which ns_line_2 asks for, that is the whole result; otherwise what lands below the
-diagonal tiles is the image of what is above them, and depends on the tile size here (128 or 256)
+diagonal tiles is the image of what is above them, and depends on the tile size here (64, 128 or 256)
 as it does on the autotuned block in the reference.  bf16 CUDA tensors only; any strides; 2-D or
 3-D (a batch).
 
@@ -19,6 +19,8 @@ groups with its fused epilogues.  These entry points serve callers that used the
 operators directly.
 """
 from __future__ import annotations
+
+from functools import lru_cache
 
 import numpy as np
 import torch
@@ -54,6 +56,14 @@ def _product_jobs(tile_class: int, batch: int, rows_p: int, cols_p: int, kdim: i
     if nsplit > 1:
         jobs["part_base"] += np.repeat(np.arange(batch) * len(ti) * nsplit, len(one))
     return np.ascontiguousarray(jobs[_plan.xcd_permutation(len(jobs), si * sj)])
+
+
+@lru_cache(maxsize=256)
+def _launch_class(kind: str, tile_class: int, batch: int, m: int, n: int) -> int:
+    """Smaller tiles where `tile_class` would leave CUs without a job, as in the optimizer's launches."""
+    unit = _plan.pad_unit(tile_class)
+    lay = _plan.MatLayout(0, m, n, m, n, _plan._round_up(m, unit), _plan._round_up(n, unit), True)
+    return _plan.launch_class(kind, tile_class, [lay] * batch)
 
 
 class _Product:
@@ -148,12 +158,14 @@ def _symmetric_product(A: torch.Tensor, out, alpha: float, beta: float, addend: 
     A3, out3 = _as_batch(A), _as_batch(out)
     batch = A3.size(0)
     tile_class = _plan.tile_class_for(M)
-    unit = _plan.pad_unit(tile_class)
-    mp = _plan._round_up(M, unit)
-    kp = mp if addend else _plan._round_up(K, _plan.GEMM_BK)
+    kp = _plan._round_up(K, _plan.GEMM_BK)
+    # X X^T of a short, very wide matrix: a few tiles with very long reductions, which are split
+    nsplit = 1 if addend or tile_class != 0 else _plan.split_factor(_plan._round_up(M, 128), kp)
+    tile_class = _launch_class("poly" if addend else "gram", tile_class, batch, M, K)
+    mp = _plan._round_up(M, _plan.pad_unit(tile_class))
+    if addend:
+        kp = mp
     with torch.cuda.device(A.device):
-        # X X^T of a short, very wide matrix: a few tiles with very long reductions, which are split
-        nsplit = 1 if addend or tile_class != 0 else _plan.split_factor(mp, kp)
         prod = _cached(("sym_product", A.device, tile_class, batch, mp, kp, nsplit),
                        lambda: _Product(A.device, tile_class, batch, mp, mp, kp, True, nsplit),
                        _PRODUCT_CACHE, _PRODUCT_CACHE_MAX)
@@ -219,13 +231,14 @@ def ns_line_3(B: torch.Tensor, X: torch.Tensor, a: float, *, out: torch.Tensor =
     batch = X3.size(0)
     assert B3.size(0) in (1, batch), "B and X must have the same batch size"
     tile_class = _plan.tile_class_for(min(M, N))
-    unit = _plan.pad_unit(tile_class)
-    mp, np_ = _plan._round_up(M, unit), _plan._round_up(N, unit)
+    mp, np_ = (_plan._round_up(s, _plan.pad_unit(tile_class)) for s in (M, N))
     # as in the optimizer's update launches: 256 x 256 tiles also for shorter matrices when their
     # padded sizes allow it and there are enough of them to give every CU one
     if (tile_class == 0 and mp % 256 == 0 and np_ % 256 == 0 and
             batch * (mp // 256) * (np_ // 256) >= _plan.RESIDENT_BIG_TILE_WORKGROUPS):
         tile_class = 1
+    tile_class = _launch_class("update", tile_class, batch, M, N)
+    mp, np_ = (_plan._round_up(s, _plan.pad_unit(tile_class)) for s in (M, N))
     with torch.cuda.device(X.device):
         prod = _cached(("update_product", X.device, tile_class, batch, mp, np_),
                        lambda: _Product(X.device, tile_class, batch, mp, np_, mp, False),

@@ -38,9 +38,9 @@ VARIANTS = ("ns5", "aol4", "aol4_rows")
 # relative Frobenius norm from the float64 one at 18 x 63), so no error bound can be stated below it.
 AOL_ROWS_MIN_SIDE = 32
 AOL_ROWS = 4                            # must match muon_amd_aol_rows_per_block()
-TILE_DIMS = {0: (128, 128), 1: (256, 256)}   # must match muon_amd_gemm_tile_rows/cols()
+TILE_DIMS = {0: (128, 128), 1: (256, 256), 2: (64, 64)}   # must match muon_amd_gemm_tile_rows/cols()
 # output tiles (rows, cols) of one XCD-resident super-block: as many tiles as an XCD holds workgroups
-SUPER_DIMS = {0: (8, 8), 1: (4, 8)}
+SUPER_DIMS = {0: (8, 8), 1: (4, 8), 2: (8, 8)}
 if os.environ.get("MUON_AMD_SUPER"):     # measurement knob: "rows,cols" of the 256 x 256 class super-block
     SUPER_DIMS[1] = tuple(int(v) for v in os.environ["MUON_AMD_SUPER"].split(","))
 EW_BLOCK_ELEMS = 8192                   # must match muon_amd_elementwise_block_elems()
@@ -105,6 +105,17 @@ class MatLayout:
     np_: int
     wide: bool            # rows <= cols: X is the matrix itself; else X is its transpose
     off: dict = field(default_factory=dict)   # byte offsets of X0, X1, A, B, CA
+
+    # What a product has to reduce over and compute: the padding of the buffers beyond the k-block of the
+    # last row or column is zero (or, in buffers that only small tiles write, whatever was there before;
+    # it is not read as part of a reduction, and rows of it only reach rows of padding).
+    @property
+    def mk(self) -> int:
+        return _round_up(self.m, GEMM_BK)
+
+    @property
+    def nk(self) -> int:
+        return _round_up(self.n, GEMM_BK)
 
     @property
     def ldn(self) -> int:     # leading dimension of X (rows of length np_)
@@ -174,15 +185,16 @@ def matrix_scratch_bytes(rows: int, cols: int, tile_class: int, aol: bool) -> in
 
 
 @lru_cache(maxsize=256)
-def _tile_order(mt: int, nt: int, sym: bool, ratio: int, super_i: int, super_j: int):
+def _tile_order(mt: int, nt: int, sym: bool, ratio: int, super_i: int, super_j: int, direct: int = 1):
     """Tiles of an mt x nt grid in super-block order.  `ratio` = tile rows / tile cols; with sym
-    only tiles whose column block (j // ratio) is on or above their row block are kept."""
+    only tiles whose column block (j // ratio) is on or above their row block are kept, blocks being
+    `direct` tile rows high (every tile of a diagonal block is kept)."""
     ti, tj = [], []
     for bi in range(0, mt, super_i):
         for bj in range(0, nt, super_j):
             for i in range(bi, min(bi + super_i, mt)):
                 for j in range(bj, min(bj + super_j, nt)):
-                    if sym and j // ratio < i:
+                    if sym and j // ratio // direct < i // direct:
                         continue
                     ti.append(i)
                     tj.append(j)
@@ -223,8 +235,8 @@ def xcd_permutation(njobs: int, group: int = 32) -> np.ndarray:
 # Cost of a job in k-blocks for balancing a launch: its reduction plus what its prologue and
 # epilogue cost in the same unit (measured: about 8 us against 0.65 us per k-block for the
 # 128 x 128 class, 12 us against 1.6 us for the 256 x 256 class).
-JOB_FIXED_KBLOCKS = {0: 12, 1: 8}
-WORKGROUPS_PER_CU = {0: 2, 1: 1}        # must match the kernels' launch bounds
+JOB_FIXED_KBLOCKS = {0: 12, 1: 8, 2: 12}
+WORKGROUPS_PER_CU = {0: 2, 1: 1, 2: 2}  # must match the kernels' launch bounds
 N_CU = 256
 
 
@@ -274,6 +286,67 @@ def whole_matrix_group(tiles_per_matrix, default: int) -> int:
         if g <= 4 * default:
             return g
     return default
+
+
+@dataclass
+class Launch:
+    tile_class: int
+    jobs: np.ndarray
+    split_slots: int
+
+
+LAUNCH_CLASS = os.environ.get("MUON_AMD_LAUNCH_CLASS", "auto")      # measurement knob: "gram,poly,update" classes
+
+
+# Time of a launch by tile class, in microseconds, measured with isolated launches of one class over the same
+# matrices (shapes from 64 x 576 to 4096 x 14336, 1 to 256 of them):
+#   a job alone on its CU      fixed + k-blocks * alone
+#   jobs in turn on a CU       k-blocks * shared + fixed_shared each (their epilogues overlap the neighbour's loop)
+# e.g. 1100 x 1500, X X^T / polynomial / update: 256 x 256 tiles 35 / 27 / 28 us (15 and 30 jobs), 128 x 128
+# tiles 14.5 / 11.8 / 14.4, 64 x 64 tiles 8.3 / 6.8 / 9.9; 768 x 3072: 128 x 128 22 / 9.4 / 11, 64 x 64 12 / 5.6 / 11;
+# 48 x (768 x 3072), where the larger tiles fill the GPU: X X^T 133 us in 128 x 128 tiles, 182 in 64 x 64.
+LAUNCH_COST = {1: dict(fixed=9.5, alone=0.98, shared=1.3, fixed_shared=13.0, base=0.0),
+               0: dict(fixed=5.1, alone=0.36, shared=0.5, fixed_shared=2.2, base=3.0),
+               2: dict(fixed=3.4, alone=0.183, shared=0.235, fixed_shared=0.8, base=2.8)}
+
+
+# ... and what a job of a split reduction adds (it parks its accumulators, and the last one of a tile adds
+# them up): ten matrices of a convolutional network, 26 us in 130 jobs of 128 x 128, 33 us in 451 of 64 x 64.
+SPLIT_HANDOVER_US = 8.0
+
+
+def launch_time_us(kind: str, tile_class: int, layouts) -> float:
+    """Estimated time of a product over `layouts` in tiles of one class (see LAUNCH_COST): one job per CU
+    as long as there are fewer jobs than CUs, whose k-blocks take longer the more CUs are busy; beyond
+    that the jobs of a CU in turn, the last partly filled round counted half."""
+    T, cost = TILE_DIMS[tile_class][0], LAUNCH_COST[tile_class]
+    jobs = kblocks = longest = split = 0
+    for lay in layouts:
+        mt, nt = -(-lay.mk // T), -(-lay.nk // T)
+        kb, ns = (lay.nk if kind == "gram" else lay.mk) // GEMM_BK, 1
+        if kind == "gram":
+            ns = split_factor(lay.mp, lay.np_)
+        n = (mt * nt if kind == "update" else mt * (mt + 1) // 2) * ns
+        split = max(split, ns - 1)
+        jobs += n
+        kblocks += n * kb / ns
+        longest = max(longest, kb / ns)
+    handover = SPLIT_HANDOVER_US if split else 0.0
+    if jobs <= N_CU:
+        return handover + cost["fixed"] + longest * (cost["alone"] + (cost["shared"] - cost["alone"]) * jobs / N_CU)
+    rounds = (jobs / N_CU + -(-jobs // N_CU)) / 2
+    return cost["base"] + rounds * (kblocks / jobs * cost["shared"] + cost["fixed_shared"] + handover)
+
+
+def launch_class(kind: str, tile_class: int, layouts) -> int:
+    """Tile class of a launch whose own class would be `tile_class`: a smaller one where that is
+    estimated to be faster, that is where the larger tiles leave CUs without a job.  Which tiles compute
+    an element does not change its bits."""
+    if LAUNCH_CLASS != "auto":
+        want = int(LAUNCH_CLASS.split(",")[("gram", "poly", "update").index(kind)])
+        return want if TILE_DIMS[want][0] <= TILE_DIMS[tile_class][0] else tile_class
+    classes = [c for c in (1, 0, 2) if TILE_DIMS[c][0] <= TILE_DIMS[tile_class][0]]
+    return min(classes, key=lambda c: launch_time_us(kind, c, layouts))
 
 
 class ChunkPlan:
@@ -332,49 +405,68 @@ class ChunkPlan:
         self.aol_seg_prefix = np.concatenate([[0], np.cumsum(segblk)]).astype(np.int32)
         # job lists: the symmetric products share their tiles but not their reduction length
         # (X X^T reduces over n, the polynomial over m), and only the former is ever split
-        self.split_slots = 0
-        self.syrk_jobs = self._jobs(sym=True, reduce_over_n=True)
-        self.sym_jobs = self._jobs(sym=True, reduce_over_n=False)
+        self.syrk_jobs, self.split_slots = self._jobs(sym=True, reduce_over_n=True)
+        self.sym_jobs, _ = self._jobs(sym=True, reduce_over_n=False)
         # The update products may run in the 256 x 256 class where the chunk as a whole is in the
         # 128 x 128 class (see update_class_for).
         self.update_class = update_class_for(tile_class, self.layouts)
-        self.full_jobs = self._jobs(sym=False, reduce_over_n=False, tile_class=self.update_class)
+        self.full_jobs, _ = self._jobs(sym=False, reduce_over_n=False, tile_class=self.update_class)
         # every tile of the m x m polynomial (no mirrored store): the first iteration of "aol4_rows",
         # whose Gram matrix is not symmetric after the row-only rescaling
-        self.poly_full_jobs = self._jobs(sym=False, reduce_over_n=False, square=True) if variant == "aol4_rows" else None
+        self.poly_full_jobs = self._jobs(sym=False, reduce_over_n=False, square=True)[0] if variant == "aol4_rows" else None
+        # what is launched: these lists, or smaller tiles for a product that would leave CUs idle with them.
+        # (The X X^T launch that leaves row sums keeps the chunk's tiles: their slots are 64 columns wide.)
+        self.launches = {
+            "gram": self._launch("gram", tile_class, self.syrk_jobs, self.split_slots),
+            "poly": self._launch("poly", tile_class, self.sym_jobs, 0),
+            "update": self._launch("update", self.update_class, self.full_jobs, 0),
+        }
+        if self.aol:
+            self.launches["gram_rowsum"] = Launch(tile_class, self.syrk_jobs, self.split_slots)
+        if self.poly_full_jobs is not None:
+            self.launches["poly_full"] = Launch(tile_class, self.poly_full_jobs, 0)
         # fp32 slots of the split jobs (scratch like the rest; the per-slot counters are not part
         # of the workspace: they must stay zero between launches, and chunks share the workspace)
         self.off_split_partials = off
-        off += _round_up(self.split_slots * self.tile_rows * self.tile_cols * 4, _ALIGN)
+        off += _round_up(max([self.split_slots * self.tile_rows * self.tile_cols * 4] +
+                             [ln.split_slots * TILE_DIMS[ln.tile_class][0] * TILE_DIMS[ln.tile_class][1] * 4
+                              for ln in self.launches.values()]), _ALIGN)
         self.workspace_bytes = off
 
     # ---- tile job lists -----------------------------------------------------------------
-    def _jobs(self, sym: bool, reduce_over_n: bool, square: bool = False, tile_class: int | None = None) -> np.ndarray:
+    def _jobs(self, sym: bool, reduce_over_n: bool, square: bool = False, tile_class: int | None = None,
+              live_only: bool = False, direct: int = 1):
+        """-> (job list in launch order, split slots it addresses).  live_only: without the tiles that lie in
+        the padding altogether (there are some only for tiles smaller than the chunk's padding unit).
+        direct: every tile of a diagonal block of so many tile rows is computed and stored as it is, the
+        blocks above are mirrored."""
         tile_class = self.tile_class if tile_class is None else tile_class
         TR, TC = TILE_DIMS[tile_class]
         ratio = TR // TC
         si, sj = SUPER_DIMS[tile_class]
-        parts = []
+        parts, slots = [], 0
         for k, lay in enumerate(self.layouts):
-            mt = lay.mp // TR
-            nt = (lay.mp if (sym or square) else lay.np_) // TC
-            ti, tj = _tile_order(mt, nt, sym, ratio, si, sj)
-            kdim = lay.np_ if reduce_over_n else lay.mp
-            nsplit = split_factor(lay.mp, kdim) if reduce_over_n else 1
+            rows, cols = (lay.mk, lay.nk) if live_only else (lay.mp, lay.np_)
+            mt = -(-rows // TR)
+            nt = -(-(rows if (sym or square) else cols) // TC)
+            ti, tj = _tile_order(mt, nt, sym, ratio, si, sj, direct)
+            kdim = lay.nk if reduce_over_n else lay.mk
+            nsplit = split_factor(lay.mp, lay.np_) if reduce_over_n else 1
             j = np.zeros(len(ti) * nsplit, dtype=_lib.TILE_JOB)
             j["desc"] = k
             j["i0"] = np.repeat(ti * TR, nsplit)
             j["j0"] = np.repeat(tj * TC, nsplit)
-            j["diag"] = np.repeat((ti == tj // ratio).astype(np.int32), nsplit) if sym else 0
+            if sym:
+                j["diag"] = np.repeat(np.where(ti == tj // ratio, 1, np.where(ti // direct == tj // ratio // direct, 2, 0)), nsplit)
             if nsplit == 1:
                 j["k1"] = kdim
             else:      # k-blocks dealt as evenly as 64-wide blocks allow; one group of slots per tile
                 edges = (np.arange(nsplit + 1) * (kdim // GEMM_BK) // nsplit) * GEMM_BK
                 idx = np.tile(np.arange(nsplit), len(ti))
                 j["k0"], j["k1"] = edges[idx], edges[idx + 1]
-                j["part_base"] = self.split_slots + np.repeat(np.arange(len(ti)) * nsplit, nsplit)
+                j["part_base"] = slots + np.repeat(np.arange(len(ti)) * nsplit, nsplit)
                 j["split"] = idx | (nsplit << 16)
-                self.split_slots += len(ti) * nsplit
+                slots += len(ti) * nsplit
             parts.append(j)
         logical = np.concatenate(parts)
         if os.environ.get("MUON_AMD_XCD_GROUP"):                        # measurement knob
@@ -383,7 +475,21 @@ class ChunkPlan:
             group = whole_matrix_group([len(p) for p in parts], si * sj)
         else:
             group = choose_xcd_group((logical["k1"] - logical["k0"]) // GEMM_BK, tile_class, si * sj)
-        return np.ascontiguousarray(logical[xcd_permutation(len(logical), group)])
+        return np.ascontiguousarray(logical[xcd_permutation(len(logical), group)]), slots
+
+    def _launch(self, kind: str, tile_class: int, jobs, slots: int) -> Launch:
+        """The launch of a product: the chunk's own tiles, or smaller ones where `launch_class` says that
+        they fill the GPU better."""
+        other = launch_class(kind, tile_class, self.layouts)
+        if other != tile_class:
+            # c A A with c A rounded is not symmetric to the last bit: which of its elements are computed and
+            # which are mirrored stays what the chunk's own tiles make of it, so that a matrix gets the same
+            # bits whatever else is in the launch (X X^T is symmetric bit for bit)
+            direct = TILE_DIMS[tile_class][0] // TILE_DIMS[other][0] if kind == "poly" else 1
+            tile_class = other
+            jobs, slots = self._jobs(sym=kind != "update", reduce_over_n=kind == "gram", tile_class=other,
+                                     live_only=True, direct=direct)
+        return Launch(tile_class, jobs, slots)
 
     # ---- descriptor tables -----------------------------------------------------------------
     def gemm_descs(self, base: int) -> np.ndarray:
@@ -396,7 +502,7 @@ class ChunkPlan:
                 s = d[ph, k]
                 s["P"] = s["Q"] = p[src]
                 s["ldp"] = s["ldq"] = lay.ldn
-                s["K"] = np_
+                s["K"] = lay.nk
                 s["C"] = s["CT"] = p["A"]
                 if self.reference_rounding:
                     s["C2"] = s["C2T"] = p["CA"]
@@ -409,7 +515,7 @@ class ChunkPlan:
             q["P"] = p["CA"] if self.reference_rounding else p["A"]
             q["Q"] = q["D"] = p["A"]
             q["ldp"] = q["ldq"] = q["ldd"] = lay.ldm
-            q["K"] = mp
+            q["K"] = lay.mk
             q["C"] = q["CT"] = p["B"]
             q["ldc"] = q["ldct"] = lay.ldm
             q["rows"] = q["colsn"] = mp
@@ -425,7 +531,7 @@ class ChunkPlan:
                 u["Q"] = u["D"] = p[src]
                 u["ldq"] = u["ldd"] = lay.ldn
                 u["q_kmajor"] = 1
-                u["K"] = mp
+                u["K"] = lay.mk
                 u["C"] = p[dst]
                 u["ldc"] = lay.ldn
                 u["rows"] = mp
