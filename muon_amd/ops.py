@@ -63,7 +63,7 @@ def _launch_class(kind: str, tile_class: int, batch: int, m: int, n: int) -> int
     """Smaller tiles where `tile_class` would leave CUs without a job, as in the optimizer's launches."""
     unit = _plan.pad_unit(tile_class)
     lay = _plan.MatLayout(0, m, n, m, n, _plan._round_up(m, unit), _plan._round_up(n, unit), True)
-    return _plan.launch_class(kind, tile_class, [lay] * batch)
+    return _plan.launch_class(kind, tile_class, [(lay, batch)])
 
 
 class _Product:

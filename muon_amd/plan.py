@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import os
 from dataclasses import dataclass, field
-from functools import lru_cache
+from functools import cached_property, lru_cache
 
 import numpy as np
 
@@ -204,6 +204,7 @@ def _tile_order(mt: int, nt: int, sym: bool, ratio: int, super_i: int, super_j: 
 XCD_MODE = os.environ.get("MUON_AMD_XCD_MODE", "interleave")
 
 
+@lru_cache(maxsize=64)
 def xcd_permutation(njobs: int, group: int = 32) -> np.ndarray:
     """physical block b runs logical job perm[b].  Block b lands on XCD b % 8, as slot b // 8 of
     that XCD.  Consecutive groups of `group` logical jobs (one super-block: as many tiles as an XCD
@@ -315,18 +316,19 @@ LAUNCH_COST = {1: dict(fixed=9.5, alone=0.98, shared=1.3, fixed_shared=13.0, bas
 SPLIT_HANDOVER_US = 8.0
 
 
-def launch_time_us(kind: str, tile_class: int, layouts) -> float:
-    """Estimated time of a product over `layouts` in tiles of one class (see LAUNCH_COST): one job per CU
+def launch_time_us(kind: str, tile_class: int, runs) -> float:
+    """Estimated time of a product over `runs` of (layout, matrices of its shape) in tiles of one class (see
+    LAUNCH_COST): one job per CU
     as long as there are fewer jobs than CUs, whose k-blocks take longer the more CUs are busy; beyond
     that the jobs of a CU in turn, the last partly filled round counted half."""
     T, cost = TILE_DIMS[tile_class][0], LAUNCH_COST[tile_class]
     jobs = kblocks = longest = split = 0
-    for lay in layouts:
+    for lay, count in runs:
         mt, nt = -(-lay.mk // T), -(-lay.nk // T)
         kb, ns = (lay.nk if kind == "gram" else lay.mk) // GEMM_BK, 1
         if kind == "gram":
             ns = split_factor(lay.mp, lay.np_)
-        n = (mt * nt if kind == "update" else mt * (mt + 1) // 2) * ns
+        n = (mt * nt if kind == "update" else mt * (mt + 1) // 2) * ns * count
         split = max(split, ns - 1)
         jobs += n
         kblocks += n * kb / ns
@@ -338,7 +340,7 @@ def launch_time_us(kind: str, tile_class: int, layouts) -> float:
     return cost["base"] + rounds * (kblocks / jobs * cost["shared"] + cost["fixed_shared"] + handover)
 
 
-def launch_class(kind: str, tile_class: int, layouts) -> int:
+def launch_class(kind: str, tile_class: int, runs) -> int:
     """Tile class of a launch whose own class would be `tile_class`: a smaller one where that is
     estimated to be faster, that is where the larger tiles leave CUs without a job.  Which tiles compute
     an element does not change its bits."""
@@ -346,7 +348,7 @@ def launch_class(kind: str, tile_class: int, layouts) -> int:
         want = int(LAUNCH_CLASS.split(",")[("gram", "poly", "update").index(kind)])
         return want if TILE_DIMS[want][0] <= TILE_DIMS[tile_class][0] else tile_class
     classes = [c for c in (1, 0, 2) if TILE_DIMS[c][0] <= TILE_DIMS[tile_class][0]]
-    return min(classes, key=lambda c: launch_time_us(kind, c, layouts))
+    return min(classes, key=lambda c: launch_time_us(kind, c, runs))
 
 
 class ChunkPlan:
@@ -378,6 +380,14 @@ class ChunkPlan:
                 off += nbytes
             self.layouts.append(lay)
         self.nmat = len(self.layouts)
+        # (first matrix, (its layout, how many in a row have its shape)): tables are built once per shape
+        self._runs = []
+        for k, lay in enumerate(self.layouts):
+            last = self._runs[-1][1] if self._runs else None
+            if last is not None and (last[0].m, last[0].n) == (lay.m, lay.n):
+                last[1] += 1
+            else:
+                self._runs.append((k, [lay, 1]))
         # elementwise block prefix (momentum / apply) and normalise tile prefix
         nblk = [-(-lay.numel // EW_BLOCK_ELEMS) for lay in self.layouts]
         self.block_prefix = np.concatenate([[0], np.cumsum(nblk)]).astype(np.int32)
@@ -403,23 +413,23 @@ class ChunkPlan:
         # segments of the rescaling launch per matrix: rows of X, (rows of X^T: none is kept), rows of A
         segblk = [b for lay in self.layouts for b in (lay.mp // AOL_ROWS, 0, lay.mp // AOL_ROWS)]
         self.aol_seg_prefix = np.concatenate([[0], np.cumsum(segblk)]).astype(np.int32)
-        # job lists: the symmetric products share their tiles but not their reduction length
-        # (X X^T reduces over n, the polynomial over m), and only the former is ever split
-        self.syrk_jobs, self.split_slots = self._jobs(sym=True, reduce_over_n=True)
-        self.sym_jobs, _ = self._jobs(sym=True, reduce_over_n=False)
+        # job lists (syrk_jobs, sym_jobs, full_jobs): the symmetric products share their tiles but not their
+        # reduction length (X X^T reduces over n, the polynomial over m), and only the former is ever split.
         # The update products may run in the 256 x 256 class where the chunk as a whole is in the
         # 128 x 128 class (see update_class_for).
+        self.split_slots = sum(count * (lay.mp // self.tile_rows) * (lay.mp // self.tile_rows + 1) // 2 * ns
+                               for _, (lay, count) in self._runs
+                               if (ns := split_factor(lay.mp, lay.np_)) > 1)
         self.update_class = update_class_for(tile_class, self.layouts)
-        self.full_jobs, _ = self._jobs(sym=False, reduce_over_n=False, tile_class=self.update_class)
         # every tile of the m x m polynomial (no mirrored store): the first iteration of "aol4_rows",
         # whose Gram matrix is not symmetric after the row-only rescaling
         self.poly_full_jobs = self._jobs(sym=False, reduce_over_n=False, square=True)[0] if variant == "aol4_rows" else None
         # what is launched: these lists, or smaller tiles for a product that would leave CUs idle with them.
         # (The X X^T launch that leaves row sums keeps the chunk's tiles: their slots are 64 columns wide.)
         self.launches = {
-            "gram": self._launch("gram", tile_class, self.syrk_jobs, self.split_slots),
-            "poly": self._launch("poly", tile_class, self.sym_jobs, 0),
-            "update": self._launch("update", self.update_class, self.full_jobs, 0),
+            "gram": self._launch("gram", tile_class),
+            "poly": self._launch("poly", tile_class),
+            "update": self._launch("update", self.update_class),
         }
         if self.aol:
             self.launches["gram_rowsum"] = Launch(tile_class, self.syrk_jobs, self.split_slots)
@@ -444,52 +454,71 @@ class ChunkPlan:
         TR, TC = TILE_DIMS[tile_class]
         ratio = TR // TC
         si, sj = SUPER_DIMS[tile_class]
-        parts, slots = [], 0
-        for k, lay in enumerate(self.layouts):
+        parts, tiles, slots = [], [], 0
+        for k, (lay, count) in self._runs:
             rows, cols = (lay.mk, lay.nk) if live_only else (lay.mp, lay.np_)
             mt = -(-rows // TR)
             nt = -(-(rows if (sym or square) else cols) // TC)
             ti, tj = _tile_order(mt, nt, sym, ratio, si, sj, direct)
             kdim = lay.nk if reduce_over_n else lay.mk
             nsplit = split_factor(lay.mp, lay.np_) if reduce_over_n else 1
-            j = np.zeros(len(ti) * nsplit, dtype=_lib.TILE_JOB)
-            j["desc"] = k
-            j["i0"] = np.repeat(ti * TR, nsplit)
-            j["j0"] = np.repeat(tj * TC, nsplit)
+            n = len(ti) * nsplit
+            # the jobs of one matrix, then those of `count` matrices of its shape (columns as in MuonTileJob)
+            one = np.zeros((n, 8), dtype=np.int32)
+            one[:, 1], one[:, 2] = np.repeat(ti * TR, nsplit), np.repeat(tj * TC, nsplit)
             if sym:
-                j["diag"] = np.repeat(np.where(ti == tj // ratio, 1, np.where(ti // direct == tj // ratio // direct, 2, 0)), nsplit)
+                one[:, 3] = np.repeat(np.where(ti == tj // ratio, 1, np.where(ti // direct == tj // ratio // direct, 2, 0)), nsplit)
             if nsplit == 1:
-                j["k1"] = kdim
+                one[:, 5] = kdim
             else:      # k-blocks dealt as evenly as 64-wide blocks allow; one group of slots per tile
                 edges = (np.arange(nsplit + 1) * (kdim // GEMM_BK) // nsplit) * GEMM_BK
                 idx = np.tile(np.arange(nsplit), len(ti))
-                j["k0"], j["k1"] = edges[idx], edges[idx + 1]
-                j["part_base"] = slots + np.repeat(np.arange(len(ti)) * nsplit, nsplit)
-                j["split"] = idx | (nsplit << 16)
-                slots += len(ti) * nsplit
-            parts.append(j)
+                one[:, 4], one[:, 5] = edges[idx], edges[idx + 1]
+                one[:, 6] = np.repeat(np.arange(len(ti)) * nsplit, nsplit)
+                one[:, 7] = idx | (nsplit << 16)
+            part = np.tile(one, (count, 1))
+            part[:, 0] = np.repeat(np.arange(k, k + count), n)
+            if nsplit > 1:
+                part[:, 6] += np.repeat(slots + np.arange(count) * n, n)
+                slots += n * count
+            parts.append(part)
+            tiles.append(n)
         logical = np.concatenate(parts)
         if os.environ.get("MUON_AMD_XCD_GROUP"):                        # measurement knob
             group = int(os.environ["MUON_AMD_XCD_GROUP"])
         elif tile_class == 1 and not sym and WHOLE_MATRIX_GROUPS and any((lay.mp // TR) % si for lay in self.layouts):
-            group = whole_matrix_group([len(p) for p in parts], si * sj)
+            group = whole_matrix_group(tiles, si * sj)
         else:
-            group = choose_xcd_group((logical["k1"] - logical["k0"]) // GEMM_BK, tile_class, si * sj)
-        return np.ascontiguousarray(logical[xcd_permutation(len(logical), group)]), slots
+            group = choose_xcd_group((logical[:, 5] - logical[:, 4]) // GEMM_BK, tile_class, si * sj)
+        return np.ascontiguousarray(logical[xcd_permutation(len(logical), group)]).view(_lib.TILE_JOB).reshape(-1), slots
 
-    def _launch(self, kind: str, tile_class: int, jobs, slots: int) -> Launch:
+    @cached_property
+    def syrk_jobs(self):
+        jobs, slots = self._jobs(sym=True, reduce_over_n=True)
+        assert slots == self.split_slots
+        return jobs
+
+    @cached_property
+    def sym_jobs(self):
+        return self._jobs(sym=True, reduce_over_n=False)[0]
+
+    @cached_property
+    def full_jobs(self):
+        return self._jobs(sym=False, reduce_over_n=False, tile_class=self.update_class)[0]
+
+    def _launch(self, kind: str, tile_class: int) -> Launch:
         """The launch of a product: the chunk's own tiles, or smaller ones where `launch_class` says that
         they fill the GPU better."""
-        other = launch_class(kind, tile_class, self.layouts)
+        other = launch_class(kind, tile_class, [run for _, run in self._runs])
         if other != tile_class:
             # c A A with c A rounded is not symmetric to the last bit: which of its elements are computed and
             # which are mirrored stays what the chunk's own tiles make of it, so that a matrix gets the same
             # bits whatever else is in the launch (X X^T is symmetric bit for bit)
             direct = TILE_DIMS[tile_class][0] // TILE_DIMS[other][0] if kind == "poly" else 1
-            tile_class = other
-            jobs, slots = self._jobs(sym=kind != "update", reduce_over_n=kind == "gram", tile_class=other,
-                                     live_only=True, direct=direct)
-        return Launch(tile_class, jobs, slots)
+            return Launch(other, *self._jobs(sym=kind != "update", reduce_over_n=kind == "gram", tile_class=other,
+                                             live_only=True, direct=direct))
+        own = {"gram": "syrk_jobs", "poly": "sym_jobs", "update": "full_jobs"}[kind]
+        return Launch(tile_class, getattr(self, own), self.split_slots if kind == "gram" else 0)
 
     # ---- descriptor tables -----------------------------------------------------------------
     def gemm_descs(self, base: int) -> np.ndarray:
