@@ -160,6 +160,55 @@ typedef struct MuonAolDesc {
     int32_t   ld_rowsum, reserved;
 } MuonAolDesc;
 
+/* One product of a chunk as it is launched: its job list (device memory), the tile class it is cut for
+ * and the split slots it addresses (0: none of its jobs is split).                           */
+typedef struct MuonChunkLaunch {
+    const MuonTileJob* jobs;
+    int32_t njobs, tile_class, split_slots, reserved;
+} MuonChunkLaunch;
+
+/* Indices into MuonChunkRun.gemm: what a product reads and writes.  X X^T and the update of an even
+ * iteration read the first buffer of X (and the update writes the second), those of an odd one
+ * the second; the last update carries the parameter step.                                    */
+#define MUON_AMD_GRAM_EVEN    0
+#define MUON_AMD_POLY         1
+#define MUON_AMD_UPDATE_EVEN  2
+#define MUON_AMD_UPDATE_ODD   3
+#define MUON_AMD_UPDATE_LAST  4
+#define MUON_AMD_POLY_FULL    5   /* the polynomial over every tile, not mirrored (AOL_ROWS_ONLY) */
+#define MUON_AMD_GRAM_ODD     6
+#define MUON_AMD_GEMM_TABLES  7
+/* Indices into MuonChunkRun.launches. */
+#define MUON_AMD_LAUNCH_GRAM        0
+#define MUON_AMD_LAUNCH_POLY        1
+#define MUON_AMD_LAUNCH_UPDATE      2
+#define MUON_AMD_LAUNCH_GRAM_ROWSUM 3
+#define MUON_AMD_LAUNCH_POLY_FULL   4
+#define MUON_AMD_LAUNCHES           5
+
+/* Everything muon_amd_run_chunk needs of a chunk, laid out once (a host struct; unless noted the
+ * pointers are device pointers to the tables and the workspace of the entry points below).    */
+typedef struct MuonChunkRun {
+    const MuonMatDesc*  mats;
+    const int32_t*      block_prefix;
+    const int32_t*      tile_prefix;
+    const MuonGemmDesc* gemm[MUON_AMD_GEMM_TABLES];
+    MuonChunkLaunch     launches[MUON_AMD_LAUNCHES];
+    const float*        scalars;        /* HOST memory: per iteration {alpha, beta, gamma} of X X^T,
+                                           of the polynomial and of the update: 9 * steps floats  */
+    float*              split_partials; /* NULL when no launch is split                           */
+    int32_t*            split_counters;
+    const MuonAolDesc*  aol;            /* NULL: no AOL rescaling after the first X X^T            */
+    const int32_t*      aol_row_prefix;
+    const int32_t*      aol_seg_prefix;
+    int32_t nmat, nblocks, ntiles;
+    int32_t steps;                      /* iterations; 0: the normalised matrix is the result      */
+    int32_t flags;                      /* MUON_AMD_ROUND_*                                        */
+    int32_t split_slots;                /* counters to clear before the products                   */
+    int32_t aol_mode, aol_row_blocks, aol_seg_blocks;
+    int32_t reserved;
+} MuonChunkRun;
+
 int         muon_amd_abi_version(void);
 const char* muon_amd_last_error(void);
 /* One-time set-up on the current device: checks that it is a gfx950 (MUON_AMD_EDEVICE if not),
@@ -174,6 +223,7 @@ size_t muon_amd_sizeof_gemm_desc(void);
 size_t muon_amd_sizeof_tile_job(void);
 size_t muon_amd_sizeof_adam_desc(void);
 size_t muon_amd_sizeof_aol_desc(void);
+size_t muon_amd_sizeof_chunk_run(void);
 
 /* Elements each block of the flat elementwise launches covers (momentum, apply, adam), and
  * the edge of the square tile of the normalise/transposing launch. */
@@ -273,6 +323,16 @@ int muon_amd_ns_gemm(const MuonGemmDesc* descs_dev, const MuonTileJob* jobs_dev,
 int muon_amd_apply(const MuonMatDesc* descs_dev, const int32_t* block_prefix_dev, int nmat,
                    int nblocks, float lr, float wd_factor, const float* scalars_dev /* {lr, wd_factor} */,
                    void* stream);
+
+/* Every launch of a chunk, in order, from one call: momentum (left out with skip_momentum != 0), norm,
+ * normalise, the products of run->steps iterations with the parameter step in the last (or, without
+ * iterations, muon_amd_apply).  The float arguments are those of the entry points above; scalars_dev:
+ * NULL, or device memory holding {one_minus_beta, beta, lr, wd_factor}.  events: NULL, or HIP events
+ * (hipEvent_t), two per launch in order, recorded around each.  Nothing of *run is kept.
+ * Returns the first failing launch's code.                                                   */
+int muon_amd_run_chunk(const MuonChunkRun* run, float one_minus_beta, float beta, int nesterov, int mutate_grad,
+                       float eps, float lr, float wd_factor, const float* scalars_dev, int skip_momentum,
+                       void* const* events, void* stream);
 
 /* ---- AOL rescaling (muon.py:776-785; no counterpart kernel in the reference, which leaves
  *      these tensor expressions to torch.compile) ------------------------------------------- */

@@ -51,6 +51,17 @@ AOL_DESC = np.dtype(
      ("m_p", "<i4"), ("n_p", "<i4"), ("ld_n", "<i4"), ("ld_m", "<i4"), ("ld_rowsum", "<i4"), ("reserved", "<i4")],
     align=True)
 
+CHUNK_LAUNCH = np.dtype([("jobs", "<u8"), ("njobs", "<i4"), ("tile_class", "<i4"), ("split_slots", "<i4"),
+                         ("reserved", "<i4")], align=True)
+LAUNCH_KINDS = ("gram", "poly", "update", "gram_rowsum", "poly_full")       # order of MuonChunkRun.launches
+CHUNK_RUN = np.dtype(
+    [("mats", "<u8"), ("block_prefix", "<u8"), ("tile_prefix", "<u8"), ("gemm", "<u8", (7,)),
+     ("launches", CHUNK_LAUNCH, (len(LAUNCH_KINDS),)), ("scalars", "<u8"), ("split_partials", "<u8"), ("split_counters", "<u8"),
+     ("aol", "<u8"), ("aol_row_prefix", "<u8"), ("aol_seg_prefix", "<u8"), ("nmat", "<i4"), ("nblocks", "<i4"), ("ntiles", "<i4"),
+     ("steps", "<i4"), ("flags", "<i4"), ("split_slots", "<i4"), ("aol_mode", "<i4"), ("aol_row_blocks", "<i4"),
+     ("aol_seg_blocks", "<i4"), ("reserved", "<i4")],
+    align=True)
+
 _c_int = ctypes.c_int
 _c_float = ctypes.c_float
 _vp = ctypes.c_void_p
@@ -65,6 +76,8 @@ SIGNATURES = {
     "muon_amd_sizeof_tile_job": (ctypes.c_size_t, []),
     "muon_amd_sizeof_adam_desc": (ctypes.c_size_t, []),
     "muon_amd_sizeof_aol_desc": (ctypes.c_size_t, []),
+    "muon_amd_sizeof_chunk_run": (ctypes.c_size_t, []),
+    "muon_amd_run_chunk": (_c_int, [_vp, _c_float, _c_float, _c_int, _c_int, _c_float, _c_float, _c_float, _vp, _c_int, _vp, _vp]),
     "muon_amd_aol_rows_per_block": (_c_int, []),
     "muon_amd_validate_aol": (_c_int, [_vp, _c_int, _vp, _vp]),
     "muon_amd_aol_rowsum": (_c_int, [_vp, _vp, _c_int, _c_int, _c_float, _vp]),
@@ -114,7 +127,7 @@ def load():
         raise MuonAmdError(f"ABI mismatch: library {lib.muon_amd_abi_version()}, binding {ABI_VERSION}")
     for dt, fn in ((MAT_DESC, lib.muon_amd_sizeof_mat_desc), (GEMM_DESC, lib.muon_amd_sizeof_gemm_desc),
                    (TILE_JOB, lib.muon_amd_sizeof_tile_job), (ADAM_DESC, lib.muon_amd_sizeof_adam_desc),
-                   (AOL_DESC, lib.muon_amd_sizeof_aol_desc)):
+                   (AOL_DESC, lib.muon_amd_sizeof_aol_desc), (CHUNK_RUN, lib.muon_amd_sizeof_chunk_run)):
         if dt.itemsize != fn():
             raise MuonAmdError(f"struct layout mismatch: binding {dt.itemsize} bytes, library {fn()}")
     _lib = lib

@@ -24,6 +24,11 @@ void set_error(const char* fmt, ...);
 // Checks the launch that was just enqueued.
 int check_launch(const char* what);
 
+// muon_amd_norm_finalize that also clears `nclear` words (the counters of split reductions: every launch
+// leaves them zero, but one that died half way must not poison every later step).
+int launch_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags, int32_t* clear, int nclear,
+                         hipStream_t stream);
+
 // ---- bf16 <-> fp32 -----------------------------------------------------------------------
 // bf16 values are carried as uint16_t (upper half of the fp32 pattern).  The fp32 -> bf16
 // conversion is round-to-nearest-even with NaN preserved (v_cvt_pk_bf16_f32 on gfx950).

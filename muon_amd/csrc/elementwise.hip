@@ -214,7 +214,9 @@ __global__ __launch_bounds__(EW_THREADS) void momentum_kernel(
 // norm finalize: muon.py:282  (X.norm(dim=(-2,-1)) + 1e-7)
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void norm_finalize_kernel(const MuonMatDesc* __restrict__ descs,
-                                                            float eps, int round_reference) {
+                                                            float eps, int round_reference,
+                                                            int32_t* __restrict__ clear, int nclear) {
+    for (int i = blockIdx.x * 64 + threadIdx.x; i < nclear; i += gridDim.x * 64) clear[i] = 0;
     const MuonMatDesc d = descs[blockIdx.x];
     float s = 0.f;
     for (int i = d.part_begin + threadIdx.x; i < d.part_end; i += 64) s += d.partials[i];
@@ -543,6 +545,15 @@ __global__ __launch_bounds__(EW_THREADS) void adam_kernel(const MuonAdamDesc* __
         adam_block<float>(d, block_base, neg_lr, wd_factor, w1, w2, eps, bias1, bias2);
 }
 
+int launch_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags, int32_t* clear, int nclear,
+                         hipStream_t stream) {
+    MUON_REQUIRE(descs_dev, "norm_finalize: null table");
+    MUON_REQUIRE(nmat > 0, "norm_finalize: nmat=%d", nmat);
+    hipLaunchKernelGGL(norm_finalize_kernel, dim3(nmat), dim3(64), 0, stream, descs_dev, eps,
+                       (flags & MUON_AMD_NORM_UNIT) ? 2 : ((flags & MUON_AMD_ROUND_REFERENCE) ? 1 : 0), clear, nclear);
+    return check_launch("norm_finalize");
+}
+
 }  // namespace muon_amd
 
 using namespace muon_amd;
@@ -610,12 +621,7 @@ int muon_amd_momentum(const MuonMatDesc* descs_dev, const int32_t* block_prefix_
 
 int muon_amd_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags,
                            void* stream) {
-    MUON_REQUIRE(descs_dev, "norm_finalize: null table");
-    MUON_REQUIRE(nmat > 0, "norm_finalize: nmat=%d", nmat);
-    hipLaunchKernelGGL(norm_finalize_kernel, dim3(nmat), dim3(64), 0,
-                       static_cast<hipStream_t>(stream), descs_dev, eps,
-                       (flags & MUON_AMD_NORM_UNIT) ? 2 : ((flags & MUON_AMD_ROUND_REFERENCE) ? 1 : 0));
-    return check_launch("norm_finalize");
+    return launch_norm_finalize(descs_dev, nmat, eps, flags, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 int muon_amd_normalize(const MuonMatDesc* descs_dev, const int32_t* tile_prefix_dev, int nmat,

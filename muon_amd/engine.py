@@ -130,6 +130,8 @@ class _ChunkRuntime:
             self.aol_ptr, self.aol_row_prefix_ptr, self.aol_seg_prefix_ptr = (b + o for o in offs[3 + len(kinds):6 + len(kinds)])
         self.single_prefix_ptr = b + offs[-1]
         self.single_blocks = single[:, 1].tolist()
+        self.chunk_run = self._chunk_run(base)
+        self.run_ptr = self.chunk_run.ctypes.data
         self.mat_dev = None
         self.mat_key = None
         self.mat_host = None
@@ -153,6 +155,7 @@ class _ChunkRuntime:
                    "validate_mats")
         if self.mat_dev is None:
             self.mat_dev = torch.empty(d.nbytes, dtype=torch.uint8, device=self.device)
+            self.chunk_run["mats"] = self.mat_dev.data_ptr()
         self.staging.upload(d, self.mat_dev)
         self.mat_key = key
         self.mat_host = d
@@ -196,94 +199,81 @@ class _ChunkRuntime:
         sz = 2 if self.src_dtypes[k] == _lib.SRC_BF16 else 4
         _launch("momentum", lay.numel * (sz + 2 + (2 * sz if self.present[k][0] else 0)), call)
 
+    def _chunk_run(self, base):
+        """The struct muon_amd_run_chunk takes (host memory, kept with the arrays it points to)."""
+        c = self.chunk
+        r = np.zeros((), dtype=_lib.CHUNK_RUN)
+        r["block_prefix"], r["tile_prefix"] = self.block_prefix_ptr, self.tile_prefix_ptr
+        r["gemm"] = self.gemm_ptr
+        for kind, ln in c.launches.items():
+            e = r["launches"][_lib.LAUNCH_KINDS.index(kind)]
+            e["jobs"], e["njobs"], e["tile_class"], e["split_slots"] = self.jobs_ptr[kind], len(ln.jobs), ln.tile_class, ln.split_slots
+        self._phase_scalars = np.array([c.phase_scalars(ph, it) for it in range(c.steps)
+                                        for ph in (_plan.PH_SYRK, _plan.PH_POLY, _plan.PH_UPD_EVEN)], dtype=np.float32)
+        r["scalars"] = self._phase_scalars.ctypes.data if c.steps else 0
+        if self.split_slots:
+            r["split_partials"], r["split_counters"] = self.split_partials_ptr, self.split_counters_ptr
+            r["split_slots"] = self.split_slots
+        if c.aol:
+            r["aol"], r["aol_row_prefix"], r["aol_seg_prefix"] = self.aol_ptr, self.aol_row_prefix_ptr, self.aol_seg_prefix_ptr
+            r["aol_mode"] = _lib.AOL_ROWS_ONLY if c.variant == "aol4_rows" else _lib.AOL_SYMMETRIC
+            r["aol_row_blocks"], r["aol_seg_blocks"] = int(c.aol_row_prefix[-1]), int(c.aol_seg_prefix[-1])
+        r["nmat"], r["nblocks"], r["ntiles"], r["steps"] = c.nmat, c.nblocks, c.ntiles, c.steps
+        r["flags"] = _lib.ROUND_REFERENCE if c.reference_rounding else _lib.ROUND_FUSED
+        return r
+
+    def _launches(self, skip_momentum):
+        """(label, algorithmic work) of the launches muon_amd_run_chunk makes, in order: flops for the
+        products (the minimum given symmetry, on the unpadded sizes), bytes for the others."""
+        c = self.chunk
+        elts = sum(lay.numel for lay in c.layouts)
+        padded = sum(lay.mp * lay.np_ for lay in c.layouts)
+        # gradient, momentum (read + write) and parameter (read + write) in their storage type, the bf16
+        # update written once and read once
+        store = [2 if t == _lib.SRC_BF16 else 4 for t in self.src_dtypes]
+        out = []
+        if not skip_momentum:
+            out.append(("momentum", sum(lay.numel * (sz + 2 + (2 * sz if has_m else 0))
+                                        for lay, sz, (has_m, _, _) in zip(c.layouts, store, self.present))))
+        out += [("norm_finalize", c.nblocks * 4), ("normalize", elts * 2 + padded * 2)]
+        syrk = sum(lay.m * (lay.m + 1) * lay.n for lay in c.layouts)
+        poly = sum(lay.m * lay.m * (lay.m + 1) for lay in c.layouts)
+        update = sum(2 * lay.m * lay.m * lay.n for lay in c.layouts)
+        for it in range(c.steps):
+            first_aol = c.aol and it == 0
+            out.append(("ns_gemm/syrk", syrk))
+            if first_aol:
+                out += [("aol_rowsum_finalize", sum(lay.mp * (lay.mp // _plan.ROWSUM_SLOT) * 4 for lay in c.layouts)),
+                        ("aol_rescale", sum(lay.mp * lay.mp * 4 for lay in c.layouts) + 4 * padded)]
+            out.append(("ns_gemm/poly", 2 * poly if first_aol and c.variant == "aol4_rows" else poly))
+            out.append(("ns_gemm/update_apply" if it == c.steps - 1 else "ns_gemm/update", update))
+        if not c.steps:
+            out.append(("apply", sum(lay.numel * (2 + (2 * sz if has_p else 0) + (2 if has_o else 0))
+                                     for lay, sz, (_, has_p, has_o) in zip(c.layouts, store, self.present))))
+        return out
+
     def run(self, one_minus_beta, beta, nesterov, mutate_grad, eps, lr, wd_factor, scalars_ptr=0,
             momentum_done=frozenset()):
         """Enqueue the chunk's launches.  scalars_ptr: device address of {one_minus_beta, beta, lr,
         wd_factor}, read by the kernels at run time in place of the by-value arguments.
         momentum_done: matrices (positions in the chunk) whose momentum stage already ran."""
-        lib = _lib.load()
-        c = self.chunk
-        s = _stream_ptr(self.device)
-        sc_mom = scalars_ptr or None
-        sc_apply = scalars_ptr + 8 if scalars_ptr else None
-        flags = _lib.ROUND_REFERENCE if c.reference_rounding else _lib.ROUND_FUSED
-        mats = self.mat_dev.data_ptr()
-        elts = sum(lay.numel for lay in c.layouts)
-        padded = sum(lay.mp * lay.np_ for lay in c.layouts)
-        # algorithmic bytes: gradient, momentum (read + write) and parameter (read + write) in
-        # their storage type, the bf16 update written once and read once
-        store = [2 if t == _lib.SRC_BF16 else 4 for t in self.src_dtypes]
-        mom_bytes = sum(lay.numel * (sz + 2 + (2 * sz if has_m else 0))
-                        for lay, sz, (has_m, _, _) in zip(c.layouts, store, self.present))
-        apply_bytes = sum(lay.numel * (2 + (2 * sz if has_p else 0) + (2 if has_o else 0))
-                          for lay, sz, (_, has_p, has_o) in zip(c.layouts, store, self.present))
-        if self.split_slots:
-            # every launch leaves the counters of the split groups zero; clearing them here as well
-            # (a fill kernel, recordable into a graph) keeps a launch that died half way from
-            # poisoning every later step
-            self.split_counters.zero_()
-        if not momentum_done:
-            _launch("momentum", mom_bytes, lambda: _lib.check(lib.muon_amd_momentum(
-                mats, self.block_prefix_ptr, c.nmat, c.nblocks, one_minus_beta, beta, int(nesterov),
-                int(mutate_grad), sc_mom, s), "momentum"))
-        else:
-            for k in range(c.nmat):
+        if momentum_done:
+            for k in range(self.chunk.nmat):
                 if k not in momentum_done:
                     self.momentum_of(k, one_minus_beta, beta, nesterov, mutate_grad, scalars_ptr)
-        norm_flags = flags | (_lib.NORM_UNIT if c.aol else 0)
-        _launch("norm_finalize", c.nblocks * 4, lambda: _lib.check(lib.muon_amd_norm_finalize(
-            mats, c.nmat, eps, norm_flags, s), "norm_finalize"))
-        _launch("normalize", elts * 2 + padded * 2, lambda: _lib.check(lib.muon_amd_normalize(
-            mats, self.tile_prefix_ptr, c.nmat, c.ntiles, s), "normalize"))
-        flops = {
-            _plan.PH_SYRK: sum(lay.m * (lay.m + 1) * lay.n for lay in c.layouts),
-            _plan.PH_POLY: sum(lay.m * lay.m * (lay.m + 1) for lay in c.layouts),
-        }
-        f_upd = sum(2 * lay.m * lay.m * lay.n for lay in c.layouts)
-
-        def gemm(name, ph, it, kind, work, extra_flags=0):
-            al, be, ga = c.phase_scalars(ph, it)
-            ln = c.launches[kind]
-            _launch(name, work, lambda: _lib.check(lib.muon_amd_ns_gemm(
-                self.gemm_ptr[ph], self.jobs_ptr[kind], len(ln.jobs), ln.tile_class, al, be, ga, flags | extra_flags,
-                self.split_partials_ptr if ln.split_slots else None, self.split_counters_ptr if ln.split_slots else None,
-                s), "ns_gemm"))
-
-        for it in range(c.steps):
-            first_aol = c.aol and it == 0
-            gemm("ns_gemm/syrk", _plan.PH_SYRK if it % 2 == 0 else _plan.PH_SYRK_ODD, it,
-                 "gram_rowsum" if first_aol else "gram", flops[_plan.PH_SYRK], _lib.GEMM_ROWSUM if first_aol else 0)
-            if first_aol:
-                # muon.py:776-785: the row sums of |A| come out of the product's epilogue as partial
-                # sums (one small launch adds them up), then X and A are rescaled in place (A becomes
-                # the Gram matrix of the rescaled X, so this iteration needs no second X X^T)
-                gram_bytes = sum(lay.mp * lay.mp * 2 for lay in c.layouts)
-                part_bytes = sum(lay.mp * (lay.mp // _plan.ROWSUM_SLOT) * 4 for lay in c.layouts)
-                _launch("aol_rowsum_finalize", part_bytes, lambda: _lib.check(lib.muon_amd_aol_rowsum_finalize(
-                    self.aol_ptr, self.aol_row_prefix_ptr, c.nmat, int(c.aol_row_prefix[-1]), eps, s),
-                    "aol_rowsum_finalize"))
-                mode = _lib.AOL_ROWS_ONLY if c.variant == "aol4_rows" else _lib.AOL_SYMMETRIC
-                _launch("aol_rescale", 2 * gram_bytes + 4 * padded, lambda: _lib.check(lib.muon_amd_aol_rescale(
-                    self.aol_ptr, self.aol_seg_prefix_ptr, c.nmat, int(c.aol_seg_prefix[-1]), mode, s),
-                    "aol_rescale"))
-            if first_aol and c.variant == "aol4_rows":
-                # A / s is not symmetric: c * A A^T + b * A over every tile, no mirrored store
-                gemm("ns_gemm/poly", _plan.PH_POLY_FULL, it, "poly_full", 2 * flops[_plan.PH_POLY])
-            else:
-                gemm("ns_gemm/poly", _plan.PH_POLY, it, "poly", flops[_plan.PH_POLY])
-            if it == c.steps - 1:
-                # the last update product takes the parameter step in its epilogue (muon.py:14, 98-99)
-                al, be, _ = c.phase_scalars(_plan.PH_UPD_LAST, it)
-                _launch("ns_gemm/update_apply", f_upd, lambda: _lib.check(lib.muon_amd_ns_gemm_apply(
-                    self.gemm_ptr[_plan.PH_UPD_LAST], self.jobs_ptr["update"], len(c.launches["update"].jobs),
-                    c.launches["update"].tile_class, al, be,
-                    flags, mats, lr, wd_factor, sc_apply, s), "ns_gemm_apply"))
-                return
-            gemm("ns_gemm/update", _plan.PH_UPD_EVEN if it % 2 == 0 else _plan.PH_UPD_ODD, it, "update", f_upd,
-                 _lib.GEMM_Q_KMAJOR)
-        # no iteration (steps == 0): the parameter step is a launch of its own
-        _launch("apply", apply_bytes, lambda: _lib.check(lib.muon_amd_apply(
-            mats, self.block_prefix_ptr, c.nmat, c.nblocks, lr, wd_factor, sc_apply, s), "apply"))
+        events = None
+        if PROFILE is not None:
+            launches = self._launches(bool(momentum_done))
+            pairs = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in launches]
+            for pair in pairs:
+                for e in pair:
+                    e.record()                    # (torch creates the event when it is first recorded)
+            events = np.array([e.cuda_event for pair in pairs for e in pair], dtype=np.uint64)
+        _lib.check(_lib.load().muon_amd_run_chunk(
+            self.run_ptr, one_minus_beta, beta, int(nesterov), int(mutate_grad), eps, lr, wd_factor, scalars_ptr or None,
+            int(bool(momentum_done)), events.ctypes.data if events is not None else None, _stream_ptr(self.device)), "run_chunk")
+        if events is not None:
+            PROFILE.extend((label, work, *pair) for (label, work), pair in zip(launches, pairs))
 
 
 class MuonGroupEngine:
