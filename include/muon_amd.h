@@ -334,6 +334,19 @@ int muon_amd_run_chunk(const MuonChunkRun* run, float one_minus_beta, float beta
                        float eps, float lr, float wd_factor, const float* scalars_dev, int skip_momentum,
                        void* const* events, void* stream);
 
+/* ---- small matrices: the whole step of a matrix in one workgroup ---------------------------
+ * muon_amd_small_class: 32, 64 or 128 (the short side rounded up) for a matrix that fits the LDS of a
+ * CU with its iterate and two Gram matrices, 0 for one that does not.                          */
+int muon_amd_small_class(int rows, int cols);
+int muon_amd_validate_small(const MuonMatDesc* descs_host, int nmat, int small_class, int max_long_side);
+/* Momentum, norm, normalise, `steps` iterations with the coefficients coeffs = {a, b, c} (host memory) and
+ * the parameter step for nmat matrices of small_class at most whose long sides are at most
+ * max_long_side, one workgroup each; of a descriptor grad, momentum, param, out, rows, cols, src_dtype
+ * and scale are used.  Same bits as the launches of muon_amd_run_chunk.                       */
+int muon_amd_small_step(const MuonMatDesc* descs_dev, int nmat, int small_class, int max_long_side, int steps,
+                        const float* coeffs, int flags, float one_minus_beta, float beta, int nesterov, int mutate_grad,
+                        float eps, float lr, float wd_factor, const float* scalars_dev, void* stream);
+
 /* ---- AOL rescaling (muon.py:776-785; no counterpart kernel in the reference, which leaves
  *      these tensor expressions to torch.compile) ------------------------------------------- */
 /* Rows each block of the two launches below covers (one wavefront per row). */

@@ -78,6 +78,10 @@ SIGNATURES = {
     "muon_amd_sizeof_aol_desc": (ctypes.c_size_t, []),
     "muon_amd_sizeof_chunk_run": (ctypes.c_size_t, []),
     "muon_amd_run_chunk": (_c_int, [_vp, _c_float, _c_float, _c_int, _c_int, _c_float, _c_float, _c_float, _vp, _c_int, _vp, _vp]),
+    "muon_amd_small_class": (_c_int, [_c_int, _c_int]),
+    "muon_amd_validate_small": (_c_int, [_vp, _c_int, _c_int, _c_int]),
+    "muon_amd_small_step": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _c_float, _c_float, _c_int, _c_int,
+                                     _c_float, _c_float, _c_float, _vp, _vp]),
     "muon_amd_aol_rows_per_block": (_c_int, []),
     "muon_amd_validate_aol": (_c_int, [_vp, _c_int, _vp, _vp]),
     "muon_amd_aol_rowsum": (_c_int, [_vp, _vp, _c_int, _c_int, _c_float, _vp]),

@@ -29,6 +29,9 @@ int check_launch(const char* what);
 int launch_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags, int32_t* clear, int nclear,
                          hipStream_t stream);
 
+// Raises the dynamic-LDS limit of the kernels of small.hip (part of muon_amd_init).
+int raise_small_limits();
+
 // ---- bf16 <-> fp32 -----------------------------------------------------------------------
 // bf16 values are carried as uint16_t (upper half of the fp32 pattern).  The fp32 -> bf16
 // conversion is round-to-nearest-even with NaN preserved (v_cvt_pk_bf16_f32 on gfx950).

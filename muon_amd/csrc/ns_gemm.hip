@@ -1057,6 +1057,7 @@ static int device_setup(const DeviceState** out) {
         int rc = raise_lds_limits<Cfg0>();
         if (rc == MUON_AMD_OK) rc = raise_lds_limits<Cfg1>();
         if (rc == MUON_AMD_OK) rc = raise_lds_limits<Cfg2>();
+        if (rc == MUON_AMD_OK) rc = raise_small_limits();
         if (rc != MUON_AMD_OK) return rc;
         void* ptr = nullptr;
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || ptr == nullptr) {

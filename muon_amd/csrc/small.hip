@@ -1,0 +1,442 @@
+// The whole Muon step of a small matrix in one workgroup: momentum, norm, normalise, the Newton-Schulz
+// iteration and the parameter step, with the iterate and its Gram matrix in LDS throughout.
+//
+// A matrix whose short side is at most 128 and whose iterate fits the 160 KB of LDS of a CU beside two
+// Gram matrices needs nothing from other CUs between two products, so the 17 launches of the general
+// path (4 us each on the GPU, 3.3 us each on the host, whatever the size) become one.  What bounds it
+// is latency: the loads of gradient and momentum, then chains of LDS reads and MFMAs.
+// muon_update of a 64 x 64 x 3 x 3 filter: 106 us in separate launches.
+//
+// Every rounding and every order of summation is the general path's (elementwise.hip, ns_gemm.hip): the
+// sum of squares goes by blocks of 8192 elements and 256 threads, the products accumulate k-step after
+// k-step, so a matrix gets the same bits on either path.
+#include "common.h"
+
+namespace muon_amd {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4s __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int SMALL_THREADS = 512, SMALL_WAVES = SMALL_THREADS / 64;
+constexpr int SUM_BLOCK = 8192;                     // elements per partial sum (EW_BLOCK_ELEMS) ...
+constexpr int SUM_THREADS = 256, SUM_ITERS = 8;     // ... and how its threads share them (4 in a row each)
+constexpr int SMALL_LDS_MAX = 163840;
+constexpr int SMALL_MAX_BLOCKS = 16;                // partial sums of the largest matrix that fits
+
+// Rows are padded by 16 bytes: 16-byte reads of one chunk of 8 consecutive rows hit all banks.
+__host__ __device__ constexpr int small_pitch(int cols) { return cols * 2 + 16; }
+static size_t small_lds_bytes(int mp, int np) {
+    return static_cast<size_t>(mp) * small_pitch(np) + 2 * static_cast<size_t>(mp) * small_pitch(mp) +
+           SMALL_MAX_BLOCKS * 4 * sizeof(float);
+}
+
+template <typename T>
+struct SmallIo;
+template <>
+struct SmallIo<float> {
+    static constexpr uintptr_t kAlign = 16;
+    static __device__ __forceinline__ f32x4s ld4(const float* p) { return *(const __attribute__((address_space(1))) f32x4s*)(p); }
+    static __device__ __forceinline__ void st4(float* p, f32x4s v) { *(__attribute__((address_space(1))) f32x4s*)(p) = v; }
+    static __device__ __forceinline__ float ld(const float* p) { return *p; }
+    static __device__ __forceinline__ void st(float* p, float v) { *p = v; }
+    static __device__ __forceinline__ float rnd(float v) { return v; }
+};
+template <>
+struct SmallIo<uint16_t> {
+    static constexpr uintptr_t kAlign = 8;
+    static __device__ __forceinline__ f32x4s ld4(const uint16_t* p) {
+        const u32x2 r = *(const __attribute__((address_space(1))) u32x2*)(p);
+        return f32x4s{bf_lo(r.x), bf_hi(r.x), bf_lo(r.y), bf_hi(r.y)};
+    }
+    static __device__ __forceinline__ void st4(uint16_t* p, f32x4s v) {
+        *(__attribute__((address_space(1))) u32x2*)(p) = u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
+    }
+    static __device__ __forceinline__ float ld(const uint16_t* p) { return bf2f(*p); }
+    static __device__ __forceinline__ void st(uint16_t* p, float v) { *p = f2bf(v); }
+    static __device__ __forceinline__ float rnd(float v) { return round_bf(v); }
+};
+
+__device__ __forceinline__ bool small_aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+
+// 16 bytes of an LDS row as an MFMA operand: lane l holds k = 8 (l / 32) .. + 7 of row l % 32.
+__device__ __forceinline__ bf16x8 row_frag(const char* base, int pitch, int row0, int ks, int lane) {
+    return *reinterpret_cast<const bf16x8*>(base + (row0 + (lane & 31)) * pitch + ks * 32 + (lane >> 5) * 16);
+}
+// The same from a k-major operand (rows = k): two transposing reads of 4 rows x 16 columns per 16 lanes.
+__device__ __forceinline__ bf16x8 col_frag(const char* base, int pitch, int col0, int ks, int lane) {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const char* const p = base + (ks * 16 + (lane >> 5) * 8 + ((lane & 15) >> 2)) * pitch +
+                          (col0 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4) * 2;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * pitch)));
+    return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
+}
+__device__ __forceinline__ f32x16 zero16() {
+    f32x16 z;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[i] = 0.f;
+    return z;
+}
+// A 32 x 32 tile of packed bf16 pairs (lane = row l % 32, pair 2q + i = columns 8q + 4 (l / 32) + 2i) to LDS rows.
+__device__ __forceinline__ void tile_store(char* base, int pitch, int row0, int col0, int lane, const uint32_t (&po)[8]) {
+    char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 4) * 2;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x2*>(p + q * 16) = u32x2{po[2 * q], po[2 * q + 1]};
+}
+// o = alpha * acc + beta * D as the epilogue of the GEMM kernel rounds it; D from LDS in the same layout.
+template <bool ROUND>
+__device__ __forceinline__ void tile_add(uint32_t (&po)[8], const f32x16& acc, float alpha, float beta, const char* base,
+                                         int pitch, int row0, int col0, int lane) {
+    const char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 4) * 2;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const u32x2 dv = *reinterpret_cast<const u32x2*>(p + q * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int k = 2 * q + i;
+            const uint32_t dk = i ? dv.y : dv.x;
+            if constexpr (ROUND) {
+                const uint32_t t1 = pack2bf(alpha * acc[2 * k], alpha * acc[2 * k + 1]);
+                const uint32_t t2 = pack2bf(beta * bf_lo(dk), beta * bf_hi(dk));
+                po[k] = pack2bf(bf_lo(t1) + bf_lo(t2), bf_hi(t1) + bf_hi(t2));
+            } else {
+                po[k] = pack2bf(fmaf(alpha, acc[2 * k], beta * bf_lo(dk)), fmaf(alpha, acc[2 * k + 1], beta * bf_hi(dk)));
+            }
+        }
+    }
+}
+
+// X from gradient and momentum (muon.py:9-10, 277-279), and the partial sums of squares: block b of 8192
+// elements by threads 256 (b % 2) .. + 255.
+template <typename T>
+__device__ __forceinline__ void small_load(const MuonMatDesc& d, char* X, int pitch, bool wide, float w, float beta,
+                                           int nesterov, int mutate_grad, float* sums, int tid) {
+    typedef SmallIo<T> S;
+    const int numel = d.rows * d.cols, cols = d.cols;
+    T* const g = static_cast<T*>(d.grad);
+    T* const mom = static_cast<T*>(d.momentum);
+    const bool has_m = mom != nullptr, write_g = has_m && nesterov && mutate_grad;
+    const bool aligned = small_aligned(g, S::kAlign) && small_aligned(mom, S::kAlign);
+    const int t = tid & (SUM_THREADS - 1);
+    for (int b = tid / SUM_THREADS; b * SUM_BLOCK < numel; b += SMALL_THREADS / SUM_THREADS) {
+        f32x4s gv[SUM_ITERS], mv[SUM_ITERS];
+#pragma unroll
+        for (int it = 0; it < SUM_ITERS; ++it) {
+            const int e = b * SUM_BLOCK + (it * SUM_THREADS + t) * 4;
+            gv[it] = mv[it] = f32x4s{0.f, 0.f, 0.f, 0.f};
+            if (aligned && e + 4 <= numel) {
+                gv[it] = S::ld4(g + e);
+                if (has_m) mv[it] = S::ld4(mom + e);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (e + k < numel) {
+                        gv[it][k] = S::ld(g + e + k);
+                        if (has_m) mv[it][k] = S::ld(mom + e + k);
+                    }
+            }
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int it = 0; it < SUM_ITERS; ++it) {
+            const int e = b * SUM_BLOCK + (it * SUM_THREADS + t) * 4;
+            if (e >= numel) continue;
+            f32x4s gg = gv[it], mm = mv[it];
+            int r = e / cols, c = e - r * cols;
+            const bool whole = e + 4 <= numel;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float u = gg[k];
+                if (has_m) {
+                    mm[k] = S::rnd(lerp_torch(mm[k], gg[k], w));            // momentum.lerp_(grad, 1 - beta)
+                    u = mm[k];
+                    if (nesterov) u = gg[k] = S::rnd(lerp_torch(gg[k], mm[k], beta));   // grad.lerp_(momentum, beta)
+                }
+                const uint16_t ub = f2bf(u);
+                if (whole || e + k < numel) {
+                    const float uf = bf2f(ub);
+                    ss = fmaf(uf, uf, ss);
+                    *reinterpret_cast<uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2) = ub;
+                }
+                if (++c == cols) {
+                    c = 0;
+                    ++r;
+                }
+            }
+            if (aligned && whole) {
+                if (has_m) S::st4(mom + e, mm);
+                if (write_g) S::st4(g + e, gg);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (e + k < numel) {
+                        if (has_m) S::st(mom + e + k, mm[k]);
+                        if (write_g) S::st(g + e + k, gg[k]);
+                    }
+            }
+        }
+        ss = wave_sum(ss);
+        if ((tid & 63) == 0) sums[b * 4 + (t >> 6)] = ss;
+    }
+}
+
+// The parameter step (muon.py:14, 98-99) from the result in LDS, 4 elements in a row per access.
+template <typename T>
+__device__ __forceinline__ void small_apply(const MuonMatDesc& d, const char* X, int pitch, bool wide, float neg_lr,
+                                            float wd_factor, int tid) {
+    typedef SmallIo<T> S;
+    const int numel = d.rows * d.cols, cols = d.cols;
+    T* const p = static_cast<T*>(d.param);
+    uint16_t* const out = d.out;
+    const bool aligned = small_aligned(p, S::kAlign) && small_aligned(out, 8);
+    constexpr int UN = 4;
+    for (int e0 = tid * 4; e0 < numel; e0 += SMALL_THREADS * 4 * UN) {
+        f32x4s pv[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const int e = e0 + u * SMALL_THREADS * 4;
+            pv[u] = f32x4s{0.f, 0.f, 0.f, 0.f};
+            if (!p) continue;
+            if (aligned && e + 4 <= numel) {
+                pv[u] = S::ld4(p + e);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (e + k < numel) pv[u][k] = S::ld(p + e + k);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const int e = e0 + u * SMALL_THREADS * 4;
+            if (e >= numel) continue;
+            int r = e / cols, c = e - r * cols;
+            float us[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                us[k] = 0.f;
+                if (e + k < numel) {
+                    const uint16_t o = *reinterpret_cast<const uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2);
+                    us[k] = round_bf(bf2f(o) * d.scale);
+                }
+                pv[u][k] = S::rnd(fmaf(neg_lr, us[k], S::rnd(pv[u][k] * wd_factor)));
+                if (++c == cols) {
+                    c = 0;
+                    ++r;
+                }
+            }
+            if (aligned && e + 4 <= numel) {
+                if (p) S::st4(p + e, pv[u]);
+                if (out) *(__attribute__((address_space(1))) u32x2*)(out + e) = u32x2{pack2bf(us[0], us[1]), pack2bf(us[2], us[3])};
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (e + k < numel) {
+                        if (p) S::st(p + e + k, pv[u][k]);
+                        if (out) out[e + k] = f2bf(us[k]);
+                    }
+            }
+        }
+    }
+}
+
+// One workgroup per matrix.  MP: its short side rounded up to 32, 64 or 128; the long side is rounded up to
+// 64 (a k-block of the general path).  The products are shared out by 32 x 32 tiles of the Gram matrix and
+// by blocks of 32 columns of X; X' overwrites X, whose columns depend on nothing but themselves and B.
+template <int MP, bool ROUND>
+__global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
+    const MuonMatDesc* __restrict__ descs, int steps, float ca, float cb, float cc, float w, float beta, int nesterov,
+    int mutate_grad, float eps, float neg_lr, float wd_factor, const float* __restrict__ sc) {
+    constexpr int MT = MP / 32, TILES = MT * MT, TPW = (TILES + SMALL_WAVES - 1) / SMALL_WAVES;
+    constexpr int PA = small_pitch(MP);
+    extern __shared__ __align__(16) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (sc) {   // {1 - beta, beta, lr, wd_factor} read at run time instead of the arguments
+        w = sc[0];
+        beta = sc[1];
+        neg_lr = -sc[2];
+        wd_factor = sc[3];
+    }
+    const MuonMatDesc d = descs[blockIdx.x];
+    const bool wide = d.rows <= d.cols;
+    const int m = wide ? d.rows : d.cols, n = wide ? d.cols : d.rows;
+    const int np = (n + 63) & ~63, px = small_pitch(np);
+    float* const sums = reinterpret_cast<float*>(lds);
+    char* const A = lds + SMALL_MAX_BLOCKS * 4 * sizeof(float);
+    char* const B = A + MP * PA;                     // c A, then the polynomial
+    char* const X = B + MP * PA;
+
+    if (m < MP || n < np) {
+        for (int o = tid * 16; o < MP * px; o += SMALL_THREADS * 16) *reinterpret_cast<u32x4*>(X + o) = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+    }
+    if (d.src_dtype == MUON_AMD_SRC_BF16) small_load<uint16_t>(d, X, px, wide, w, beta, nesterov, mutate_grad, sums, tid);
+    else small_load<float>(d, X, px, wide, w, beta, nesterov, mutate_grad, sums, tid);
+    __syncthreads();
+    float den;                                       // muon.py:282, as norm_finalize_kernel forms it
+    {
+        const int nblk = (d.rows * d.cols + SUM_BLOCK - 1) / SUM_BLOCK;
+        const float* const q = sums + lane * 4;
+        const float nrm = sqrtf(wave_sum(lane < nblk ? (q[0] + q[1]) + (q[2] + q[3]) : 0.f));
+        den = ROUND ? round_bf(round_bf(nrm) + eps) : nrm + eps;
+    }
+    const int chunks = np / 8;                       // of 8 columns
+    for (int i = tid; i < m * chunks; i += SMALL_THREADS) {
+        const int r = i / chunks, c = (i - r * chunks) * 8;
+        u32x4* const p = reinterpret_cast<u32x4*>(X + r * px + c * 2);
+        const u32x4 v = *p;
+        u32x4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float lo = c + 2 * k < n ? bf_lo(v[k]) / den : 0.f, hi = c + 2 * k + 1 < n ? bf_hi(v[k]) / den : 0.f;
+            o[k] = pack2bf(lo, hi);
+        }
+        *p = o;
+    }
+    __syncthreads();
+
+    for (int step = 0; step < steps; ++step) {
+        // A = X X^T and, where the reference rounds it, c A
+#pragma unroll
+        for (int s = 0; s < TPW; ++s) {
+            const int t = wave + s * SMALL_WAVES;
+            if (t >= TILES) continue;
+            const int i0 = t / MT * 32, j0 = t % MT * 32;
+            f32x16 acc = zero16();
+#pragma unroll 4
+            for (int ks = 0; ks < np / 16; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag(X, px, j0, ks, lane), row_frag(X, px, i0, ks, lane), acc, 0, 0, 0);
+            uint32_t po[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) po[k] = pack2bf(acc[2 * k], acc[2 * k + 1]);
+            tile_store(A, PA, i0, j0, lane, po);
+            if constexpr (ROUND) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) po[k] = pack2bf(cc * bf_lo(po[k]), cc * bf_hi(po[k]));
+                tile_store(B, PA, i0, j0, lane, po);
+            }
+        }
+        __syncthreads();
+        // B = b A + (c A) A
+        uint32_t pb[TPW][8];
+#pragma unroll
+        for (int s = 0; s < TPW; ++s) {
+            const int t = wave + s * SMALL_WAVES;
+            if (t >= TILES) continue;
+            const int i0 = t / MT * 32, j0 = t % MT * 32;
+            f32x16 acc = zero16();
+#pragma unroll
+            for (int ks = 0; ks < MP / 16; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag(A, PA, j0, ks, lane), row_frag(ROUND ? B : A, PA, i0, ks, lane), acc, 0, 0, 0);
+            tile_add<ROUND>(pb[s], acc, ROUND ? 1.f : cc, cb, A, PA, i0, j0, lane);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < TPW; ++s) {
+            const int t = wave + s * SMALL_WAVES;
+            if (t >= TILES) continue;
+            tile_store(B, PA, t / MT * 32, t % MT * 32, lane, pb[s]);
+        }
+        __syncthreads();
+        // X = a X + B X, a block of 32 columns at a time
+        for (int j0 = wave * 32; j0 < np; j0 += SMALL_WAVES * 32) {
+            bf16x8 q[MP / 16];
+#pragma unroll
+            for (int ks = 0; ks < MP / 16; ++ks) q[ks] = col_frag(X, px, j0, ks, lane);
+#pragma unroll
+            for (int i0 = 0; i0 < MP; i0 += 32) {
+                f32x16 acc = zero16();
+#pragma unroll
+                for (int ks = 0; ks < MP / 16; ++ks)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[ks], row_frag(B, PA, i0, ks, lane), acc, 0, 0, 0);
+                uint32_t po[8];
+                // (with one rounding the alpha of the general path is a run-time 1: beta * D is rounded before
+                // the sum there, and must not be contracted into it here)
+                float alpha = 1.f;
+                if constexpr (!ROUND) asm volatile("" : "+s"(alpha));
+                tile_add<ROUND>(po, acc, alpha, ca, X, px, i0, j0, lane);
+                tile_store(X, px, i0, j0, lane, po);
+            }
+        }
+        __syncthreads();
+    }
+    if (d.src_dtype == MUON_AMD_SRC_BF16) small_apply<uint16_t>(d, X, px, wide, neg_lr, wd_factor, tid);
+    else small_apply<float>(d, X, px, wide, neg_lr, wd_factor, tid);
+}
+
+template <int MP, bool ROUND>
+static int raise_small_limit() {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(ns_small_kernel<MP, ROUND>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            SMALL_LDS_MAX) != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("small: cannot raise dynamic LDS to %d bytes", SMALL_LDS_MAX);
+        return MUON_AMD_ELAUNCH;
+    }
+    return MUON_AMD_OK;
+}
+
+int raise_small_limits() {
+    int rc = raise_small_limit<32, true>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<32, false>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<64, true>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<64, false>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<128, true>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<128, false>();
+    return rc;
+}
+
+}  // namespace muon_amd
+
+using namespace muon_amd;
+
+extern "C" {
+
+int muon_amd_small_class(int rows, int cols) {
+    if (rows <= 0 || cols <= 0) return 0;
+    const int m = rows < cols ? rows : cols;
+    const int64_t n = rows < cols ? cols : rows;
+    const int mp = m <= 32 ? 32 : m <= 64 ? 64 : m <= 128 ? 128 : 0;
+    if (!mp || n > 65536 || (static_cast<int64_t>(rows) * cols + SUM_BLOCK - 1) / SUM_BLOCK > SMALL_MAX_BLOCKS) return 0;
+    return small_lds_bytes(mp, static_cast<int>((n + 63) & ~63)) <= SMALL_LDS_MAX ? mp : 0;
+}
+
+int muon_amd_validate_small(const MuonMatDesc* descs, int nmat, int small_class, int max_long_side) {
+    MUON_REQUIRE(descs && nmat > 0, "validate_small: nmat=%d", nmat);
+    for (int i = 0; i < nmat; ++i) {
+        const MuonMatDesc& d = descs[i];
+        const int own = muon_amd_small_class(d.rows, d.cols);
+        MUON_REQUIRE(own && own <= small_class && (d.rows > d.cols ? d.rows : d.cols) <= max_long_side,
+                     "mat %d: %d x %d does not fit class %d with a long side of %d", i, d.rows, d.cols, small_class, max_long_side);
+        MUON_REQUIRE(d.grad && (d.param || d.out), "mat %d: null source or neither param nor out given", i);
+        MUON_REQUIRE(d.src_dtype == MUON_AMD_SRC_F32 || d.src_dtype == MUON_AMD_SRC_BF16, "mat %d: src_dtype=%d", i, d.src_dtype);
+    }
+    return MUON_AMD_OK;
+}
+
+int muon_amd_small_step(const MuonMatDesc* descs_dev, int nmat, int small_class, int max_long_side, int steps,
+                        const float* coeffs, int flags, float one_minus_beta, float beta, int nesterov, int mutate_grad,
+                        float eps, float lr, float wd_factor, const float* scalars_dev, void* stream) {
+    MUON_REQUIRE(descs_dev && coeffs, "small_step: null table");
+    MUON_REQUIRE(nmat > 0 && steps >= 0, "small_step: nmat=%d steps=%d", nmat, steps);
+    MUON_REQUIRE(small_class == 32 || small_class == 64 || small_class == 128, "small_step: class %d", small_class);
+    MUON_REQUIRE(max_long_side > 0 && max_long_side <= 65536, "small_step: long side %d", max_long_side);
+    const size_t bytes = small_lds_bytes(small_class, (max_long_side + 63) & ~63);
+    MUON_REQUIRE(bytes <= SMALL_LDS_MAX, "small_step: a long side of %d does not fit", max_long_side);
+    const int rc = muon_amd_init();
+    if (rc != MUON_AMD_OK) return rc;
+    const auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(nmat), dim3(SMALL_THREADS), bytes, static_cast<hipStream_t>(stream), descs_dev, steps,
+                           coeffs[0], coeffs[1], coeffs[2], one_minus_beta, beta, nesterov, mutate_grad, eps, -lr, wd_factor,
+                           scalars_dev);
+    };
+    const bool round = (flags & MUON_AMD_ROUND_REFERENCE) != 0;
+    if (small_class == 32) round ? go(ns_small_kernel<32, true>) : go(ns_small_kernel<32, false>);
+    else if (small_class == 64) round ? go(ns_small_kernel<64, true>) : go(ns_small_kernel<64, false>);
+    else round ? go(ns_small_kernel<128, true>) : go(ns_small_kernel<128, false>);
+    return check_launch("small_step");
+}
+
+}  // extern "C"

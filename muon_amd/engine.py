@@ -81,6 +81,7 @@ class _ChunkRuntime:
         self.staging = _Staging(device)
         lib = _lib.load()
         self.chunk = chunk
+        self.matrices = [lay.index for lay in chunk.layouts]
         self.device = device
         gemm = chunk.gemm_descs(base)
         phases = {"gram": (_plan.PH_SYRK, _plan.PH_SYRK_ODD), "gram_rowsum": (_plan.PH_SYRK,), "poly": (_plan.PH_POLY,),
@@ -276,6 +277,42 @@ class _ChunkRuntime:
             PROFILE.extend((label, work, *pair) for (label, work), pair in zip(launches, pairs))
 
 
+class _SmallRuntime:
+    """Matrices whose whole step is one workgroup each: one launch, no workspace.  `index`: their positions
+    in the engine's list."""
+
+    def __init__(self, small_class, index, shapes, steps, reference_rounding, device):
+        self.index, self.device, self.small_class, self.steps = index, device, small_class, steps
+        self.shapes = [shapes[i] for i in index]
+        self.longest = max(max(sh) for sh in self.shapes)
+        self.flags = _lib.ROUND_REFERENCE if reference_rounding else _lib.ROUND_FUSED
+        self.template = np.zeros(len(index), dtype=_lib.MAT_DESC)
+        self.template["rows"], self.template["cols"] = np.array(self.shapes, dtype=np.int32).T
+        self.coeffs = np.array(_plan.NS_COEFFS, dtype=np.float32)
+        self.flops = steps * sum(m * (m + 1) * n + m * m * (m + 1) + 2 * m * m * n
+                                 for m, n in (sorted(sh) for sh in self.shapes))
+        self.mat_dev = torch.empty(self.template.nbytes, dtype=torch.uint8, device=device)
+        self.staging = _Staging(device)
+        self.mat_key = None
+
+    def bind(self, grads, momenta, params, outs, scales, src_dtypes):
+        """(Re)upload the matrix descriptors if any tensor address changed since the last call."""
+        key = (tuple(grads), tuple(momenta), tuple(params), tuple(outs), tuple(scales), tuple(src_dtypes))
+        if key == self.mat_key:
+            return
+        d = self.template.copy()
+        d["grad"], d["momentum"], d["param"], d["out"], d["scale"], d["src_dtype"] = grads, momenta, params, outs, scales, src_dtypes
+        _lib.check(_lib.load().muon_amd_validate_small(_lib.host_ptr(d), len(d), self.small_class, self.longest), "validate_small")
+        self.staging.upload(d, self.mat_dev)
+        self.mat_key = key
+
+    def run(self, one_minus_beta, beta, nesterov, mutate_grad, eps, lr, wd_factor, scalars_ptr=0):
+        _launch("small_step", self.flops, lambda: _lib.check(_lib.load().muon_amd_small_step(
+            self.mat_dev.data_ptr(), len(self.index), self.small_class, self.longest, self.steps, self.coeffs.ctypes.data,
+            self.flags, one_minus_beta, beta, int(nesterov), int(mutate_grad), eps, lr, wd_factor, scalars_ptr or None,
+            _stream_ptr(self.device)), "small_step"))
+
+
 class MuonGroupEngine:
     """Runs the Muon update of a fixed list of matrix shapes on one device.
 
@@ -289,19 +326,22 @@ class MuonGroupEngine:
     N_SCALARS = 4          # {1 - beta, beta, lr, 1 - lr * weight_decay}
 
     def __init__(self, shapes, device, steps: int = 5, reference_rounding: bool = True,
-                 workspace_cap: int | None = None, variant: str = "ns5", allow_lanes: bool = True):
+                 workspace_cap: int | None = None, variant: str = "ns5", allow_lanes: bool = True, allow_small: bool = True):
         self.device = torch.device(device)
         with torch.cuda.device(self.device):
             _lib.check(_lib.load().muon_amd_init(), "init")
         self.shapes = [(int(r), int(c)) for r, c in shapes]
         cap = DEFAULT_WORKSPACE_CAP if workspace_cap is None else int(workspace_cap)
-        # Lanes: disjoint sets of matrices with a workspace and (beyond the first, which runs on the
+        # Nothing but small matrices: no chunks.  Else
+        # lanes: disjoint sets of matrices with a workspace and (beyond the first, which runs on the
         # caller's stream) a stream each; the chunks of a lane share its workspace and run back to back.
-        lanes = _plan.plan_lanes(self.shapes, steps, reference_rounding, cap, variant, allow_lanes)
+        small = _plan.small_groups(self.shapes, variant) if allow_small else None
+        self.small = [_SmallRuntime(c, idx, self.shapes, steps, reference_rounding, self.device) for c, idx in small or ()]
+        lanes = [] if small else _plan.plan_lanes(self.shapes, steps, reference_rounding, cap, variant, allow_lanes)
         self.chunks = [c for lane in lanes for c in lane]
         self.workspaces = [torch.empty(max(c.workspace_bytes for c in lane), dtype=torch.uint8, device=self.device)
                            for lane in lanes]
-        self.workspace = self.workspaces[0]
+        self.workspace = self.workspaces[0] if lanes else None
         assert all(ws.data_ptr() % 256 == 0 for ws in self.workspaces)
         self.lane_runtimes = [[_ChunkRuntime(c, ws.data_ptr(), self.device) for c in lane]
                               for lane, ws in zip(lanes, self.workspaces)]
@@ -310,7 +350,7 @@ class MuonGroupEngine:
         self._hyper = None
         # matrices whose momentum stage may run ahead of the step: those of the first chunk (the
         # later chunks reuse its workspace while the step runs); matrix index -> position in the chunk
-        self._early_pos = {lay.index: k for k, lay in enumerate(self.chunks[0].layouts)}
+        self._early_pos = {lay.index: k for k, lay in enumerate(self.chunks[0].layouts)} if lanes else {}
         self._early_stream = None
         self._early_events = {}
         self._early_done = {}         # position -> (gradient address, caller's token) the stage consumed
@@ -334,8 +374,7 @@ class MuonGroupEngine:
             self._skip = frozenset(done)
         else:
             self._skip = frozenset()
-        for rt in self.runtimes:
-            idx = [lay.index for lay in rt.chunk.layouts]
+        for rt, idx in [(rt, rt.index) for rt in self.small] + [(rt, rt.matrices) for rt in self.runtimes]:
             rt.bind([grads[i] for i in idx], [momenta[i] for i in idx], [params[i] for i in idx],
                     [outs[i] for i in idx], [scales[i] for i in idx], [src_dtypes[i] for i in idx])
         # 1 - beta and 1 - lr * weight_decay are python doubles, as in muon.py:9 and muon.py:98
@@ -358,9 +397,13 @@ class MuonGroupEngine:
         or (join=False) when the caller calls `join`, having enqueued work that does not depend on
         these matrices in between (the Adam launch of the same step)."""
         h = self._hyper
-        main = torch.cuda.current_stream(self.device)
-        for side in self.lane_streams[1:]:
-            side.wait_stream(main)
+        for rt in self.small:
+            rt.run(h["one_minus_beta"], h["beta"], h["nesterov"], h["mutate_grad"], h["eps"], h["lr"], h["wd_factor"],
+                   scalars_ptr=scalars_ptr)
+        if len(self.lane_streams) > 1:
+            main = torch.cuda.current_stream(self.device)
+            for side in self.lane_streams[1:]:
+                side.wait_stream(main)
         for li, runtimes in enumerate(self.lane_runtimes):
             with (torch.cuda.stream(self.lane_streams[li]) if li else contextlib.nullcontext()):
                 for n, rt in enumerate(runtimes):
@@ -372,9 +415,10 @@ class MuonGroupEngine:
 
     def join(self):
         """The current stream waits for the lanes that run on streams of their own."""
-        main = torch.cuda.current_stream(self.device)
-        for side in self.lane_streams[1:]:
-            main.wait_stream(side)
+        if len(self.lane_streams) > 1:
+            main = torch.cuda.current_stream(self.device)
+            for side in self.lane_streams[1:]:
+                main.wait_stream(side)
 
     def early_stream(self):
         """The side stream the early stages run on (default priority; created on first use)."""

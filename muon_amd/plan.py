@@ -627,6 +627,26 @@ def _shape_order_key(shapes, i):
     return (-tile_class_for(min(shapes[i])), -min(shapes[i]), -max(shapes[i]), -shapes[i][0], i)
 
 
+SMALL = os.environ.get("MUON_AMD_SMALL", "1") != "0"      # measurement knob: small matrices in one workgroup each
+
+
+def small_groups(shapes, variant: str = "ns5"):
+    """-> [(class, positions in `shapes`)] when every matrix of the group fits one workgroup (its whole step
+    is then one launch, see small.hip), else None: beside larger matrices the small ones ride in the
+    grouped launches, where a launch of their own would only add its time (bits are the same).  One
+    launch covers all of them in the largest class any of them needs if they all fit it."""
+    if not SMALL or variant != "ns5" or not shapes:
+        return None
+    lib = _lib.load()
+    own = [lib.muon_amd_small_class(r, c) for r, c in shapes]
+    if not all(own):
+        return None
+    top, longest = max(own), max(max(sh) for sh in shapes)
+    if lib.muon_amd_small_class(top, max(longest, top)) == top:
+        return [(top, list(range(len(shapes))))]
+    return [(c, [i for i, k in enumerate(own) if k == c]) for c in sorted(set(own))]
+
+
 LANES = os.environ.get("MUON_AMD_LANES", "auto")        # "auto", or a number of lanes to force ("1" switches them off)
 LANE_UPDATE_TILES = (600, 2600)
 

@@ -16,6 +16,7 @@ SHAPES = [(1, 1, 1), (1, 64, 64), (1, 65, 129), (1, 63, 577), (1, 128, 320), (3,
 def test_tile_class_of_a_launch_does_not_change_the_bits(shape, rounding, monkeypatch):
     import muon_amd
     from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
     torch.manual_seed(sum(shape))
     G = torch.randn(*shape, device="cuda")
     outs, classes = [], []
@@ -35,6 +36,7 @@ def test_tile_class_of_a_launch_does_not_change_the_bits(shape, rounding, monkey
 def test_fused_parameter_step_in_small_tiles_gives_the_bits_of_large_ones(monkeypatch):
     import muon_amd
     from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
     shapes = [(70, 200), (200, 70), (64, 64), (33, 500), (300, 257)]
     results = []
     for forced in ("0,0,0", "2,2,2"):
