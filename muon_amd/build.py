@@ -5,7 +5,8 @@
 After the library is built, the GEMM kernels are compiled once more to assembly and checked
 (`check_fragment_waits`): their main loop requests its LDS fragments through inline assembly and
 waits for them by hand, which is only correct while the compiler does not touch a requested
-register before the wait that covers it.
+register before the wait that covers it.  The same listing is checked for vector instructions that
+overwrite the data of a wide store right behind it (`check_store_data`).
 """
 from __future__ import annotations
 
@@ -102,6 +103,31 @@ def check_fragment_waits(asm_text: str) -> int:
     return nreads
 
 
+def check_store_data(asm_text: str) -> int:
+    """No vector instruction may overwrite a data register of a buffer, global or flat store of more than 8 bytes
+    within two wait states of it: the store still reads that register for its last lanes.  The compiler
+    leaves out those wait states after a buffer store with a scalar offset.  Raises if the listing
+    holds such a pair; returns the number of
+    stores looked at."""
+    code = [t for t in (l.split(";")[0].strip() for l in asm_text.split("\n")) if t and not t.startswith(".") and not t.endswith(":")]
+    nstores = 0
+    for i, t in enumerate(code):
+        m = re.match(r"(buffer|global|flat)_store_dwordx[34]\s+(.*)", t)
+        if not m:
+            continue
+        nstores += 1
+        data = _vregs(m.group(2).split(",")[0 if m.group(1) == "buffer" else 1])
+        states = 0
+        for u in code[i + 1:i + 3]:
+            if states >= 2 or u.startswith("s_endpgm"):
+                break
+            op, _, args = u.partition(" ")
+            if op.startswith("v_") and _vregs(args.split(",")[0]) & data:
+                raise RuntimeError(f"ns_gemm.hip: '{u}' overwrites the data of '{t}' while it is read")
+            states += int(args) + 1 if op == "s_nop" else 1
+    return nstores
+
+
 def build(verbose: bool = True, check: bool = True) -> str:
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     tmp = OUT + ".tmp"
@@ -121,7 +147,9 @@ def build(verbose: bool = True, check: bool = True) -> str:
             if proc.returncode != 0:
                 sys.stderr.write(proc.stdout + proc.stderr)
                 raise RuntimeError("hipcc failed writing the assembly listing of ns_gemm.hip")
-            n = check_fragment_waits(open(listing).read())
+            text = open(listing).read()
+            n = check_fragment_waits(text)
+            check_store_data(text)
             if verbose:
                 print(f"ns_gemm.hip: {n} hand-waited fragment reads followed through the listing, none touched early", flush=True)
     os.replace(tmp, OUT)

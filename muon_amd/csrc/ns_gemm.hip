@@ -56,10 +56,15 @@ __device__ __forceinline__ u32x2 gload8(const uint16_t* p) {
 // the next launch reads long after this XCD's L2 has turned over; keeping them out of the way of
 // the operand panels measured +0.5 % on the Llama step (and a loss for GPT-2-size matrices, whose
 // outputs the next launch does find in L2, so the small class stores normally).
+// The two wait states after it belong to it: a store of more than 8 bytes reads its data registers over several
+// cycles, and a vector instruction that overwrites one of them right behind it reached the last lanes
+// of the store (first register, lanes 12-15 of each 16).  The compiler keeps its distance for stores
+// without a scalar offset only, so the store is written out here.
 template <bool STREAM>
 __device__ __forceinline__ void bstore16(const uint16_t* base, uint32_t voff, uint32_t soff, u32x4 v) {
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, 0xffffffff, 0x00020000);
-    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, static_cast<int>(voff), static_cast<int>(soff), STREAM ? 2 : 0);
+    if constexpr (STREAM) asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1" :: "v"(v), "v"(voff), "s"(rsrc), "s"(soff));
+    else asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen\n\ts_nop 1" :: "v"(v), "v"(voff), "s"(rsrc), "s"(soff));
 }
 
 constexpr int BK = 64;   // k extent of one ring stage (128 bytes per LDS row)

@@ -631,3 +631,16 @@ def test_lanes_split_groups_like_gpt2_small_and_nothing_else():
         assert len(plan.plan_lanes(shapes, 5, True, 16 << 30)) == 1
     assert len(plan.plan_lanes(gpt2, 5, True, 16 << 30, allow_lanes=False)) == 1
     assert len(plan.plan_lanes(gpt2, 5, True, 64 << 20)) == 1                     # several chunks: one lane
+
+
+def test_build_refuses_store_data_overwritten_behind_the_store():
+    """The listing of a kernel in which a vector instruction follows a 16-byte store with a scalar offset and takes one
+    of its data registers (such a kernel stored wrong values for the last lanes)."""
+    from muon_amd.build import check_store_data
+    store = "\tbuffer_store_dwordx4 v[170:173], v164, s[28:31], s26 offen nt\n"
+    bad = "\tv_add_u32_e32 v170, v174, v199\n"
+    for text in (store + bad, store + "\ts_nop 0\n" + bad, "\tglobal_store_dwordx4 v[2:3], v[170:173], off\n" + bad):
+        with pytest.raises(RuntimeError, match="overwrites the data"):
+            check_store_data(text)
+    for text in (store + "\ts_nop 1\n" + bad, store + "\tv_add_u32_e32 v174, v170, v199\n", store + "\ts_nop 0\n\ts_mov_b32 s1, s2\n" + bad):
+        assert check_store_data(text) == 1
