@@ -3,9 +3,12 @@
 //
 // A matrix whose short side is at most 128 and whose iterate fits the 160 KB of LDS of a CU beside two
 // Gram matrices needs nothing from other CUs between two products, so the 17 launches of the general
-// path (4 us each on the GPU, 3.3 us each on the host, whatever the size) become one.  What bounds it
-// is latency: the loads of gradient and momentum, then chains of LDS reads and MFMAs.
-// muon_update of a 64 x 64 x 3 x 3 filter: 106 us in separate launches.
+// path (4 us each on the GPU, 3.3 us each on the host, whatever the size) become one.  One CU is what a matrix
+// gets, and what bounds it there is the vector ALU and LDS: of the 39 us of a 64 x 576 matrix the loads take 8, the
+// normalise pass 2, each of the five iterations 5 (X X^T 1.9, the update 2.7) and the parameter step 2.5.
+// muon_update of a 64 x 64 x 3 x 3 filter: 106 us in separate launches; 62 us with 8 waves, the index of
+// every element from a division of its own, scaled divisions, all four 32 x 32 tiles of X X^T and 8-byte accesses
+// to tiles; 48 us with 16 waves and without those.
 //
 // Every rounding and every order of summation is the general path's (elementwise.hip, ns_gemm.hip): the
 // sum of squares goes by blocks of 8192 elements and 256 threads, the products accumulate k-step after
@@ -21,7 +24,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int SMALL_THREADS = 512, SMALL_WAVES = SMALL_THREADS / 64;
+constexpr int SMALL_THREADS = 1024, SMALL_WAVES = SMALL_THREADS / 64;
 constexpr int SUM_BLOCK = 8192;                     // elements per partial sum (EW_BLOCK_ELEMS) ...
 constexpr int SUM_THREADS = 256, SUM_ITERS = 8;     // ... and how its threads share them (4 in a row each)
 constexpr int SMALL_LDS_MAX = 163840;
@@ -81,37 +84,116 @@ __device__ __forceinline__ f32x16 zero16() {
     for (int i = 0; i < 16; ++i) z[i] = 0.f;
     return z;
 }
-// A 32 x 32 tile of packed bf16 pairs (lane = row l % 32, pair 2q + i = columns 8q + 4 (l / 32) + 2i) to LDS rows.
+// A 32 x 32 tile of packed bf16 pairs as the MFMAs leave it (lane = row l % 32, pair 2q + i = columns
+// 8q + 4 (l / 32) + 2i) to LDS rows and back.  The halves of two neighbouring chunks of 8 columns are exchanged between
+// lanes l and l + 32, so that a lane moves 8 columns in a row: 16-byte accesses hit all banks, the 8-byte
+// ones of the layout itself meet rows 16 apart in the same bank.
 __device__ __forceinline__ void tile_store(char* base, int pitch, int row0, int col0, int lane, const uint32_t (&po)[8]) {
-    char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 4) * 2;
+    char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 8) * 2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x2*>(p + q * 16) = u32x2{po[2 * q], po[2 * q + 1]};
+    for (int q = 0; q < 4; q += 2) {
+        const auto x = __builtin_amdgcn_permlane32_swap(po[2 * q], po[2 * q + 2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(po[2 * q + 1], po[2 * q + 3], false, false);
+        *reinterpret_cast<u32x4*>(p + q * 16) = u32x4{x[0], y[0], x[1], y[1]};
+    }
 }
-// o = alpha * acc + beta * D as the epilogue of the GEMM kernel rounds it; D from LDS in the same layout.
+__device__ __forceinline__ void tile_load(uint32_t (&po)[8], const char* base, int pitch, int row0, int col0, int lane) {
+    const char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 8) * 2;
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(p + q * 16);
+        const auto x = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+        po[2 * q] = x[0];
+        po[2 * q + 1] = y[0];
+        po[2 * q + 2] = x[1];
+        po[2 * q + 3] = y[1];
+    }
+}
+// The same tile as the columns of its mirror image.
+__device__ __forceinline__ void tile_store_mirrored(char* base, int pitch, int row0, int col0, int lane, const uint32_t (&po)[8]) {
+    char* const p = base + (col0 + (lane >> 5) * 4) * pitch + (row0 + (lane & 31)) * 2;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        char* const c = p + (8 * (k >> 1) + 2 * (k & 1)) * pitch;
+        *reinterpret_cast<uint16_t*>(c) = static_cast<uint16_t>(po[k]);
+        *reinterpret_cast<uint16_t*>(c + pitch) = static_cast<uint16_t>(po[k] >> 16);
+    }
+}
+// o = alpha * acc + beta * D as the epilogue of the GEMM kernel rounds it; po holds D on entry and o on return.
 template <bool ROUND>
-__device__ __forceinline__ void tile_add(uint32_t (&po)[8], const f32x16& acc, float alpha, float beta, const char* base,
-                                         int pitch, int row0, int col0, int lane) {
-    const char* const p = base + (row0 + (lane & 31)) * pitch + (col0 + (lane >> 5) * 4) * 2;
+__device__ __forceinline__ void tile_add(uint32_t (&po)[8], const f32x16& acc, float alpha, float beta) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const u32x2 dv = *reinterpret_cast<const u32x2*>(p + q * 16);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int k = 2 * q + i;
-            const uint32_t dk = i ? dv.y : dv.x;
-            if constexpr (ROUND) {
-                const uint32_t t1 = pack2bf(alpha * acc[2 * k], alpha * acc[2 * k + 1]);
-                const uint32_t t2 = pack2bf(beta * bf_lo(dk), beta * bf_hi(dk));
-                po[k] = pack2bf(bf_lo(t1) + bf_lo(t2), bf_hi(t1) + bf_hi(t2));
-            } else {
-                po[k] = pack2bf(fmaf(alpha, acc[2 * k], beta * bf_lo(dk)), fmaf(alpha, acc[2 * k + 1], beta * bf_hi(dk)));
-            }
+    for (int k = 0; k < 8; ++k) {
+        const uint32_t dk = po[k];
+        if constexpr (ROUND) {
+            // every term rounded to bf16, their sum rounded again
+            po[k] = pack2bf(bf_pair_sum(pack2bf(alpha * acc[2 * k], beta * bf_lo(dk))),
+                            bf_pair_sum(pack2bf(alpha * acc[2 * k + 1], beta * bf_hi(dk))));
+        } else {
+            po[k] = pack2bf(fmaf(alpha, acc[2 * k], beta * bf_lo(dk)), fmaf(alpha, acc[2 * k + 1], beta * bf_hi(dk)));
         }
     }
 }
 
+// Row and column of an element index that grows by a fixed stride: two divisions, then additions.
+struct Walk {
+    int r, c, dr, dc, cols;
+    __device__ __forceinline__ Walk(int e, int stride, int cols_) : cols(cols_) {
+        r = e / cols;
+        c = e - r * cols;
+        dr = stride / cols;
+        dc = stride - dr * cols;
+    }
+    __device__ __forceinline__ void next() {
+        r += dr;
+        c += dc;
+        if (c >= cols) {
+            c -= cols;
+            ++r;
+        }
+    }
+};
+
+// One tile of X X^T.  The reads of the next U k-steps are in flight under the MFMAs of the current ones; the
+// rows of a diagonal tile are read once for both operands.  `nks` is a multiple of 4.
+template <bool DIAG>
+__device__ __forceinline__ void gram_tile(f32x16& acc, const char* X, int px, int i0, int j0, int nks, int lane) {
+    constexpr int U = 4;
+    bf16x8 fp[2][U], fq[2][U];
+    const auto fetch = [&](int buf, int ks) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            fp[buf][u] = row_frag(X, px, i0, ks + u, lane);
+            if constexpr (!DIAG) fq[buf][u] = row_frag(X, px, j0, ks + u, lane);
+        }
+    };
+    const auto multiply = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(DIAG ? fp[buf][u] : fq[buf][u], fp[buf][u], acc, 0, 0, 0);
+    };
+    fetch(0, 0);
+    int ks = 0;
+    for (; ks + 3 * U <= nks; ks += 2 * U) {
+        fetch(1, ks + U);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        fetch(0, ks + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+    }
+    if (ks + 2 * U <= nks) {
+        fetch(1, ks + U);
+        multiply(0);
+        multiply(1);
+    } else {
+        multiply(0);
+    }
+}
+
 // X from gradient and momentum (muon.py:9-10, 277-279), and the partial sums of squares: block b of 8192
-// elements by threads 256 (b % 2) .. + 255.
+// elements by threads 256 (b % 4) .. + 255.
 template <typename T>
 __device__ __forceinline__ void small_load(const MuonMatDesc& d, char* X, int pitch, bool wide, float w, float beta,
                                            int nesterov, int mutate_grad, float* sums, int tid) {
@@ -121,62 +203,82 @@ __device__ __forceinline__ void small_load(const MuonMatDesc& d, char* X, int pi
     T* const mom = static_cast<T*>(d.momentum);
     const bool has_m = mom != nullptr, write_g = has_m && nesterov && mutate_grad;
     const bool aligned = small_aligned(g, S::kAlign) && small_aligned(mom, S::kAlign);
+    const bool in_row = (cols & 3) == 0;
     const int t = tid & (SUM_THREADS - 1);
     for (int b = tid / SUM_THREADS; b * SUM_BLOCK < numel; b += SMALL_THREADS / SUM_THREADS) {
-        f32x4s gv[SUM_ITERS], mv[SUM_ITERS];
-#pragma unroll
-        for (int it = 0; it < SUM_ITERS; ++it) {
-            const int e = b * SUM_BLOCK + (it * SUM_THREADS + t) * 4;
-            gv[it] = mv[it] = f32x4s{0.f, 0.f, 0.f, 0.f};
-            if (aligned && e + 4 <= numel) {
-                gv[it] = S::ld4(g + e);
-                if (has_m) mv[it] = S::ld4(mom + e);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (e + k < numel) {
-                        gv[it][k] = S::ld(g + e + k);
-                        if (has_m) mv[it][k] = S::ld(mom + e + k);
-                    }
-            }
-        }
         float ss = 0.f;
+        Walk at(b * SUM_BLOCK + t * 4, SUM_THREADS * 4, cols);
+#pragma unroll 1
+        for (int first = b * SUM_BLOCK + t * 4; first < (b + 1) * SUM_BLOCK; first += SUM_BLOCK / 2) {
+            f32x4s gv[SUM_ITERS / 2], mv[SUM_ITERS / 2];
 #pragma unroll
-        for (int it = 0; it < SUM_ITERS; ++it) {
-            const int e = b * SUM_BLOCK + (it * SUM_THREADS + t) * 4;
-            if (e >= numel) continue;
-            f32x4s gg = gv[it], mm = mv[it];
-            int r = e / cols, c = e - r * cols;
-            const bool whole = e + 4 <= numel;
+            for (int it = 0; it < SUM_ITERS / 2; ++it) {
+                const int e = first + it * SUM_THREADS * 4;
+                gv[it] = mv[it] = f32x4s{0.f, 0.f, 0.f, 0.f};
+                if (aligned && e + 4 <= numel) {
+                    gv[it] = S::ld4(g + e);
+                    if (has_m) mv[it] = S::ld4(mom + e);
+                } else {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float u = gg[k];
-                if (has_m) {
-                    mm[k] = S::rnd(lerp_torch(mm[k], gg[k], w));            // momentum.lerp_(grad, 1 - beta)
-                    u = mm[k];
-                    if (nesterov) u = gg[k] = S::rnd(lerp_torch(gg[k], mm[k], beta));   // grad.lerp_(momentum, beta)
-                }
-                const uint16_t ub = f2bf(u);
-                if (whole || e + k < numel) {
-                    const float uf = bf2f(ub);
-                    ss = fmaf(uf, uf, ss);
-                    *reinterpret_cast<uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2) = ub;
-                }
-                if (++c == cols) {
-                    c = 0;
-                    ++r;
+                    for (int k = 0; k < 4; ++k)
+                        if (e + k < numel) {
+                            gv[it][k] = S::ld(g + e + k);
+                            if (has_m) mv[it][k] = S::ld(mom + e + k);
+                        }
                 }
             }
-            if (aligned && whole) {
-                if (has_m) S::st4(mom + e, mm);
-                if (write_g) S::st4(g + e, gg);
-            } else {
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (e + k < numel) {
-                        if (has_m) S::st(mom + e + k, mm[k]);
-                        if (write_g) S::st(g + e + k, gg[k]);
+            for (int it = 0; it < SUM_ITERS / 2; ++it, at.next()) {
+                const int e = first + it * SUM_THREADS * 4;
+                if (e >= numel) continue;
+                f32x4s gg = gv[it], mm = mv[it];
+                const bool whole = e + 4 <= numel;
+                uint32_t ub[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float u = gg[k];
+                    if (has_m) {
+                        mm[k] = S::rnd(lerp_torch(mm[k], gg[k], w));            // momentum.lerp_(grad, 1 - beta)
+                        u = mm[k];
+                        if (nesterov) u = gg[k] = S::rnd(lerp_torch(gg[k], mm[k], beta));   // grad.lerp_(momentum, beta)
                     }
+                    ub[k] = f2bf(u);
+                    if (whole || e + k < numel) {
+                        const float uf = bf2f(static_cast<uint16_t>(ub[k]));
+                        ss = fmaf(uf, uf, ss);
+                    }
+                }
+                if (in_row) {          // (then every group of four is whole, and lies in one row)
+                    if (wide) {
+                        *reinterpret_cast<u32x2*>(X + at.r * pitch + at.c * 2) = u32x2{ub[0] | (ub[1] << 16), ub[2] | (ub[3] << 16)};
+                    } else {
+                        char* const p = X + at.c * pitch + at.r * 2;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) *reinterpret_cast<uint16_t*>(p + k * pitch) = static_cast<uint16_t>(ub[k]);
+                    }
+                } else {
+                    int r = at.r, c = at.c;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (whole || e + k < numel)
+                            *reinterpret_cast<uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2) = static_cast<uint16_t>(ub[k]);
+                        if (++c == cols) {
+                            c = 0;
+                            ++r;
+                        }
+                    }
+                }
+                if (aligned && whole) {
+                    if (has_m) S::st4(mom + e, mm);
+                    if (write_g) S::st4(g + e, gg);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (e + k < numel) {
+                            if (has_m) S::st(mom + e + k, mm[k]);
+                            if (write_g) S::st(g + e + k, gg[k]);
+                        }
+                }
             }
         }
         ss = wave_sum(ss);
@@ -193,7 +295,9 @@ __device__ __forceinline__ void small_apply(const MuonMatDesc& d, const char* X,
     T* const p = static_cast<T*>(d.param);
     uint16_t* const out = d.out;
     const bool aligned = small_aligned(p, S::kAlign) && small_aligned(out, 8);
-    constexpr int UN = 4;
+    const bool in_row = (cols & 3) == 0;
+    constexpr int UN = 2;
+    Walk at(tid * 4, SMALL_THREADS * 4, cols);
     for (int e0 = tid * 4; e0 < numel; e0 += SMALL_THREADS * 4 * UN) {
         f32x4s pv[UN];
 #pragma unroll
@@ -210,23 +314,31 @@ __device__ __forceinline__ void small_apply(const MuonMatDesc& d, const char* X,
             }
         }
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
+        for (int u = 0; u < UN; ++u, at.next()) {
             const int e = e0 + u * SMALL_THREADS * 4;
             if (e >= numel) continue;
-            int r = e / cols, c = e - r * cols;
             float us[4];
+            if (in_row && wide) {
+                const u32x2 o = *reinterpret_cast<const u32x2*>(X + at.r * pitch + at.c * 2);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) us[k] = (k & 1) ? bf_hi(o[k / 2]) : bf_lo(o[k / 2]);
+            } else {
+                int r = at.r, c = at.c;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    us[k] = 0.f;
+                    if (e + k < numel)
+                        us[k] = bf2f(*reinterpret_cast<const uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2));
+                    if (++c == cols) {
+                        c = 0;
+                        ++r;
+                    }
+                }
+            }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                us[k] = 0.f;
-                if (e + k < numel) {
-                    const uint16_t o = *reinterpret_cast<const uint16_t*>(wide ? X + r * pitch + c * 2 : X + c * pitch + r * 2);
-                    us[k] = round_bf(bf2f(o) * d.scale);
-                }
+                us[k] = round_bf(us[k] * d.scale);
                 pv[u][k] = S::rnd(fmaf(neg_lr, us[k], S::rnd(pv[u][k] * wd_factor)));
-                if (++c == cols) {
-                    c = 0;
-                    ++r;
-                }
             }
             if (aligned && e + 4 <= numel) {
                 if (p) S::st4(p + e, pv[u]);
@@ -251,9 +363,12 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
     const MuonMatDesc* __restrict__ descs, int steps, float ca, float cb, float cc, float w, float beta, int nesterov,
     int mutate_grad, float eps, float neg_lr, float wd_factor, const float* __restrict__ sc) {
     constexpr int MT = MP / 32, TILES = MT * MT, TPW = (TILES + SMALL_WAVES - 1) / SMALL_WAVES;
+    constexpr int SYM_TILES = MT * (MT + 1) / 2, SPW = (SYM_TILES + SMALL_WAVES - 1) / SMALL_WAVES;
+    constexpr bool KEEP_B = MP <= 64;                // (of the 128 registers a thread can have at 16 waves)
     constexpr int PA = small_pitch(MP);
     extern __shared__ __align__(16) char lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int lane = tid & 63;
     if (sc) {   // {1 - beta, beta, lr, wd_factor} read at run time instead of the arguments
         w = sc[0];
         beta = sc[1];
@@ -283,40 +398,56 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
         const float nrm = sqrtf(wave_sum(lane < nblk ? (q[0] + q[1]) + (q[2] + q[3]) : 0.f));
         den = ROUND ? round_bf(round_bf(nrm) + eps) : nrm + eps;
     }
-    const int chunks = np / 8;                       // of 8 columns
-    for (int i = tid; i < m * chunks; i += SMALL_THREADS) {
-        const int r = i / chunks, c = (i - r * chunks) * 8;
-        u32x4* const p = reinterpret_cast<u32x4*>(X + r * px + c * 2);
-        const u32x4 v = *p;
-        u32x4 o;
+    {
+        const UniformDivisor by(den);
+        const int chunks = np / 8;                   // of 8 columns
+        Walk at(tid, SMALL_THREADS, chunks);
+        for (; at.r < m; at.next()) {
+            u32x4* const p = reinterpret_cast<u32x4*>(X + at.r * px + at.c * 16);
+            const u32x4 v = *p;
+            u32x4 o;                                 // (columns beyond n hold zero and stay zero)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float lo = c + 2 * k < n ? bf_lo(v[k]) / den : 0.f, hi = c + 2 * k + 1 < n ? bf_hi(v[k]) / den : 0.f;
-            o[k] = pack2bf(lo, hi);
+            for (int k = 0; k < 4; ++k) o[k] = pack2bf(by.divide(bf_lo(v[k])), by.divide(bf_hi(v[k])));
+            if (!by.ok) {                            // (an element is at most the norm: only den can be out of range)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) o[k] = pack2bf(bf_lo(v[k]) / den, bf_hi(v[k]) / den);
+            }
+            if (at.c * 8 + 8 > n) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    o[k] &= (at.c * 8 + 2 * k < n ? 0xffffu : 0u) | (at.c * 8 + 2 * k + 1 < n ? 0xffff0000u : 0u);
+            }
+            *p = o;
         }
-        *p = o;
     }
     __syncthreads();
 
     for (int step = 0; step < steps; ++step) {
-        // A = X X^T and, where the reference rounds it, c A
+        asm volatile("" : "+v"(lane));               // LDS addresses are formed where they are used, not kept in registers
+        // A = X X^T and, where the reference rounds it, c A: the tiles on and above the diagonal (X X^T is
+        // symmetric bit for bit), each by one wave.  The reads of the next four k-steps are in flight under
+        // the MFMAs of the current four; the rows of a diagonal tile are read once for both operands.
 #pragma unroll
-        for (int s = 0; s < TPW; ++s) {
+        for (int s = 0; s < SPW; ++s) {
             const int t = wave + s * SMALL_WAVES;
-            if (t >= TILES) continue;
-            const int i0 = t / MT * 32, j0 = t % MT * 32;
+            if (t >= SYM_TILES) continue;
+            int ti = 0, tj = t;                      // diagonal tiles first, then the first off-diagonal, ...
+            for (int len = MT; tj >= len; --len) tj -= len, ++ti;
+            const int i0 = tj * 32, j0 = (tj + ti) * 32;
+            const bool diag = ti == 0;
             f32x16 acc = zero16();
-#pragma unroll 4
-            for (int ks = 0; ks < np / 16; ++ks)
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag(X, px, j0, ks, lane), row_frag(X, px, i0, ks, lane), acc, 0, 0, 0);
+            if (diag) gram_tile<true>(acc, X, px, i0, j0, np / 16, lane);
+            else gram_tile<false>(acc, X, px, i0, j0, np / 16, lane);
             uint32_t po[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) po[k] = pack2bf(acc[2 * k], acc[2 * k + 1]);
             tile_store(A, PA, i0, j0, lane, po);
+            if (!diag) tile_store_mirrored(A, PA, i0, j0, lane, po);
             if constexpr (ROUND) {
 #pragma unroll
                 for (int k = 0; k < 8; ++k) po[k] = pack2bf(cc * bf_lo(po[k]), cc * bf_hi(po[k]));
                 tile_store(B, PA, i0, j0, lane, po);
+                if (!diag) tile_store_mirrored(B, PA, i0, j0, lane, po);
             }
         }
         __syncthreads();
@@ -331,7 +462,8 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
 #pragma unroll
             for (int ks = 0; ks < MP / 16; ++ks)
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag(A, PA, j0, ks, lane), row_frag(ROUND ? B : A, PA, i0, ks, lane), acc, 0, 0, 0);
-            tile_add<ROUND>(pb[s], acc, ROUND ? 1.f : cc, cb, A, PA, i0, j0, lane);
+            tile_load(pb[s], A, PA, i0, j0, lane);
+            tile_add<ROUND>(pb[s], acc, ROUND ? 1.f : cc, cb);
         }
         __syncthreads();
 #pragma unroll
@@ -341,24 +473,34 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
             tile_store(B, PA, t / MT * 32, t % MT * 32, lane, pb[s]);
         }
         __syncthreads();
-        // X = a X + B X, a block of 32 columns at a time
+        // X = a X + B X, a block of 32 columns at a time; the rows of B stay in registers where they fit
+        bf16x8 bq[KEEP_B ? MT : 1][KEEP_B ? MP / 16 : 1];
+        if constexpr (KEEP_B) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int ks = 0; ks < MP / 16; ++ks) bq[i][ks] = row_frag(B, PA, i * 32, ks, lane);
+        }
         for (int j0 = wave * 32; j0 < np; j0 += SMALL_WAVES * 32) {
             bf16x8 q[MP / 16];
 #pragma unroll
             for (int ks = 0; ks < MP / 16; ++ks) q[ks] = col_frag(X, px, j0, ks, lane);
-#pragma unroll
-            for (int i0 = 0; i0 < MP; i0 += 32) {
+#pragma unroll KEEP_B ? MT : 1
+            for (int i = 0; i < MT; ++i) {
                 f32x16 acc = zero16();
-#pragma unroll
-                for (int ks = 0; ks < MP / 16; ++ks)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[ks], row_frag(B, PA, i0, ks, lane), acc, 0, 0, 0);
                 uint32_t po[8];
+                tile_load(po, X, px, i * 32, j0, lane);
+#pragma unroll
+                for (int ks = 0; ks < MP / 16; ++ks) {
+                    const bf16x8 b = KEEP_B ? bq[KEEP_B ? i : 0][KEEP_B ? ks : 0] : row_frag(B, PA, i * 32, ks, lane);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[ks], b, acc, 0, 0, 0);
+                }
                 // (with one rounding the alpha of the general path is a run-time 1: beta * D is rounded before
                 // the sum there, and must not be contracted into it here)
                 float alpha = 1.f;
                 if constexpr (!ROUND) asm volatile("" : "+s"(alpha));
-                tile_add<ROUND>(po, acc, alpha, ca, X, px, i0, j0, lane);
-                tile_store(X, px, i0, j0, lane, po);
+                tile_add<ROUND>(po, acc, alpha, ca);
+                tile_store(X, px, i * 32, j0, lane, po);
             }
         }
         __syncthreads();
