@@ -1,0 +1,40 @@
+"""The normalise launch alone (a run without iterations): rows that start at any 2-byte address, tiles and chunks
+cut by the edge of the matrix, both orientations, and norms out of the range of the short division."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _normalised(G):
+    import muon_amd
+    return muon_amd.zeropower_via_newtonschulz5(G, steps=0)
+
+
+@pytest.mark.parametrize("cols", [128, 129, 1100, 1101, 1102, 1104])
+@pytest.mark.parametrize("rows", [1, 127, 300, 1500])
+def test_normalise_divides_as_the_specification(rows, cols, monkeypatch):
+    from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
+    torch.manual_seed(rows + cols)
+    G = torch.randn(rows, cols, device="cuda")
+    X = G.bfloat16()
+    norm = X.double().norm().to(torch.bfloat16)         # the kernel's fp32 sum may land on a neighbouring bf16 value
+    step = torch.tensor([0, 1, -1], dtype=torch.int16, device="cuda")
+    candidates = [(norm.view(torch.int16) + s).view(torch.bfloat16) + 1e-7 for s in step]
+    got = _normalised(G)
+    assert any(torch.equal(got, X / c) for c in candidates)
+
+
+@pytest.mark.parametrize("shape", [(200, 330), (330, 200)])
+def test_normalise_beyond_the_range_of_the_short_division(shape, monkeypatch):
+    from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
+    torch.manual_seed(1)
+    G = torch.randn(*shape, device="cuda")
+    tiny = (G * 1e-30).bfloat16()                       # the squares underflow: the denominator is epsilon
+    assert torch.equal(_normalised(tiny), tiny / torch.tensor(1e-7, device="cuda").bfloat16())
+    assert (_normalised(G * 1e30) == 0).all()           # the squares overflow: every element over infinity
+    assert (_normalised(torch.zeros_like(G)) == 0).all()
+    G[3, 5] = float("nan")
+    assert _normalised(G).isnan().all()
