@@ -5,6 +5,8 @@
 // finds its matrix by a binary search in a small prefix table and then streams a fixed-size
 // contiguous range of it with 16-byte accesses, so a step costs a handful of launches however
 // many parameters the model has.
+#include <type_traits>
+
 #include "common.h"
 
 namespace muon_amd {
@@ -25,35 +27,40 @@ constexpr int NT_THREADS = 512;
 // compiler).  MUON_EW_NT adds the non-temporal hint to these streaming accesses.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2e __attribute__((ext_vector_type(2)));
+// Tensors start at any element (a slice of a flat buffer, a matrix of a batch with an odd element count), and the
+// target's vector accesses take any address.  Adam over 50257 x 768 one element off 16 bytes: 288 us element by
+// element, 174 (fp32) and 245 -> 111 us (bf16) with these; 165 and 101 us aligned.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2e_any __attribute__((ext_vector_type(2), aligned(2)));
 #ifndef MUON_EW_NT
 #define MUON_EW_NT 1   // measured +3% on the Llama-3-8B tensors
 #endif
 __device__ __forceinline__ f32x4 gld4(const float* p) {
 #if MUON_EW_NT
-    return __builtin_nontemporal_load((const __attribute__((address_space(1))) f32x4*)(p));
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) f32x4_any*)(p));
 #else
-    return *(const __attribute__((address_space(1))) f32x4*)(p);
+    return *(const __attribute__((address_space(1))) f32x4_any*)(p);
 #endif
 }
 __device__ __forceinline__ void gst4(float* p, f32x4 v) {
 #if MUON_EW_NT
-    __builtin_nontemporal_store(v, (__attribute__((address_space(1))) f32x4*)(p));
+    __builtin_nontemporal_store(v, (__attribute__((address_space(1))) f32x4_any*)(p));
 #else
-    *(__attribute__((address_space(1))) f32x4*)(p) = v;
+    *(__attribute__((address_space(1))) f32x4_any*)(p) = v;
 #endif
 }
 __device__ __forceinline__ u32x2e gld2u(const uint16_t* p) {
 #if MUON_EW_NT
-    return __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x2e*)(p));
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x2e_any*)(p));
 #else
-    return *(const __attribute__((address_space(1))) u32x2e*)(p);
+    return *(const __attribute__((address_space(1))) u32x2e_any*)(p);
 #endif
 }
 __device__ __forceinline__ void gst2u(uint16_t* p, u32x2e v) {
 #if MUON_EW_NT
-    __builtin_nontemporal_store(v, (__attribute__((address_space(1))) u32x2e*)(p));
+    __builtin_nontemporal_store(v, (__attribute__((address_space(1))) u32x2e_any*)(p));
 #else
-    *(__attribute__((address_space(1))) u32x2e*)(p) = v;
+    *(__attribute__((address_space(1))) u32x2e_any*)(p) = v;
 #endif
 }
 
@@ -129,61 +136,73 @@ __device__ __forceinline__ float momentum_block(const MuonMatDesc& d, int64_t bl
     T* __restrict__ mom = static_cast<T*>(d.momentum);
     uint16_t* __restrict__ u = d.u;
     float ss = 0.f;
-    const bool aligned = aligned_to(g, Stored<T>::kAlign) && aligned_to(mom, Stored<T>::kAlign) && aligned_to(u, 8);
-
+    // FULL: every group of four lies in the matrix.  Otherwise those that do are treated alike, and the last one to
+    // three elements of the matrix follow, as the last group of the thread that would hold them.  (The last block of a
+    // matrix element by element was 32 memory latencies in a row: one 1500 x 1100 Newton-Schulz 165.8 -> 161.8 us,
+    // 16 of 777 x 1001, every other one at an odd address, 424 -> 403 us.)
+    const auto pass_over = [&](int64_t base, auto full) {
+        constexpr bool FULL = decltype(full)::value;
+        f32x4 gv[EW_ITERS], mv[EW_ITERS];
+#pragma unroll
+        for (int it = 0; it < EW_ITERS; ++it) {
+            const int64_t e = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
+            gv[it] = mv[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (FULL || e + EW_VEC <= numel) {
+                gv[it] = Stored<T>::ld4(g + e);
+                if (has_m) mv[it] = Stored<T>::ld4(mom + e);
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < EW_ITERS; ++it) {
+            const int64_t e = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
+            if (!FULL && e + EW_VEC > numel) continue;
+            f32x4 gg = gv[it], mm = mv[it];
+            float uu[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float gout = gg[k], mk = mm[k];
+                uu[k] = momentum_one<T>(gg[k], &mk, has_m, w, beta, nesterov, &gout);
+                mm[k] = mk;
+                gg[k] = gout;
+                const float ub = round_bf(uu[k]);
+                ss = fmaf(ub, ub, ss);
+            }
+            if (has_m) Stored<T>::st4(mom + e, mm);
+            if (write_g) Stored<T>::st4(g + e, gg);
+            u32x2e pk;
+            pk.x = pack2bf(uu[0], uu[1]);
+            pk.y = pack2bf(uu[2], uu[3]);
+            gst2u(u + e, pk);
+        }
+        if constexpr (!FULL) {
+            const int64_t rest = numel & ~static_cast<int64_t>(EW_VEC - 1);
+            if (static_cast<int>((rest - base) / EW_VEC) % EW_THREADS != static_cast<int>(threadIdx.x)) return;
+            float gs[EW_VEC - 1], ms[EW_VEC - 1];
+#pragma unroll
+            for (int k = 0; k < EW_VEC - 1; ++k) {
+                const bool in = rest + k < numel;
+                gs[k] = in ? Stored<T>::ld(g + rest + k) : 0.f;
+                ms[k] = in && has_m ? Stored<T>::ld(mom + rest + k) : 0.f;
+            }
+#pragma unroll
+            for (int k = 0; k < EW_VEC - 1; ++k) {
+                const int64_t e = rest + k;
+                if (e >= numel) continue;
+                float gout = gs[k], mk = ms[k];
+                const uint16_t ub = f2bf(momentum_one<T>(gs[k], &mk, has_m, w, beta, nesterov, &gout));
+                if (has_m) Stored<T>::st(mom + e, mk);
+                if (write_g) Stored<T>::st(g + e, gout);
+                u[e] = ub;
+                const float uf = bf2f(ub);
+                ss = fmaf(uf, uf, ss);
+            }
+        }
+    };
     for (int pass = 0; pass < EW_PASSES; ++pass) {
         const int64_t base = block_base + static_cast<int64_t>(pass) * EW_PASS_ELEMS;
         if (base >= numel) break;
-        if (aligned && base + EW_PASS_ELEMS <= numel) {
-            f32x4 gv[EW_ITERS], mv[EW_ITERS];
-#pragma unroll
-            for (int it = 0; it < EW_ITERS; ++it) {
-                const int64_t e = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
-                gv[it] = Stored<T>::ld4(g + e);
-                if (has_m) mv[it] = Stored<T>::ld4(mom + e);
-                else mv[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-#pragma unroll
-            for (int it = 0; it < EW_ITERS; ++it) {
-                const int64_t e = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
-                f32x4 gg = gv[it], mm = mv[it];
-                float uu[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    float gout = gg[k], mk = mm[k];
-                    uu[k] = momentum_one<T>(gg[k], &mk, has_m, w, beta, nesterov, &gout);
-                    mm[k] = mk;
-                    gg[k] = gout;
-                    const float ub = round_bf(uu[k]);
-                    ss = fmaf(ub, ub, ss);
-                }
-                if (has_m) Stored<T>::st4(mom + e, mm);
-                if (write_g) Stored<T>::st4(g + e, gg);
-                u32x2e pk;
-                pk.x = pack2bf(uu[0], uu[1]);
-                pk.y = pack2bf(uu[2], uu[3]);
-                gst2u(u + e, pk);
-            }
-        } else {
-            for (int it = 0; it < EW_ITERS; ++it) {
-                const int64_t e0 = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
-#pragma unroll
-                for (int k = 0; k < EW_VEC; ++k) {
-                    const int64_t e = e0 + k;
-                    if (e >= numel) break;
-                    const float gval = Stored<T>::ld(g + e);
-                    float mval = has_m ? Stored<T>::ld(mom + e) : 0.f;
-                    float gout = gval;
-                    const float uval = momentum_one<T>(gval, &mval, has_m, w, beta, nesterov, &gout);
-                    if (has_m) Stored<T>::st(mom + e, mval);
-                    if (write_g) Stored<T>::st(g + e, gout);
-                    const uint16_t ub = f2bf(uval);
-                    u[e] = ub;
-                    const float uf = bf2f(ub);
-                    ss = fmaf(uf, uf, ss);
-                }
-            }
-        }
+        if (base + EW_PASS_ELEMS <= numel) pass_over(base, std::true_type{});
+        else pass_over(base, std::false_type{});
     }
     return ss;
 }
@@ -460,13 +479,10 @@ __device__ __forceinline__ void adam_block(const MuonAdamDesc& d, int64_t block_
     T* __restrict__ m = static_cast<T*>(d.exp_avg);
     T* __restrict__ v = static_cast<T*>(d.exp_avg_sq);
     T* __restrict__ upd = static_cast<T*>(d.update);
-    constexpr uintptr_t A = Stored<T>::kAlign;
-    const bool aligned = aligned_to(p, A) && aligned_to(g, A) && aligned_to(m, A) && aligned_to(v, A) &&
-                         aligned_to(upd, A);
     for (int pass = 0; pass < EW_PASSES; ++pass) {
         const int64_t base = block_base + static_cast<int64_t>(pass) * EW_PASS_ELEMS;
         if (base >= numel) break;
-        if (aligned && base + EW_PASS_ELEMS <= numel) {
+        if (base + EW_PASS_ELEMS <= numel) {
             f32x4 gv[EW_ITERS], mv[EW_ITERS], vv[EW_ITERS], pv[EW_ITERS];
 #pragma unroll
             for (int it = 0; it < EW_ITERS; ++it) {
@@ -495,34 +511,57 @@ __device__ __forceinline__ void adam_block(const MuonAdamDesc& d, int64_t block_
                 if (upd) Stored<T>::st4(upd + e, uu);
             }
         } else {
-            // The last, partial pass of a tensor (or a tensor at an odd address): element accesses, four
-            // elements at a time with their loads ahead of the arithmetic.  The loop stays rolled: a
-            // launch over a few small tensors runs this code once per wave, and what it then waits for
-            // is the instruction fetch (unrolled, the pass is several thousand instructions long).
-#pragma unroll 1
-            for (int it = 0; it < EW_ITERS; ++it) {
-                const int64_t e0 = base + (it * EW_THREADS + threadIdx.x) * EW_VEC;
-                if (e0 >= numel) break;
-                float gs[EW_VEC], ms[EW_VEC], vs[EW_VEC], ps[EW_VEC];
+            // The last, partial pass of a tensor, with the loads of a group ahead of the arithmetic of the group
+            // before.  The loop stays rolled: a launch over a few small tensors runs this code once per wave, and
+            // what it then waits for is the instruction fetch (unrolled, the pass is several thousand instructions long).
+            f32x4 gn, mn, vn, pn;
+            const auto fetch = [&](int64_t e) {
+                gn = mn = vn = pn = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (e + EW_VEC <= numel) {
+                    gn = Stored<T>::ld4(g + e);
+                    mn = Stored<T>::ld4(m + e);
+                    vn = Stored<T>::ld4(v + e);
+                    if (p) pn = Stored<T>::ld4(p + e);
+                } else {
 #pragma unroll
-                for (int k = 0; k < EW_VEC; ++k) {
-                    const int64_t e = e0 + k;
-                    const bool in = e < numel;
-                    gs[k] = in ? Stored<T>::ld(g + e) : 0.f;
-                    ms[k] = in ? Stored<T>::ld(m + e) : 0.f;
-                    vs[k] = in ? Stored<T>::ld(v + e) : 0.f;
-                    ps[k] = (in && p) ? Stored<T>::ld(p + e) : 0.f;
+                    for (int k = 0; k < EW_VEC - 1; ++k) {
+                        if (e + k >= numel) continue;
+                        gn[k] = Stored<T>::ld(g + e + k);
+                        mn[k] = Stored<T>::ld(m + e + k);
+                        vn[k] = Stored<T>::ld(v + e + k);
+                        if (p) pn[k] = Stored<T>::ld(p + e + k);
+                    }
                 }
+            };
+            int64_t e = base + threadIdx.x * EW_VEC;
+            fetch(e);
+#pragma unroll 1
+            for (; e < numel; e += EW_THREADS * EW_VEC) {
+                const f32x4 gg = gn;
+                f32x4 mm = mn, v2 = vn, pp = pn, uu;
+                fetch(e + EW_THREADS * EW_VEC);
 #pragma unroll
                 for (int k = 0; k < EW_VEC; ++k) {
-                    const int64_t e = e0 + k;
-                    if (e >= numel) continue;
-                    float mm = ms[k], v2 = vs[k];
-                    const float uu = adam_one<T>(gs[k], &mm, &v2, w1, w2, eps, bias1, bias2);
-                    Stored<T>::st(m + e, mm);
-                    Stored<T>::st(v + e, v2);
-                    if (p) Stored<T>::st(p + e, apply_one<T>(ps[k], uu, neg_lr, wd_factor));
-                    if (upd) Stored<T>::st(upd + e, uu);
+                    float mk = mm[k], vk = v2[k];
+                    uu[k] = adam_one<T>(gg[k], &mk, &vk, w1, w2, eps, bias1, bias2);
+                    mm[k] = mk;
+                    v2[k] = vk;
+                    pp[k] = apply_one<T>(pp[k], uu[k], neg_lr, wd_factor);
+                }
+                if (e + EW_VEC <= numel) {
+                    Stored<T>::st4(m + e, mm);
+                    Stored<T>::st4(v + e, v2);
+                    if (p) Stored<T>::st4(p + e, pp);
+                    if (upd) Stored<T>::st4(upd + e, uu);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < EW_VEC - 1; ++k) {
+                        if (e + k >= numel) continue;
+                        Stored<T>::st(m + e + k, mm[k]);
+                        Stored<T>::st(v + e + k, v2[k]);
+                        if (p) Stored<T>::st(p + e + k, pp[k]);
+                        if (upd) Stored<T>::st(upd + e + k, uu[k]);
+                    }
                 }
             }
         }
