@@ -206,7 +206,7 @@ typedef struct MuonChunkRun {
     int32_t flags;                      /* MUON_AMD_ROUND_*                                        */
     int32_t split_slots;                /* counters to clear before the products                   */
     int32_t aol_mode, aol_row_blocks, aol_seg_blocks;
-    int32_t reserved;
+    int32_t norm_in_normalize;          /* 1: the normalise launch forms the norms itself         */
 } MuonChunkRun;
 
 int         muon_amd_abi_version(void);

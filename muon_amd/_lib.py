@@ -59,7 +59,7 @@ CHUNK_RUN = np.dtype(
      ("launches", CHUNK_LAUNCH, (len(LAUNCH_KINDS),)), ("scalars", "<u8"), ("split_partials", "<u8"), ("split_counters", "<u8"),
      ("aol", "<u8"), ("aol_row_prefix", "<u8"), ("aol_seg_prefix", "<u8"), ("nmat", "<i4"), ("nblocks", "<i4"), ("ntiles", "<i4"),
      ("steps", "<i4"), ("flags", "<i4"), ("split_slots", "<i4"), ("aol_mode", "<i4"), ("aol_row_blocks", "<i4"),
-     ("aol_seg_blocks", "<i4"), ("reserved", "<i4")],
+     ("aol_seg_blocks", "<i4"), ("norm_in_normalize", "<i4")],
     align=True)
 
 _c_int = ctypes.c_int

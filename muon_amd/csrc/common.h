@@ -28,6 +28,9 @@ int check_launch(const char* what);
 // leaves them zero, but one that died half way must not poison every later step).
 int launch_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags, int32_t* clear, int nclear,
                          hipStream_t stream);
+// Both in one launch: muon_amd_normalize with the denominators formed from the partial sums.
+int launch_norm_normalize(const MuonMatDesc* descs_dev, const int32_t* tile_prefix_dev, int nmat, int ntiles, float eps,
+                          int flags, int32_t* clear, int nclear, hipStream_t stream);
 
 // Raises the dynamic-LDS limit of the kernels of small.hip (part of muon_amd_init).
 int raise_small_limits();

@@ -233,27 +233,23 @@ __global__ __launch_bounds__(EW_THREADS) void momentum_kernel(
 // ------------------------------------------------------------------------------------------
 // norm finalize: muon.py:282  (X.norm(dim=(-2,-1)) + 1e-7)
 // ------------------------------------------------------------------------------------------
+// The denominator of a matrix from its partial sums, by every lane of a wave.
+__device__ __forceinline__ float norm_plus_eps(const MuonMatDesc& d, float eps, int round_reference, int lane) {
+    if (round_reference == 2) return 1.f;          // no pre-scale: the AOL variant rescales by rows instead
+    float s = 0.f;
+    for (int i = d.part_begin + lane; i < d.part_end; i += 64) s += d.partials[i];
+    const float nrm = sqrtf(wave_sum(s));
+    // the norm of a bf16 tensor is a bf16 tensor, and so is that + a python scalar
+    return round_reference ? round_bf(round_bf(nrm) + eps) : nrm + eps;
+}
+
 __global__ __launch_bounds__(64) void norm_finalize_kernel(const MuonMatDesc* __restrict__ descs,
                                                             float eps, int round_reference,
                                                             int32_t* __restrict__ clear, int nclear) {
     for (int i = blockIdx.x * 64 + threadIdx.x; i < nclear; i += gridDim.x * 64) clear[i] = 0;
     const MuonMatDesc d = descs[blockIdx.x];
-    float s = 0.f;
-    for (int i = d.part_begin + threadIdx.x; i < d.part_end; i += 64) s += d.partials[i];
-    s = wave_sum(s);
-    if (threadIdx.x == 0) {
-        float nrm = sqrtf(s);
-        float den;
-        if (round_reference == 2) {
-            den = 1.f;                     // no pre-scale: the AOL variant rescales by rows instead
-        } else if (round_reference) {
-            nrm = round_bf(nrm);           // the norm of a bf16 tensor is a bf16 tensor
-            den = round_bf(nrm + eps);     // bf16 tensor + python scalar -> bf16 tensor
-        } else {
-            den = nrm + eps;
-        }
-        *d.denom = den;
-    }
+    const float den = norm_plus_eps(d, eps, round_reference, threadIdx.x);
+    if (threadIdx.x == 0) *d.denom = den;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -279,9 +275,13 @@ __device__ __forceinline__ void gst4u(uint16_t* p, u32x4e v) {     // read again
 // blocks than the GPU holds: so 512 threads per tile rather than 256, 16-byte loads also where a row's length is
 // no multiple of 8, and a division of three instructions.  1500 x 1100 Newton-Schulz 178 -> 169 us (the
 // launch alone 19 us before), one 768 x 3072 step 179 -> 176 us, 8 Llama-3-8B layers the same.
+// NORM: every wave forms the denominator of its matrix from the partial sums, under the loads of the tile (the order of
+// the sum is norm_finalize_kernel's, whose launch this saves), and the launch clears the counters of split reductions.
+template <bool NORM>
 __global__ __launch_bounds__(NT_THREADS) void normalize_kernel(const MuonMatDesc* __restrict__ descs,
                                                          const int32_t* __restrict__ prefix,
-                                                         int nmat) {
+                                                         int nmat, float eps, int round_reference,
+                                                         int32_t* __restrict__ clear, int nclear) {
     constexpr int PITCH = NT_TILE / 2 + 2;               // words per LDS row (even: 8-byte stores)
     __shared__ __align__(8) uint32_t tile[NT_TILE][PITCH];
     const int b = blockIdx.x;
@@ -290,9 +290,9 @@ __global__ __launch_bounds__(NT_THREADS) void normalize_kernel(const MuonMatDesc
     const int lb = b - prefix[mi];
     const int tiles_c = d.cols_p / NT_TILE;
     const int R0 = (lb / tiles_c) * NT_TILE, C0 = (lb % tiles_c) * NT_TILE;
-    const float den = *d.denom;
     const uint16_t* __restrict__ u = d.u;
-    const UniformDivisor by(den);
+    if constexpr (NORM)
+        for (int i = b * NT_THREADS + threadIdx.x; i < nclear; i += gridDim.x * NT_THREADS) clear[i] = 0;
 
     constexpr int CH = NT_TILE / 8;                      // 8-element chunks per tile row
     constexpr int NI = NT_TILE * CH / NT_THREADS;        // chunks per thread
@@ -317,6 +317,10 @@ __global__ __launch_bounds__(NT_THREADS) void normalize_kernel(const MuonMatDesc
             }
         }
     }
+    float den;
+    if constexpr (NORM) den = norm_plus_eps(d, eps, round_reference, threadIdx.x & 63);
+    else den = *d.denom;
+    const UniformDivisor by(den);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int q = threadIdx.x + i * NT_THREADS;
@@ -593,13 +597,23 @@ __global__ __launch_bounds__(EW_THREADS) void adam_kernel(const MuonAdamDesc* __
         adam_block<float>(d, block_base, neg_lr, wd_factor, w1, w2, eps, bias1, bias2);
 }
 
+static int norm_mode(int flags) { return (flags & MUON_AMD_NORM_UNIT) ? 2 : ((flags & MUON_AMD_ROUND_REFERENCE) ? 1 : 0); }
+
 int launch_norm_finalize(const MuonMatDesc* descs_dev, int nmat, float eps, int flags, int32_t* clear, int nclear,
                          hipStream_t stream) {
     MUON_REQUIRE(descs_dev, "norm_finalize: null table");
     MUON_REQUIRE(nmat > 0, "norm_finalize: nmat=%d", nmat);
-    hipLaunchKernelGGL(norm_finalize_kernel, dim3(nmat), dim3(64), 0, stream, descs_dev, eps,
-                       (flags & MUON_AMD_NORM_UNIT) ? 2 : ((flags & MUON_AMD_ROUND_REFERENCE) ? 1 : 0), clear, nclear);
+    hipLaunchKernelGGL(norm_finalize_kernel, dim3(nmat), dim3(64), 0, stream, descs_dev, eps, norm_mode(flags), clear, nclear);
     return check_launch("norm_finalize");
+}
+
+int launch_norm_normalize(const MuonMatDesc* descs_dev, const int32_t* tile_prefix_dev, int nmat, int ntiles, float eps,
+                          int flags, int32_t* clear, int nclear, hipStream_t stream) {
+    MUON_REQUIRE(descs_dev && tile_prefix_dev, "normalize: null table");
+    MUON_REQUIRE(nmat > 0 && ntiles > 0, "normalize: nmat=%d ntiles=%d", nmat, ntiles);
+    hipLaunchKernelGGL(normalize_kernel<true>, dim3(ntiles), dim3(NT_THREADS), 0, stream, descs_dev, tile_prefix_dev, nmat, eps,
+                       norm_mode(flags), clear, nclear);
+    return check_launch("normalize");
 }
 
 }  // namespace muon_amd
@@ -676,8 +690,8 @@ int muon_amd_normalize(const MuonMatDesc* descs_dev, const int32_t* tile_prefix_
                        int ntiles, void* stream) {
     MUON_REQUIRE(descs_dev && tile_prefix_dev, "normalize: null table");
     MUON_REQUIRE(nmat > 0 && ntiles > 0, "normalize: nmat=%d ntiles=%d", nmat, ntiles);
-    hipLaunchKernelGGL(normalize_kernel, dim3(ntiles), dim3(NT_THREADS), 0,
-                       static_cast<hipStream_t>(stream), descs_dev, tile_prefix_dev, nmat);
+    hipLaunchKernelGGL(normalize_kernel<false>, dim3(ntiles), dim3(NT_THREADS), 0,
+                       static_cast<hipStream_t>(stream), descs_dev, tile_prefix_dev, nmat, 0.f, 0, nullptr, 0);
     return check_launch("normalize");
 }
 

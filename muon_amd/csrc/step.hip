@@ -45,11 +45,16 @@ int muon_amd_run_chunk(const MuonChunkRun* run, float one_minus_beta, float beta
             return muon_amd_momentum(c.mats, c.block_prefix, c.nmat, c.nblocks, one_minus_beta, beta, nesterov,
                                      mutate_grad, scalars_dev, stream);
         });
-    go([&] {
-        return launch_norm_finalize(c.mats, c.nmat, eps, c.flags | (c.aol ? MUON_AMD_NORM_UNIT : 0), c.split_counters,
-                                    c.split_slots, go.stream);
-    });
-    go([&] { return muon_amd_normalize(c.mats, c.tile_prefix, c.nmat, c.ntiles, stream); });
+    const int norm_flags = c.flags | (c.aol ? MUON_AMD_NORM_UNIT : 0);
+    if (c.norm_in_normalize) {
+        go([&] {
+            return launch_norm_normalize(c.mats, c.tile_prefix, c.nmat, c.ntiles, eps, norm_flags, c.split_counters,
+                                         c.split_slots, go.stream);
+        });
+    } else {
+        go([&] { return launch_norm_finalize(c.mats, c.nmat, eps, norm_flags, c.split_counters, c.split_slots, go.stream); });
+        go([&] { return muon_amd_normalize(c.mats, c.tile_prefix, c.nmat, c.ntiles, stream); });
+    }
     const auto gemm = [&](int desc, int kind, const float* abg, int extra) {
         const MuonChunkLaunch& ln = c.launches[kind];
         float* const partials = ln.split_slots ? c.split_partials : nullptr;

@@ -220,6 +220,7 @@ class _ChunkRuntime:
             r["aol_mode"] = _lib.AOL_ROWS_ONLY if c.variant == "aol4_rows" else _lib.AOL_SYMMETRIC
             r["aol_row_blocks"], r["aol_seg_blocks"] = int(c.aol_row_prefix[-1]), int(c.aol_seg_prefix[-1])
         r["nmat"], r["nblocks"], r["ntiles"], r["steps"] = c.nmat, c.nblocks, c.ntiles, c.steps
+        r["norm_in_normalize"] = c.norm_in_normalize
         r["flags"] = _lib.ROUND_REFERENCE if c.reference_rounding else _lib.ROUND_FUSED
         return r
 
@@ -236,7 +237,9 @@ class _ChunkRuntime:
         if not skip_momentum:
             out.append(("momentum", sum(lay.numel * (sz + 2 + (2 * sz if has_m else 0))
                                         for lay, sz, (has_m, _, _) in zip(c.layouts, store, self.present))))
-        out += [("norm_finalize", c.nblocks * 4), ("normalize", elts * 2 + padded * 2)]
+        if not c.norm_in_normalize:
+            out.append(("norm_finalize", c.nblocks * 4))
+        out.append(("normalize", elts * 2 + padded * 2))
         syrk = sum(lay.m * (lay.m + 1) * lay.n for lay in c.layouts)
         poly = sum(lay.m * lay.m * (lay.m + 1) for lay in c.layouts)
         update = sum(2 * lay.m * lay.m * lay.n for lay in c.layouts)

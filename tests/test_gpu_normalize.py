@@ -38,3 +38,24 @@ def test_normalise_beyond_the_range_of_the_short_division(shape, monkeypatch):
     assert (_normalised(torch.zeros_like(G)) == 0).all()
     G[3, 5] = float("nan")
     assert _normalised(G).isnan().all()
+
+
+@pytest.mark.parametrize("shapes", [[(1, 9)], [(130, 700)], [(1000, 520), (520, 1000), (128, 8192)]])
+def test_norms_formed_in_the_normalise_launch(shapes, monkeypatch):
+    """Norms from the normalise launch itself and from a launch of their own: the same bits (one to 64 partial sums;
+    128 x 8192 has a split reduction, whose counters either launch clears)."""
+    import muon_amd
+    from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
+    results = []
+    for blocks in ((0, 0), (512, 4096)):
+        monkeypatch.setattr(plan, "NORM_IN_NORMALIZE_BLOCKS", blocks)
+        torch.manual_seed(3)
+        params = [torch.nn.Parameter(torch.randn(*s, device="cuda")) for s in shapes]
+        opt = muon_amd.SingleDeviceMuon(params, lr=0.02)
+        for _ in range(2):
+            for p in params:
+                p.grad = torch.randn_like(p)
+            opt.step()
+        results.append([p.detach().clone() for p in params])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
