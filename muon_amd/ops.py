@@ -10,8 +10,8 @@ Arithmetic: bf16 operands, fp32 accumulation, one rounding to bf16 of the finish
 the reference's kernels do (muon.py:399-400, 531-536, 675-696).  The two symmetric products compute
 the tiles on and above the diagonal and store each with its mirror image (muon.py:402-413): for a
 symmetric A, which ns_line_2 asks for, that is the whole result; otherwise what lands below the
-diagonal tiles is the image of what is above them, and depends on the tile size here (64, 128 or 256)
-as it does on the autotuned block in the reference.  bf16 CUDA tensors only; any strides; 2-D or
+diagonal blocks is the image of what is above them, and depends on their size (here 128, and 256 from
+1024 rows on) as it does on the autotuned block in the reference.  bf16 CUDA tensors only; any strides; 2-D or
 3-D (a batch).
 
 The optimizer classes do not come through here: they run the same kernel over whole parameter
@@ -31,18 +31,20 @@ from .functional import _PRODUCT_CACHE, _PRODUCT_CACHE_MAX, _cached, _exclusive
 
 
 def _product_jobs(tile_class: int, batch: int, rows_p: int, cols_p: int, kdim: int, sym: bool,
-                  nsplit: int = 1) -> np.ndarray:
+                  nsplit: int = 1, direct: int = 1) -> np.ndarray:
     """One job per output tile and matrix (for a mirrored product: per tile on or above the
     diagonal), in super-block order dealt to the XCDs.  nsplit > 1: the reduction of every tile is
     shared by nsplit jobs that meet in a group of fp32 slots (tile t of the launch: slots
-    t * nsplit ..), as the optimizer does for the X X^T of short, very wide matrices."""
+    t * nsplit ..), as the optimizer does for the X X^T of short, very wide matrices.  direct: every
+    tile of a diagonal block of so many tile rows is computed, only the blocks above are mirrored."""
     TR, TC = _plan.TILE_DIMS[tile_class]
     si, sj = _plan.SUPER_DIMS[tile_class]
-    ti, tj = _plan._tile_order(rows_p // TR, cols_p // TC, sym, TR // TC, si, sj)
+    ti, tj = _plan._tile_order(rows_p // TR, cols_p // TC, sym, TR // TC, si, sj, direct)
     one = np.zeros(len(ti) * nsplit, dtype=_lib.TILE_JOB)
     one["i0"], one["j0"] = np.repeat(ti * TR, nsplit), np.repeat(tj * TC, nsplit)
     if sym:
-        one["diag"] = np.repeat((ti == tj // (TR // TC)).astype(np.int32), nsplit)
+        tr = tj // (TR // TC)
+        one["diag"] = np.repeat(np.where(ti == tr, 1, np.where(ti // direct == tr // direct, 2, 0)).astype(np.int32), nsplit)
     if nsplit == 1:
         one["k1"] = kdim
     else:
@@ -71,8 +73,8 @@ class _Product:
     their counters, of one product shape on one device."""
 
     def __init__(self, device, tile_class: int, batch: int, rows_p: int, cols_p: int, kdim: int, sym: bool,
-                 nsplit: int = 1):
-        self.jobs = _product_jobs(tile_class, batch, rows_p, cols_p, kdim, sym, nsplit)
+                 nsplit: int = 1, direct: int = 1):
+        self.jobs = _product_jobs(tile_class, batch, rows_p, cols_p, kdim, sym, nsplit, direct)
         self.device = device
         self.tile_class = tile_class
         self.batch = batch
@@ -143,6 +145,22 @@ def _addresses(t3: torch.Tensor, batch: int):
     return [t3.data_ptr() + k * step for k in range(batch)]
 
 
+def _symmetric_plan(batch: int, M: int, K: int, addend: bool):
+    """-> (tile class, padded M, padded K, jobs that share a reduction, tile rows of a diagonal block) of a
+    mirrored product."""
+    own = _plan.tile_class_for(M)
+    kp = _plan._round_up(K, _plan.GEMM_BK)
+    # X X^T of a short, very wide matrix: a few tiles with very long reductions, which are split
+    nsplit = 1 if addend or own != 0 else _plan.split_factor(_plan._round_up(M, 128), kp)
+    tile_class = _launch_class("poly" if addend else "gram", own, batch, M, K)
+    mp = _plan._round_up(M, _plan.pad_unit(tile_class))
+    # X X^T is symmetric bit for bit.  alpha A A^T + beta A is as symmetric as A: for another A, which elements are
+    # computed and which are mirrored stays what the matrix's own tiles make of it, whatever tiles the launch takes
+    # (up to 128 rows everything is computed).  That is 17 tiles of 64 x 64 instead of 15 for 320 rows.
+    direct = _plan.TILE_DIMS[own][0] // _plan.TILE_DIMS[tile_class][0] if addend else 1
+    return tile_class, mp, mp if addend else kp, nsplit, direct
+
+
 def _symmetric_product(A: torch.Tensor, out, alpha: float, beta: float, addend: bool) -> torch.Tensor:
     M, K = A.shape[-2:]
     if out is None:
@@ -157,17 +175,10 @@ def _symmetric_product(A: torch.Tensor, out, alpha: float, beta: float, addend: 
         return out
     A3, out3 = _as_batch(A), _as_batch(out)
     batch = A3.size(0)
-    tile_class = _plan.tile_class_for(M)
-    kp = _plan._round_up(K, _plan.GEMM_BK)
-    # X X^T of a short, very wide matrix: a few tiles with very long reductions, which are split
-    nsplit = 1 if addend or tile_class != 0 else _plan.split_factor(_plan._round_up(M, 128), kp)
-    tile_class = _launch_class("poly" if addend else "gram", tile_class, batch, M, K)
-    mp = _plan._round_up(M, _plan.pad_unit(tile_class))
-    if addend:
-        kp = mp
+    tile_class, mp, kp, nsplit, direct = _symmetric_plan(batch, M, K, addend)
     with torch.cuda.device(A.device):
-        prod = _cached(("sym_product", A.device, tile_class, batch, mp, kp, nsplit),
-                       lambda: _Product(A.device, tile_class, batch, mp, mp, kp, True, nsplit),
+        prod = _cached(("sym_product", A.device, tile_class, batch, mp, kp, nsplit, direct),
+                       lambda: _Product(A.device, tile_class, batch, mp, mp, kp, True, nsplit, direct),
                        _PRODUCT_CACHE, _PRODUCT_CACHE_MAX)
         with _exclusive(prod, A.device):
             src = _padded(A3, mp, kp)

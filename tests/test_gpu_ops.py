@@ -188,3 +188,24 @@ def test_operators_against_the_golden_fixture(M, golden_dir):
                  ("line3", M.ns_line_3(B.cuda(), X.cuda(), 3.4445), 3.4445 * Xd + Bd @ Xd))
         for key, got, terms in cases:
             _check(got, torch.from_numpy(z[f"{name}/{key}_exact"]).double(), terms, bf(z[f"{name}/{key}"]), f"{name} {key}")
+
+
+@pytest.mark.parametrize("shape", [(2, 40, 40), (1, 128, 128), (4, 160, 160), (1, 300, 300), (32, 200, 200), (1, 1100, 1100)])
+def test_ns_line_2_of_a_matrix_that_is_not_symmetric(M, shape):
+    """The blocks on and above the diagonal are computed, those below hold their mirror images; the blocks are those of
+    the matrix's own tile class (128, from a short side of 1024 on 256), whatever tiles the launch takes: up to
+    128 rows the result is exact for any square matrix."""
+    from muon_amd import plan
+    A = _rand(shape, 0.05, 41)
+    m = shape[-1]
+    T = plan.TILE_DIMS[plan.tile_class_for(m)][0]
+    got = M.ns_line_2(A.cuda(), C_, B_).cpu()
+    Ad = A.double()
+    exact = C_ * (Ad @ Ad.mT) + B_ * Ad
+    terms = abs(C_) * (Ad.abs() @ Ad.abs().mT) + abs(B_) * Ad.abs()
+    block = torch.arange(m) // T
+    below = block[:, None] > block[None, :]
+    exact, terms = torch.where(below, exact.mT, exact), torch.where(below, terms.mT, terms)
+    bound = 2.0 ** -8 * 1.001 * exact.abs() + 2.0 ** -13 * terms
+    assert ((got.double() - exact).abs() <= bound).all()
+    assert torch.equal(got[..., below], got.mT[..., below])

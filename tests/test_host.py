@@ -644,3 +644,28 @@ def test_build_refuses_store_data_overwritten_behind_the_store():
             check_store_data(text)
     for text in (store + "\ts_nop 1\n" + bad, store + "\tv_add_u32_e32 v174, v170, v199\n", store + "\ts_nop 0\n\ts_mov_b32 s1, s2\n" + bad):
         assert check_store_data(text) == 1
+
+
+@pytest.mark.parametrize("m", [40, 65, 128, 192, 300, 520, 1024, 1100, 1536])
+@pytest.mark.parametrize("batch", [1, 4, 32])
+def test_mirrored_region_of_ns_line_2_does_not_depend_on_the_tiles(m, batch):
+    """Which elements of alpha A A^T + beta A are computed and which are mirrored (visible for an A that is not
+    symmetric) follows from the matrix's own tile class, also where a launch takes smaller tiles."""
+    from muon_amd import ops
+    own = plan.tile_class_for(m)
+    T = plan.TILE_DIMS[own][0]
+    i, j = np.indices((m, m))
+    want = np.where(i // T == j // T, 1, np.where(i < j, 1, 2))           # computed, or the image of what is above
+    tile_class, mp, kp, nsplit, direct = ops._symmetric_plan(batch, m, m, True)
+    jobs = ops._product_jobs(tile_class, batch, mp, mp, kp, True, nsplit, direct)
+    t = plan.TILE_DIMS[tile_class][0]
+    got = np.zeros((mp, mp), dtype=np.int64)
+    for job in jobs[jobs["desc"] == 0]:
+        rows, cols = slice(job["i0"], job["i0"] + t), slice(job["j0"], job["j0"] + t)
+        assert (got[rows, cols] == 0).all()
+        got[rows, cols] = 1
+        if not job["diag"]:
+            assert (got[cols, rows] == 0).all()
+            got[cols, rows] = 2
+    assert (got[:m, :m] == want).all()
+    assert (jobs["k0"] == 0).all() and (jobs["k1"] == kp).all() and len(jobs) == batch * (jobs["desc"] == 0).sum()
