@@ -59,13 +59,6 @@ __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
 __device__ __forceinline__ float bf_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-// bf16(x) + bf16(y) in fp32, for x and y as pack2bf leaves them: one dot product with (1, 1) in place of two unpacking
-// instructions and an addition.  Its sum of two bf16 values rounds to the same bf16 value as the fp32 sum
-// for all 2^32 pairs (checked on the device over every pair; NaNs stay NaNs, -0 + -0 gives +0).
-__device__ __forceinline__ float bf_pair_sum(uint32_t p) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, p), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), 0.f, false);
-}
-
 // Division of many values by one positive b, correctly rounded as `/` is, without its scaling steps: with y = 1 / b
 // correctly rounded, q = x y and the exact remainder x - b q, the quotient is q + (x - b q) y (P. Markstein,
 // "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Three

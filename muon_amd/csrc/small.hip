@@ -127,9 +127,11 @@ __device__ __forceinline__ void tile_add(uint32_t (&po)[8], const f32x16& acc, f
     for (int k = 0; k < 8; ++k) {
         const uint32_t dk = po[k];
         if constexpr (ROUND) {
-            // every term rounded to bf16, their sum rounded again
-            po[k] = pack2bf(bf_pair_sum(pack2bf(alpha * acc[2 * k], beta * bf_lo(dk))),
-                            bf_pair_sum(pack2bf(alpha * acc[2 * k + 1], beta * bf_hi(dk))));
+            // every term rounded to bf16, their sum rounded again, by the instructions of the GEMM epilogue (a dot
+            // product with (1, 1) in place of unpacking and adding gives +0 for -0 + -0)
+            const uint32_t t1 = pack2bf(alpha * acc[2 * k], alpha * acc[2 * k + 1]);
+            const uint32_t t2 = pack2bf(beta * bf_lo(dk), beta * bf_hi(dk));
+            po[k] = pack2bf(bf_lo(t1) + bf_lo(t2), bf_hi(t1) + bf_hi(t2));
         } else {
             po[k] = pack2bf(fmaf(alpha, acc[2 * k], beta * bf_lo(dk)), fmaf(alpha, acc[2 * k + 1], beta * bf_hi(dk)));
         }

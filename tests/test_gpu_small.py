@@ -72,3 +72,27 @@ def test_what_does_not_fit_one_workgroup_takes_the_general_path():
     assert [lib.muon_amd_small_class(*s) for s in ((129, 129), (128, 321), (64, 1089), (32, 5000), (1, 200000))] == [0] * 5
     assert [lib.muon_amd_small_class(*s) for s in ((128, 320), (320, 128), (64, 1088), (20, 2000))] == [128, 128, 64, 32]
     assert plan.small_groups([(64, 64), (256, 256)]) is None and plan.small_groups([(64, 64)], "aol4") is None
+
+
+@pytest.mark.parametrize("rounding", ["reference", "fused"])
+@pytest.mark.parametrize("steps", [1, 2, 5])
+def test_small_step_gives_the_signs_of_zeros_of_the_general_path(rounding, steps, monkeypatch):
+    """Terms that round to negative zeros: rows that are orthogonal up to products near the smallest bf16 value, and
+    elements that are negative zeros themselves.  Compared as bit patterns."""
+    import muon_amd
+    from muon_amd import plan
+    torch.manual_seed(11)
+    G = torch.zeros(200, 8, 40)
+    sign = torch.randint(0, 2, G.shape) * 2.0 - 1
+    G = torch.where(torch.rand(G.shape) < 0.3, 10.0 ** (torch.rand(G.shape) * 24 - 44), G) * sign     # signed zeros among them
+    G[:, torch.arange(8), torch.arange(8)] = 1.0
+    G[:, 1::3, 20:] *= 1e21                              # some factors whose products with those are subnormal
+    G = G.cuda()
+    got = []
+    for small in (True, False):
+        monkeypatch.setattr(plan, "SMALL", small)
+        muon_amd.clear_engine_cache()
+        got.append(muon_amd.zeropower_via_newtonschulz5(G, steps=steps, rounding=rounding).view(torch.int16))
+    muon_amd.clear_engine_cache()
+    assert (got[1] == -0x8000).any() and (got[1] == 0).any()
+    assert torch.equal(*got)
