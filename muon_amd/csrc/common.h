@@ -51,6 +51,7 @@ __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 // Two fp32 values rounded to bf16 and packed (lo in bits 0-15): one v_cvt_pk_bf16_f32.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
     const f32x2_t v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
@@ -59,11 +60,14 @@ __device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
 __device__ __forceinline__ float bf_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
 
-// Division of many values by one positive b, correctly rounded as `/` is, without its scaling steps: with y = 1 / b
-// correctly rounded, q = x y and the exact remainder x - b q, the quotient is q + (x - b q) y (P. Markstein,
+// Division of many bf16 values by one positive b, rounded to fp32 as `/` rounds it, without its scaling steps: with
+// y = 1 / b correctly rounded, q = x y and the exact remainder x - b q, the quotient is q + (x - b q) y (P. Markstein,
 // "Computation of elementary functions on the IBM RISC System/6000 processor", 1990).  Three
-// instructions per value instead of about ten.  `divide` may be used where `ok` and the quotient is finite (an
-// infinity would come out as NaN); the remainder is formed negated, which keeps the sign of a zero.
+// instructions per value instead of about ten.  The remainder has to be exact and the quotient normal: that is so
+// where b lies in the range `ok` stands for and the magnitude of x is zero or at least 2^-64 (`tiny` finds the
+// others, which go to `/`), and the quotient must be finite (an infinity would come out as NaN).  The remainder
+// is formed negated, which keeps the sign of a zero.  Without the test of x, elements below about 2^-100 were off by
+// one fp32 step now and then, which showed in the bf16 result over fp32 divisors.
 struct UniformDivisor {
     float b, y;
     bool ok;
@@ -72,6 +76,16 @@ struct UniformDivisor {
     __device__ __forceinline__ float divide(float x) const {
         const float q = x * y;
         return fmaf(-fmaf(b, q, -x), y, q);
+    }
+    // Whether any of these pairs of bf16 values holds a magnitude below 2^-64 that is not zero.
+    template <typename V>
+    static __device__ __forceinline__ bool tiny(const V& pairs) {
+        u16x2_t least = {0xffffu, 0xffffu};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)          // (zero wraps around to the largest number)
+            least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2_t, pairs[k] & 0x7fff7fffu) - u16x2_t{1u, 1u});
+        constexpr unsigned short LIMIT = ((127 - 64) << 7) - 1;
+        return least[0] < LIMIT || least[1] < LIMIT;
     }
 };
 

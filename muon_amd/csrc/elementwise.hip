@@ -273,7 +273,8 @@ __device__ __forceinline__ void gst4u(uint16_t* p, u32x4e v) {     // read again
 // rows r .. r+7 holds 8 consecutive elements of the two transposed rows 2c and 2c+1.
 // What bounds it is memory for large launches (5.3 TB/s over the Llama-3-8B layers) and latency for those with fewer
 // blocks than the GPU holds: so 512 threads per tile rather than 256, 16-byte loads also where a row's length is
-// no multiple of 8, and a division of three instructions.  1500 x 1100 Newton-Schulz 178 -> 169 us (the
+// no multiple of 8, and a division of three instructions (with the test for elements it is not exact for, about two
+// more).  1500 x 1100 Newton-Schulz 178 -> 169 us (the
 // launch alone 19 us before), one 768 x 3072 step 179 -> 176 us, 8 Llama-3-8B layers the same.
 // NORM: every wave forms the denominator of its matrix from the partial sums, under the loads of the tile (the order of
 // the sum is norm_finalize_kernel's, whose launch this saves), and the launch clears the counters of split reductions.
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(NT_THREADS) void normalize_kernel(const MuonMatDesc
         for (int k = 0; k < 4; ++k) o[k] = pack2bf(by.divide(bf_lo(raws[i][k])), by.divide(bf_hi(raws[i][k])));
         if (den == 1.f) {                    // (the AOL variant: no pre-scale)
             o = raws[i];
-        } else if (!by.ok) {                 // (an element is at most the norm: only den can be out of range)
+        } else if (!by.ok || UniformDivisor::tiny(raws[i])) {      // (an element is at most the norm: no quotient overflows)
             const bool inside = gr < d.rows;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
             u32x4 o;                                 // (columns beyond n hold zero and stay zero)
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = pack2bf(by.divide(bf_lo(v[k])), by.divide(bf_hi(v[k])));
-            if (!by.ok) {                            // (an element is at most the norm: only den can be out of range)
+            if (!by.ok || UniformDivisor::tiny(v)) { // (an element is at most the norm: no quotient overflows)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) o[k] = pack2bf(bf_lo(v[k]) / den, bf_hi(v[k]) / den);
             }

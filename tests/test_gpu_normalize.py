@@ -59,3 +59,31 @@ def test_norms_formed_in_the_normalise_launch(shapes, monkeypatch):
             opt.step()
         results.append([p.detach().clone() for p in params])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("small", [True, False])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_elements_too_small_for_the_short_division(small, transposed, monkeypatch):
+    """Every bf16 value below 2^-60, zeros of either sign among them, over fp32 denominators: the bits of the ordinary
+    division.  One element per matrix makes the norm, exactly; the squares of the others vanish beside its own."""
+    import muon_amd
+    from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", small)
+    muon_amd.clear_engine_cache()
+    bits = torch.arange((127 - 60) << 7, dtype=torch.int32)
+    values = torch.cat([bits, bits | 0x8000]).to(torch.int16).view(torch.bfloat16)
+    rows, cols = 68, 256
+    assert values.numel() <= rows * cols - 1 < values.numel() + cols
+    # 0.25 .. some hundreds, and two norms for which the short division of such values misses the bf16 result
+    for norm in [0x3E80 + 37 * k for k in range(24)] + [0x38E3, 0x3ABC]:
+        top = torch.tensor([norm], dtype=torch.int16).view(torch.bfloat16)
+        x = torch.zeros(rows * cols, dtype=torch.bfloat16)
+        x[:values.numel()] = values
+        x[-1] = top
+        x = x.view(rows, cols)
+        x = x.T.contiguous() if transposed else x
+        got = muon_amd.zeropower_via_newtonschulz5(x.cuda(), steps=0, rounding="fused").cpu()
+        want = (x.float() / (top.float() + 1e-7)).bfloat16()
+        differ = got.view(torch.int16) != want.view(torch.int16)
+        assert not differ.any(), (float(top), int(differ.sum()), x[differ][:4], got[differ][:4], want[differ][:4])
+    muon_amd.clear_engine_cache()

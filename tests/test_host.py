@@ -669,3 +669,38 @@ def test_mirrored_region_of_ns_line_2_does_not_depend_on_the_tiles(m, batch):
             got[cols, rows] = 2
     assert (got[:m, :m] == want).all()
     assert (jobs["k0"] == 0).all() and (jobs["k1"] == kp).all() and len(jobs) == batch * (jobs["desc"] == 0).sum()
+
+
+def _fma32(a, b, c):
+    """fp32 a * b + c, rounded once: the product is exact in 64 bits, the sum is rounded to odd there, which the
+    rounding to 32 bits then sees as the exact value."""
+    with np.errstate(all="ignore"):
+        p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
+        s = p + c
+        t = s - p
+        err = (p - (s - t)) + (c - t)
+        bits = s.view(np.int64)
+        away = (err != 0) & (bits & 1 == 0)
+        up = (err > 0) == (s > 0)
+        s = np.where(away, np.where(up, bits + 1, bits - 1), bits).view(np.float64)
+        return s.astype(np.float32)
+
+
+def test_short_division_is_the_ordinary_one_where_it_is_taken():
+    """q = x y, q + (x - b q) y with y = 1 / b against x / b: every bf16 x that the kernels divide that way (a
+    magnitude of 2^-64 at least, and at most the divisor's next power of two) and divisors over the range
+    they take, bf16 and fp32 ones; bit for bit, the sign of a zero included."""
+    rng = np.random.default_rng(0)
+    mant = np.concatenate([rng.integers(0, 1 << 23, 60), np.arange(128) << 16, [(1 << 23) - 1]])
+    exps = np.concatenate([rng.integers(127 - 60, 127 + 60, len(mant) - 4), [127 - 60, 127 - 59, 127 + 59, 127]])
+    divisors = ((exps.astype(np.uint32) << 23) | mant.astype(np.uint32)).view(np.float32)
+    every = (np.arange(1 << 15, dtype=np.uint32) << 16).view(np.float32)
+    for b in divisors:
+        x = every[(every == 0) | ((every >= 2.0 ** -64) & (every <= 2.0 * b))]
+        x = np.concatenate([x, -x])
+        bb = np.full_like(x, b)
+        y = np.full_like(x, np.float32(1) / b)
+        q = x * y
+        got = _fma32(-_fma32(bb, q, -x), y, q)
+        zero = x == 0
+        assert (got[~zero].view(np.int32) == (x / bb)[~zero].view(np.int32)).all(), float(b)
