@@ -177,7 +177,9 @@ def _symmetric_product(A: torch.Tensor, out, alpha: float, beta: float, addend: 
     batch = A3.size(0)
     tile_class, mp, kp, nsplit, direct = _symmetric_plan(batch, M, K, addend)
     with torch.cuda.device(A.device):
-        prod = _cached(("sym_product", A.device, tile_class, batch, mp, kp, nsplit, direct),
+        # (an object of its own for each operator: a loop that calls both over one padded size would else find the
+        # other's descriptors at every call, and upload its own behind the launches still in flight)
+        prod = _cached(("ns_line_2" if addend else "ns_line_1", A.device, tile_class, batch, mp, kp, nsplit, direct),
                        lambda: _Product(A.device, tile_class, batch, mp, mp, kp, True, nsplit, direct),
                        _PRODUCT_CACHE, _PRODUCT_CACHE_MAX)
         with _exclusive(prod, A.device):
@@ -251,7 +253,7 @@ def ns_line_3(B: torch.Tensor, X: torch.Tensor, a: float, *, out: torch.Tensor =
     tile_class = _launch_class("update", tile_class, batch, M, N)
     mp, np_ = (_plan._round_up(s, _plan.pad_unit(tile_class)) for s in (M, N))
     with torch.cuda.device(X.device):
-        prod = _cached(("update_product", X.device, tile_class, batch, mp, np_),
+        prod = _cached(("ns_line_3", X.device, tile_class, batch, mp, np_),
                        lambda: _Product(X.device, tile_class, batch, mp, np_, mp, False),
                        _PRODUCT_CACHE, _PRODUCT_CACHE_MAX)
         with _exclusive(prod, X.device):

@@ -209,3 +209,20 @@ def test_ns_line_2_of_a_matrix_that_is_not_symmetric(M, shape):
     bound = 2.0 ** -8 * 1.001 * exact.abs() + 2.0 ** -13 * terms
     assert ((got.double() - exact).abs() <= bound).all()
     assert torch.equal(got[..., below], got.mT[..., below])
+
+
+def test_products_over_fixed_buffers_upload_their_descriptors_once(M, monkeypatch):
+    from muon_amd import engine
+    uploads = []
+    upload = engine._Staging.upload
+    monkeypatch.setattr(engine._Staging, "upload", lambda self, arr, into: (uploads.append(self), upload(self, arr, into))[1])
+    for shape in ((8, 192, 192), (4, 320, 320)):
+        uploads.clear()
+        X = _rand(shape, 0.05, 42).cuda()
+        A, B, C = (torch.empty(shape[0], shape[1], shape[1], dtype=torch.bfloat16, device="cuda") for _ in range(3))
+        for _ in range(4):
+            M.ns_line_1(X, out=A)
+            M.ns_line_2(A, C_, B_, out=B)
+            M.ns_line_3(B, X, A_, out=C)
+        assert len(uploads) == len(set(uploads)) == 3, shape
+        assert torch.equal(A, M.ns_line_1(X)) and torch.equal(C, M.ns_line_3(B, X, A_))

@@ -704,3 +704,29 @@ def test_short_division_is_the_ordinary_one_where_it_is_taken():
         got = _fma32(-_fma32(bb, q, -x), y, q)
         zero = x == 0
         assert (got[~zero].view(np.int32) == (x / bb)[~zero].view(np.int32)).all(), float(b)
+
+
+@pytest.mark.parametrize("shape", [(21, 320, 320), (4, 160, 192), (8, 192, 192), (1, 64, 64), (2, 300, 310)])
+def test_each_product_operator_keeps_an_object_of_its_own(shape, monkeypatch):
+    """ns_line_1 and ns_line_2 over the same padded sizes: with one cached object for both, a loop that calls them in
+    turn would upload its descriptors again at every call (and wait for the upload before)."""
+    import contextlib
+    from muon_amd import ops
+    keys = []
+
+    class Stop(Exception):
+        pass
+
+    def cached(key, make, *rest):
+        keys.append(key)
+        raise Stop
+
+    monkeypatch.setattr(ops, "_check_input", lambda t, name: None)
+    monkeypatch.setattr(ops, "_cached", cached)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    X = torch.zeros(*shape, dtype=torch.bfloat16)
+    A = torch.zeros(shape[0], shape[1], shape[1], dtype=torch.bfloat16)
+    for call in (lambda: muon_amd.ns_line_1(X), lambda: muon_amd.ns_line_2(A, 2.0, -4.0), lambda: muon_amd.ns_line_3(A, X, 3.0)):
+        with pytest.raises(Stop):
+            call()
+    assert len(set(keys)) == 3
