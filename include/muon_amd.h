@@ -41,7 +41,8 @@ extern "C" {
 #define MUON_AMD_GEMM_ROWSUM     4  /* muon_amd_ns_gemm only, for a mirrored product without addend
                                        (A = X X^T): also leave, per row of the result, partial sums
                                        of |A_ij| in MuonGemmDesc.rowsum (muon.py:779-781 fused into
-                                       the product's epilogue) */
+                                       the product's epilogue); tile classes 0 and 1 only, whose
+                                       wave tiles are as wide as a slot */
 #define MUON_AMD_GEMM_Q_KMAJOR   8  /* muon_amd_ns_gemm: every descriptor of the launch gives its second
                                        operand k-major (MuonGemmDesc.q_kmajor = 1); muon_amd_ns_gemm_apply
                                        always takes it that way */

@@ -496,6 +496,7 @@ struct GemmCfg {
     static constexpr int BM = BT_, BN = BT_, WGM = WGM_, WGN = WGN_, MINB = MINB_, NHALF = NHALF_;
     static constexpr int NW = WGM * WGN, NT = NW * 64;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
+    static constexpr bool ROW_SUMS = WN == 64;        // row sums go to slots of 64 columns, one per wave tile
     static constexpr int HALF_BYTES = BT_ * ROW_BYTES;
     static constexpr int DPH = BT_ / 8 / NW;          // DMA instructions (8 rows each) per wave per half
     static constexpr size_t RING_BYTES = static_cast<size_t>(NHALF) * HALF_BYTES;
@@ -988,12 +989,12 @@ constexpr int kNumTileClasses = 3;
 struct TileClass {
     int bm, bn, threads;
     size_t lds_bytes;
-    bool split_k;
+    bool split_k, row_sums;
 };
 static const TileClass kTileClasses[kNumTileClasses] = {
-    {Cfg0::BM, Cfg0::BN, Cfg0::NT, Cfg0::LDS_BYTES, Cfg0::SPLIT_K},
-    {Cfg1::BM, Cfg1::BN, Cfg1::NT, Cfg1::LDS_BYTES, Cfg1::SPLIT_K},
-    {Cfg2::BM, Cfg2::BN, Cfg2::NT, Cfg2::LDS_BYTES, Cfg2::SPLIT_K},
+    {Cfg0::BM, Cfg0::BN, Cfg0::NT, Cfg0::LDS_BYTES, Cfg0::SPLIT_K, Cfg0::ROW_SUMS},
+    {Cfg1::BM, Cfg1::BN, Cfg1::NT, Cfg1::LDS_BYTES, Cfg1::SPLIT_K, Cfg1::ROW_SUMS},
+    {Cfg2::BM, Cfg2::BN, Cfg2::NT, Cfg2::LDS_BYTES, Cfg2::SPLIT_K, Cfg2::ROW_SUMS},
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -1037,7 +1038,8 @@ template <typename Cfg>
 static int raise_lds_limits() {
     int rc = raise_lds_limit<Cfg, false, false, true, false>();
     if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, false, false, false>();
-    if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, false, false, true>();
+    if constexpr (Cfg::ROW_SUMS)
+        if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, false, false, true>();
     if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, true, true, false>();
     if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, false, true, false, false>();
     if (rc == MUON_AMD_OK) rc = raise_lds_limit<Cfg, true, true, true, false>();
@@ -1113,7 +1115,7 @@ static int launch_gemm(const DeviceState& st, const MuonGemmDesc* descs, const M
         if (round) go(ns_gemm_kernel<Cfg, false, true, true, false>);
         else go(ns_gemm_kernel<Cfg, false, true, false, false>);
     } else if (flags & MUON_AMD_GEMM_ROWSUM) {
-        go(ns_gemm_kernel<Cfg, false, false, false, true>);
+        if constexpr (Cfg::ROW_SUMS) go(ns_gemm_kernel<Cfg, false, false, false, true>);
     } else {
         if (round) go(ns_gemm_kernel<Cfg, false, false, true, false>);
         else go(ns_gemm_kernel<Cfg, false, false, false, false>);
@@ -1203,6 +1205,8 @@ int muon_amd_validate_gemm(const MuonGemmDesc* descs, int ndesc, const MuonTileJ
                                    (reinterpret_cast<uintptr_t>(d.rowsum) % 4) == 0),
                      "gemm desc %d: row sums need a mirrored product without addend and %d slots per row (ld_rowsum=%d)",
                      i, d.colsn / 64, d.ld_rowsum);
+        MUON_REQUIRE(!d.rowsum || kTileClasses[tile_class].row_sums,
+                     "gemm desc %d: tile class %d does not form row sums", i, tile_class);
     }
     for (int j = 0; j < njobs; ++j) {
         const MuonTileJob& t = jobs[j];
@@ -1246,8 +1250,10 @@ int muon_amd_ns_gemm(const MuonGemmDesc* descs_dev, const MuonTileJob* jobs_dev,
     MUON_REQUIRE(descs_dev && jobs_dev, "ns_gemm: null table");
     MUON_REQUIRE((split_partials_dev == nullptr) == (split_counters_dev == nullptr),
                  "ns_gemm: split partials and counters go together");
-    MUON_REQUIRE(njobs > 0, "ns_gemm: njobs=%d", njobs);
     MUON_REQUIRE(tile_class >= 0 && tile_class < kNumTileClasses, "ns_gemm: unknown tile class %d", tile_class);
+    MUON_REQUIRE(!(flags & MUON_AMD_GEMM_ROWSUM) || kTileClasses[tile_class].row_sums,
+                 "ns_gemm: tile class %d does not form row sums", tile_class);
+    MUON_REQUIRE(njobs > 0, "ns_gemm: njobs=%d", njobs);
     const DeviceState* st = nullptr;
     const int rc = device_setup(&st);
     if (rc != MUON_AMD_OK) return rc;
@@ -1277,8 +1283,10 @@ int muon_amd_ns_gemm_noalloc(const MuonGemmDesc* descs_dev, const MuonTileJob* j
                              int tile_class, float alpha, float beta, float gamma, int flags,
                              int split_slots, void* stream) {
     MUON_REQUIRE(descs_dev && jobs_dev, "ns_gemm_noalloc: null table");
-    MUON_REQUIRE(njobs > 0, "ns_gemm_noalloc: njobs=%d", njobs);
     MUON_REQUIRE(tile_class >= 0 && tile_class < kNumTileClasses, "ns_gemm_noalloc: unknown tile class %d", tile_class);
+    MUON_REQUIRE(!(flags & MUON_AMD_GEMM_ROWSUM) || kTileClasses[tile_class].row_sums,
+                 "ns_gemm_noalloc: tile class %d does not form row sums", tile_class);
+    MUON_REQUIRE(njobs > 0, "ns_gemm_noalloc: njobs=%d", njobs);
     MUON_REQUIRE(split_slots >= 0, "ns_gemm_noalloc: split_slots=%d", split_slots);
     MUON_REQUIRE(split_slots <= kStaticSplitSlots,
                  "ns_gemm_noalloc: the job list uses %d split slots, the static scratch holds %d "

@@ -89,7 +89,11 @@ class _ChunkRuntime:
                   "update": (_plan.PH_UPD_EVEN, _plan.PH_UPD_ODD, _plan.PH_UPD_LAST)}
         for kind, ln in chunk.launches.items():
             for ph in phases[kind]:
-                _lib.check(lib.muon_amd_validate_gemm(_lib.host_ptr(gemm[ph]), chunk.nmat, _lib.host_ptr(ln.jobs),
+                descs = gemm[ph]
+                if kind != "gram_rowsum":         # (the table of X X^T names the slots; only that launch fills them)
+                    descs = descs.copy()
+                    descs["rowsum"] = 0
+                _lib.check(lib.muon_amd_validate_gemm(_lib.host_ptr(descs), chunk.nmat, _lib.host_ptr(ln.jobs),
                                                       len(ln.jobs), ln.tile_class, ln.split_slots), "validate_gemm")
         self.mat_template = chunk.mat_descs(base)
         # one static device blob: gemm descs | block prefix | tile prefix | the job list of every kind of

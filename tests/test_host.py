@@ -730,3 +730,25 @@ def test_each_product_operator_keeps_an_object_of_its_own(shape, monkeypatch):
         with pytest.raises(Stop):
             call()
     assert len(set(keys)) == 3
+
+
+def test_row_sums_are_refused_in_the_64_class():
+    """The slots of a row are 64 columns wide, the wave tiles of that class 32: its epilogue would write twice the slots
+    that a row has, past the end of the buffer in the last row."""
+    lib = _lib.load()
+    d = np.zeros(1, dtype=_lib.GEMM_DESC)
+    d["P"] = d["Q"] = 1 << 20
+    d["C"] = d["CT"] = 1 << 24
+    d["ldp"] = d["ldq"] = d["ldc"] = d["ldct"] = d["K"] = d["rows"] = d["colsn"] = 256
+    d["rowsum"], d["ld_rowsum"] = 1 << 28, 4
+    for tile_class, ok in ((0, True), (1, True), (2, False)):
+        from muon_amd import ops
+        T = plan.TILE_DIMS[tile_class][0]
+        jobs = ops._product_jobs(tile_class, 1, 256, 256, 256, True)
+        assert jobs["i0"].max() == 256 - T
+        rc = lib.muon_amd_validate_gemm(_lib.host_ptr(d), 1, _lib.host_ptr(jobs), len(jobs), tile_class, 0)
+        assert (rc == 0) == ok, (tile_class, lib.muon_amd_last_error())
+    for launch in (lambda flags: lib.muon_amd_ns_gemm(1 << 20, 1 << 20, 0, 2, 1.0, 0.0, 0.0, flags, None, None, None),
+                   lambda flags: lib.muon_amd_ns_gemm_noalloc(1 << 20, 1 << 20, 0, 2, 1.0, 0.0, 0.0, flags, 0, None)):
+        assert launch(0) == -1 and b"njobs=0" in lib.muon_amd_last_error()      # (no jobs: never a launch)
+        assert launch(_lib.GEMM_ROWSUM) == -1 and b"row sums" in lib.muon_amd_last_error()
