@@ -51,3 +51,29 @@ def test_fused_parameter_step_in_small_tiles_gives_the_bits_of_large_ones(monkey
             opt.step()
         results.append([p.detach().clone() for p in ps])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("rescale", ["symmetric", "rows"])
+@pytest.mark.parametrize("shape", [(1, 40, 65), (3, 65, 129), (1, 128, 320), (2, 250, 250), (2, 600, 130), (1, 1027, 1100), (1, 1100, 1500)])
+def test_tile_classes_mixed_in_the_aol_variant(shape, rescale, monkeypatch):
+    """Its first X X^T, which leaves the row sums, keeps the matrix's own class while the others take smaller tiles, over
+    buffers whose padding holds NaNs (nothing of it may reach a result)."""
+    import muon_amd
+    from muon_amd import plan
+    torch.manual_seed(sum(shape))
+    G = torch.randn(*shape, device="cuda")
+    outs = []
+    for forced in ("1,1,1", "0,0,0", "2,2,2", "2,0,2", "0,2,0"):
+        monkeypatch.setattr(plan, "LAUNCH_CLASS", forced)
+        muon_amd.clear_engine_cache()
+        muon_amd.zeropower_via_aol4(G, rescale=rescale)
+        eng = next(iter(muon_amd.functional._ENGINE_CACHE.values()))
+        assert eng.chunks[0].launches["gram_rowsum"].tile_class == eng.chunks[0].tile_class
+        assert forced != "2,2,2" or {eng.chunks[0].launches[k].tile_class for k in ("gram", "poly", "update")} == {2}
+        for ws in eng.workspaces:
+            ws.fill_(0xff)
+        outs.append(muon_amd.zeropower_via_aol4(G, rescale=rescale))
+    muon_amd.clear_engine_cache()
+    assert torch.isfinite(outs[0].float()).all()
+    for other in outs[1:]:
+        assert torch.equal(outs[0], other)
