@@ -31,8 +31,7 @@ def _cached(key, make, cache=None, limit=_ENGINE_CACHE_MAX):
         if eng is None:
             eng = make()
             eng._fn_lock = threading.Lock()       # one caller at a time enqueues on this engine
-            eng._fn_done = None                   # event after the launches of its last call ...
-            eng._fn_stream = None                 # ... and the stream it was recorded on
+            eng._fn_done = None                   # event after the launches of its last call
             cache[key] = eng
             while len(cache) > limit:
                 cache.popitem(last=False)
@@ -51,14 +50,15 @@ def _exclusive(eng, device):
     with eng._fn_lock:
         stream = torch.cuda.current_stream(device)
         capturing = torch.cuda.is_current_stream_capturing()
-        if eng._fn_done is not None and not capturing and eng._fn_stream != stream.cuda_stream:
+        # (always: equal handles need not be one stream -- the per-thread default streams of two threads, a new stream
+        # in the place of a destroyed one -- and the wait costs a call on the same stream about a microsecond)
+        if eng._fn_done is not None and not capturing:
             stream.wait_event(eng._fn_done)
         yield
         if not capturing:
             if eng._fn_done is None:
                 eng._fn_done = torch.cuda.Event()
             eng._fn_done.record(stream)           # (a wait already enqueued stays on the record it saw)
-            eng._fn_stream = stream.cuda_stream
 
 
 def clear_engine_cache() -> None:

@@ -752,3 +752,32 @@ def test_row_sums_are_refused_in_the_64_class():
                    lambda flags: lib.muon_amd_ns_gemm_noalloc(1 << 20, 1 << 20, 0, 2, 1.0, 0.0, 0.0, flags, 0, None)):
         assert launch(0) == -1 and b"njobs=0" in lib.muon_amd_last_error()      # (no jobs: never a launch)
         assert launch(_lib.GEMM_ROWSUM) == -1 and b"row sums" in lib.muon_amd_last_error()
+
+
+def test_calls_on_one_engine_are_ordered_whatever_handle_their_stream_has(monkeypatch):
+    """Two streams may show the same handle (the per-thread default streams of two threads, a new stream in the place
+    of a destroyed one): every call waits for the launches of the call before it."""
+    from types import SimpleNamespace
+    from muon_amd import functional
+    waits, records = [], []
+
+    class Event:
+        def record(self, stream):
+            records.append((self, stream))
+
+    class Stream:
+        cuda_stream = 2
+
+        def wait_event(self, event):
+            waits.append((event, self))
+
+    streams = [Stream(), Stream()]
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    eng = functional._cached(("a test",), SimpleNamespace, cache=functional.OrderedDict())
+    for s in streams:
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device, s=s: s)
+        with functional._exclusive(eng, "cuda:0"):
+            pass
+    assert [s for _, s in records] == streams
+    assert [(e, s) for e, s in waits] == [(records[0][0], streams[1])]
