@@ -341,8 +341,8 @@ int muon_amd_run_chunk(const MuonChunkRun* run, float one_minus_beta, float beta
 int muon_amd_small_class(int rows, int cols);
 int muon_amd_validate_small(const MuonMatDesc* descs_host, int nmat, int small_class, int max_long_side);
 /* Momentum, norm, normalise, `steps` iterations with the coefficients coeffs = {a, b, c} (host memory) and
- * the parameter step for nmat matrices of small_class at most whose long sides are at most
- * max_long_side, one workgroup each; of a descriptor grad, momentum, param, out, rows, cols, src_dtype
+ * the parameter step for nmat matrices of small_class at most (0: of any class, each in its own) whose long
+ * sides are at most max_long_side, one workgroup each; of a descriptor grad, momentum, param, out, rows, cols, src_dtype
  * and scale are used.  Same bits as the launches of muon_amd_run_chunk.                       */
 int muon_amd_small_step(const MuonMatDesc* descs_dev, int nmat, int small_class, int max_long_side, int steps,
                         const float* coeffs, int flags, float one_minus_beta, float beta, int nesterov, int mutate_grad,

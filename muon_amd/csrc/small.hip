@@ -357,27 +357,18 @@ __device__ __forceinline__ void small_apply(const MuonMatDesc& d, const char* X,
     }
 }
 
-// One workgroup per matrix.  MP: its short side rounded up to 32, 64 or 128; the long side is rounded up to
+// One matrix by one workgroup.  MP: its short side rounded up to 32, 64 or 128; the long side is rounded up to
 // 64 (a k-block of the general path).  The products are shared out by 32 x 32 tiles of the Gram matrix and
 // by blocks of 32 columns of X; X' overwrites X, whose columns depend on nothing but themselves and B.
 template <int MP, bool ROUND>
-__global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
-    const MuonMatDesc* __restrict__ descs, int steps, float ca, float cb, float cc, float w, float beta, int nesterov,
-    int mutate_grad, float eps, float neg_lr, float wd_factor, const float* __restrict__ sc) {
+__device__ __forceinline__ void small_matrix(char* lds, const MuonMatDesc& d, int steps, float ca, float cb, float cc, float w, float beta,
+                                             int nesterov, int mutate_grad, float eps, float neg_lr, float wd_factor) {
     constexpr int MT = MP / 32, TILES = MT * MT, TPW = (TILES + SMALL_WAVES - 1) / SMALL_WAVES;
     constexpr int SYM_TILES = MT * (MT + 1) / 2, SPW = (SYM_TILES + SMALL_WAVES - 1) / SMALL_WAVES;
     constexpr bool KEEP_B = MP <= 64;                // (of the 128 registers a thread can have at 16 waves)
     constexpr int PA = small_pitch(MP);
-    extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int lane = tid & 63;
-    if (sc) {   // {1 - beta, beta, lr, wd_factor} read at run time instead of the arguments
-        w = sc[0];
-        beta = sc[1];
-        neg_lr = -sc[2];
-        wd_factor = sc[3];
-    }
-    const MuonMatDesc d = descs[blockIdx.x];
     const bool wide = d.rows <= d.cols;
     const int m = wide ? d.rows : d.cols, n = wide ? d.cols : d.rows;
     const int np = (n + 63) & ~63, px = small_pitch(np);
@@ -511,6 +502,33 @@ __global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
     else small_apply<float>(d, X, px, wide, neg_lr, wd_factor, tid);
 }
 
+// One workgroup per matrix, all of class MP at most, or (MP = 0) each in its own class: a launch per class takes at least
+// what its longest matrix takes, one after the other, and the largest class for all of them pads the others.  32 x 2400,
+// 16 of 64 x 64 and 4 of 128 x 300: 67 us, 136 in a launch per class, 100 on the general path; 2000 of 20 x 30 and one of
+// 128 x 300: 100 us, 213 in class 128, 247 on the general path.  A class of its own is 1 to 6 % faster over many
+// matrices than this kernel (1000 of 128 x 128: 149 against 159 us), so both are here.
+template <int MP, bool ROUND>
+__global__ __launch_bounds__(SMALL_THREADS) void ns_small_kernel(
+    const MuonMatDesc* __restrict__ descs, int steps, float ca, float cb, float cc, float w, float beta, int nesterov,
+    int mutate_grad, float eps, float neg_lr, float wd_factor, const float* __restrict__ sc) {
+    extern __shared__ __align__(16) char lds[];
+    if (sc) {   // {1 - beta, beta, lr, wd_factor} read at run time instead of the arguments
+        w = sc[0];
+        beta = sc[1];
+        neg_lr = -sc[2];
+        wd_factor = sc[3];
+    }
+    const MuonMatDesc d = descs[blockIdx.x];
+    if constexpr (MP != 0) {
+        small_matrix<MP, ROUND>(lds, d, steps, ca, cb, cc, w, beta, nesterov, mutate_grad, eps, neg_lr, wd_factor);
+    } else {
+        const int m = d.rows < d.cols ? d.rows : d.cols;
+        if (m <= 32) small_matrix<32, ROUND>(lds, d, steps, ca, cb, cc, w, beta, nesterov, mutate_grad, eps, neg_lr, wd_factor);
+        else if (m <= 64) small_matrix<64, ROUND>(lds, d, steps, ca, cb, cc, w, beta, nesterov, mutate_grad, eps, neg_lr, wd_factor);
+        else small_matrix<128, ROUND>(lds, d, steps, ca, cb, cc, w, beta, nesterov, mutate_grad, eps, neg_lr, wd_factor);
+    }
+}
+
 template <int MP, bool ROUND>
 static int raise_small_limit() {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(ns_small_kernel<MP, ROUND>), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -523,7 +541,9 @@ static int raise_small_limit() {
 }
 
 int raise_small_limits() {
-    int rc = raise_small_limit<32, true>();
+    int rc = raise_small_limit<0, true>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<0, false>();
+    if (rc == MUON_AMD_OK) rc = raise_small_limit<32, true>();
     if (rc == MUON_AMD_OK) rc = raise_small_limit<32, false>();
     if (rc == MUON_AMD_OK) rc = raise_small_limit<64, true>();
     if (rc == MUON_AMD_OK) rc = raise_small_limit<64, false>();
@@ -552,7 +572,7 @@ int muon_amd_validate_small(const MuonMatDesc* descs, int nmat, int small_class,
     for (int i = 0; i < nmat; ++i) {
         const MuonMatDesc& d = descs[i];
         const int own = muon_amd_small_class(d.rows, d.cols);
-        MUON_REQUIRE(own && own <= small_class && (d.rows > d.cols ? d.rows : d.cols) <= max_long_side,
+        MUON_REQUIRE(own && (own <= small_class || small_class == 0) && (d.rows > d.cols ? d.rows : d.cols) <= max_long_side,
                      "mat %d: %d x %d does not fit class %d with a long side of %d", i, d.rows, d.cols, small_class, max_long_side);
         MUON_REQUIRE(d.grad && (d.param || d.out), "mat %d: null source or neither param nor out given", i);
         MUON_REQUIRE(d.src_dtype == MUON_AMD_SRC_F32 || d.src_dtype == MUON_AMD_SRC_BF16, "mat %d: src_dtype=%d", i, d.src_dtype);
@@ -565,9 +585,10 @@ int muon_amd_small_step(const MuonMatDesc* descs_dev, int nmat, int small_class,
                         float eps, float lr, float wd_factor, const float* scalars_dev, void* stream) {
     MUON_REQUIRE(descs_dev && coeffs, "small_step: null table");
     MUON_REQUIRE(nmat > 0 && steps >= 0, "small_step: nmat=%d steps=%d", nmat, steps);
-    MUON_REQUIRE(small_class == 32 || small_class == 64 || small_class == 128, "small_step: class %d", small_class);
+    MUON_REQUIRE(small_class == 0 || small_class == 32 || small_class == 64 || small_class == 128, "small_step: class %d", small_class);
     MUON_REQUIRE(max_long_side > 0 && max_long_side <= 65536, "small_step: long side %d", max_long_side);
-    const size_t bytes = small_lds_bytes(small_class, (max_long_side + 63) & ~63);
+    // (classes mixed: as much as any matrix can need; a CU holds one workgroup of 16 waves in any case)
+    const size_t bytes = small_class ? small_lds_bytes(small_class, (max_long_side + 63) & ~63) : SMALL_LDS_MAX;
     MUON_REQUIRE(bytes <= SMALL_LDS_MAX, "small_step: a long side of %d does not fit", max_long_side);
     const int rc = muon_amd_init();
     if (rc != MUON_AMD_OK) return rc;
@@ -577,7 +598,8 @@ int muon_amd_small_step(const MuonMatDesc* descs_dev, int nmat, int small_class,
                            scalars_dev);
     };
     const bool round = (flags & MUON_AMD_ROUND_REFERENCE) != 0;
-    if (small_class == 32) round ? go(ns_small_kernel<32, true>) : go(ns_small_kernel<32, false>);
+    if (small_class == 0) round ? go(ns_small_kernel<0, true>) : go(ns_small_kernel<0, false>);
+    else if (small_class == 32) round ? go(ns_small_kernel<32, true>) : go(ns_small_kernel<32, false>);
     else if (small_class == 64) round ? go(ns_small_kernel<64, true>) : go(ns_small_kernel<64, false>);
     else round ? go(ns_small_kernel<128, true>) : go(ns_small_kernel<128, false>);
     return check_launch("small_step");

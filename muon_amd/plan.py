@@ -640,18 +640,16 @@ SMALL = os.environ.get("MUON_AMD_SMALL", "1") != "0"      # measurement knob: sm
 def small_groups(shapes, variant: str = "ns5"):
     """-> [(class, positions in `shapes`)] when every matrix of the group fits one workgroup (its whole step
     is then one launch, see small.hip), else None: beside larger matrices the small ones ride in the
-    grouped launches, where a launch of their own would only add its time (bits are the same).  One
-    launch covers all of them in the largest class any of them needs if they all fit it."""
+    grouped launches, where a launch of their own would only add its time (bits are the same).  Class 0 stands for
+    matrices of several classes, each of which runs in its own; what takes longest comes first."""
     if not SMALL or variant != "ns5" or not shapes:
         return None
     lib = _lib.load()
     own = [lib.muon_amd_small_class(r, c) for r, c in shapes]
     if not all(own):
         return None
-    top, longest = max(own), max(max(sh) for sh in shapes)
-    if lib.muon_amd_small_class(top, max(longest, top)) == top:
-        return [(top, list(range(len(shapes))))]
-    return [(c, [i for i, k in enumerate(own) if k == c]) for c in sorted(set(own))]
+    order = sorted(range(len(shapes)), key=lambda i: (-own[i], -max(shapes[i])))
+    return [(own[0] if len(set(own)) == 1 else 0, order)]
 
 
 LANES = os.environ.get("MUON_AMD_LANES", "auto")        # "auto", or a number of lanes to force ("1" switches them off)

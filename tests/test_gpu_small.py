@@ -96,3 +96,25 @@ def test_small_step_gives_the_signs_of_zeros_of_the_general_path(rounding, steps
     muon_amd.clear_engine_cache()
     assert (got[1] == -0x8000).any() and (got[1] == 0).any()
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("rounding", ["reference", "fused"])
+def test_classes_mixed_in_one_launch_give_the_bits_of_the_general_path(rounding, monkeypatch):
+    """Every shape of the list beside the others, the largest of each class among them, in two storage types."""
+    import muon_amd
+    from muon_amd import plan
+    for dtype in (torch.float32, torch.bfloat16):
+        finals = []
+        for small in (True, False):
+            monkeypatch.setattr(plan, "SMALL", small)
+            torch.manual_seed(8)
+            ps = [torch.nn.Parameter(torch.randn(s, device="cuda").to(dtype)) for s in SHAPES + [(32, 2432), (64, 1088)]]
+            opt = muon_amd.SingleDeviceMuon(ps, weight_decay=0.1, ns_rounding=rounding)
+            for _ in range(2):
+                for p in ps:
+                    p.grad = torch.randn(p.shape, device="cuda").to(dtype)
+                opt.step()
+            eng = next(iter(opt._muon_engines.values()))
+            assert [rt.small_class for rt in eng.small] == ([0] if small else [])
+            finals.append([p.detach().clone() for p in ps] + [opt.state[p]["momentum_buffer"].clone() for p in ps])
+        assert all(torch.equal(a, b) for a, b in zip(*finals))

@@ -781,3 +781,22 @@ def test_calls_on_one_engine_are_ordered_whatever_handle_their_stream_has(monkey
             pass
     assert [s for _, s in records] == streams
     assert [(e, s) for e, s in waits] == [(records[0][0], streams[1])]
+
+
+def test_small_matrices_of_several_classes_take_one_launch():
+    """A launch per class took longer than the grouped launches (each waits for its longest matrix)."""
+    lib = _lib.load()
+    shapes = [(64, 64)] * 16 + [(32, 2400)] + [(300, 128)] * 4 + [(5, 3)]
+    groups = plan.small_groups(shapes)
+    assert len(groups) == 1 and groups[0][0] == 0 and sorted(groups[0][1]) == list(range(len(shapes)))
+    assert [shapes[i] for i in groups[0][1][:4]] == [(300, 128)] * 4
+    assert plan.small_groups([(64, 70)] * 3)[0][0] == 64 and plan.small_groups([(20, 2000)])[0][0] == 32
+    d = np.zeros(len(shapes), dtype=_lib.MAT_DESC)
+    d["rows"], d["cols"] = np.array(shapes, dtype=np.int32).T
+    d["grad"] = d["out"] = 1 << 20
+    assert lib.muon_amd_validate_small(_lib.host_ptr(d), len(d), 0, 2400) == 0
+    assert lib.muon_amd_validate_small(_lib.host_ptr(d), len(d), 0, 2399) == -1
+    assert lib.muon_amd_validate_small(_lib.host_ptr(d), len(d), 128, 2400) == 0      # (refused where it is launched: no LDS for it)
+    for rows, cols in ((129, 129), (128, 321), (64, 1089), (32, 2433)):
+        d["rows"][0], d["cols"][0] = rows, cols
+        assert lib.muon_amd_validate_small(_lib.host_ptr(d), len(d), 0, 4096) == -1, (rows, cols)
