@@ -106,9 +106,8 @@ def check_fragment_waits(asm_text: str) -> int:
 def check_store_data(asm_text: str) -> int:
     """No vector instruction may overwrite a data register of a buffer, global or flat store of more than 8 bytes
     within two wait states of it: the store still reads that register for its last lanes.  The compiler
-    leaves out those wait states after a buffer store with a scalar offset.  Raises if the listing
-    holds such a pair; returns the number of
-    stores looked at."""
+    leaves out those wait states after a buffer store with a scalar offset.  A vector instruction writes its first
+    operand, a swap both.  Raises if the listing holds such a pair; returns the number of stores looked at."""
     code = [t for t in (l.split(";")[0].strip() for l in asm_text.split("\n")) if t and not t.startswith(".") and not t.endswith(":")]
     nstores = 0
     for i, t in enumerate(code):
@@ -122,7 +121,8 @@ def check_store_data(asm_text: str) -> int:
             if states >= 2 or u.startswith("s_endpgm"):
                 break
             op, _, args = u.partition(" ")
-            if op.startswith("v_") and _vregs(args.split(",")[0]) & data:
+            written = args if re.match(r"v_(permlane\d+_)?swap", op) else args.split(",")[0]
+            if op.startswith("v_") and _vregs(written) & data:
                 raise RuntimeError(f"ns_gemm.hip: '{u}' overwrites the data of '{t}' while it is read")
             states += int(args) + 1 if op == "s_nop" else 1
     return nstores

@@ -800,3 +800,15 @@ def test_small_matrices_of_several_classes_take_one_launch():
     for rows, cols in ((129, 129), (128, 321), (64, 1089), (32, 2433)):
         d["rows"][0], d["cols"][0] = rows, cols
         assert lib.muon_amd_validate_small(_lib.host_ptr(d), len(d), 0, 4096) == -1, (rows, cols)
+
+
+def test_build_refuses_store_data_swapped_behind_the_store():
+    """A swap writes both of its operands."""
+    from muon_amd.build import check_store_data
+    store = "\tbuffer_store_dwordx4 v[170:173], v164, s[28:31], s26 offen\n"
+    for swap in ("v_permlane32_swap_b32_e32", "v_permlane16_swap_b32_e64", "v_swap_b32"):
+        for args in ("v9, v171", "v171, v9"):
+            with pytest.raises(RuntimeError, match="overwrites the data"):
+                check_store_data(f"{store}\t{swap} {args}\n")
+        assert check_store_data(f"{store}\ts_nop 1\n\t{swap} v9, v171\n") == 1
+        assert check_store_data(f"{store}\t{swap} v9, v174\n") == 1
