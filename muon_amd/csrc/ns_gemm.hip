@@ -47,11 +47,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// Accesses through the global (not flat) address space: pointers fetched from a descriptor are
-// generic to the compiler, and a flat access would also count against the LDS wait counter.
-__device__ __forceinline__ u32x2 gload8(const uint16_t* p) {
-    return *(const __attribute__((address_space(1))) u32x2*)(p);
-}
 // STREAM: non-temporal hint.  The outputs of the large tile class are hundreds of megabytes that
 // the next launch reads long after this XCD's L2 has turned over; keeping them out of the way of
 // the operand panels measured +0.5 % on the Llama step (and a loss for GPT-2-size matrices, whose
@@ -492,7 +487,7 @@ __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const 
 template <int BT_, int WGM_, int WGN_, int MINB_, int NHALF_, bool SPLIT_K_>
 struct GemmCfg {
     static constexpr bool SPLIT_K = SPLIT_K_;     // jobs may share a tile's reduction
-    static constexpr bool STREAM_STORES = BT_ >= 256;   // see gstore16
+    static constexpr bool STREAM_STORES = BT_ >= 256;   // see bstore16
     static constexpr int BM = BT_, BN = BT_, WGM = WGM_, WGN = WGN_, MINB = MINB_, NHALF = NHALF_;
     static constexpr int NW = WGM * WGN, NT = NW * 64;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
