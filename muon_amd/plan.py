@@ -1,8 +1,9 @@
 """Host-side planning of the grouped Newton-Schulz launches (pure numpy; no GPU needed).
 
 A *chunk* is a set of matrices that runs through the whole Muon step together: one momentum
-launch, one norm launch, one normalise launch, 3 GEMM launches per Newton-Schulz iteration and
-one apply launch, however many matrices it holds.  Chunks exist only to bound the bf16
+launch, one normalise launch (which forms the norms too where the chunk is small; else a norm launch
+before it) and 3 GEMM launches per Newton-Schulz iteration, the last of which takes the parameter
+step, however many matrices it holds.  Chunks exist only to bound the bf16
 workspace; they share one workspace and run back to back on the stream.
 
 Per matrix (m = min(rows, cols), n = max(rows, cols), padded to the chunk's GEMM tile) the
@@ -233,9 +234,20 @@ def xcd_permutation(njobs: int, group: int = 32) -> np.ndarray:
     return perm
 
 
-# Cost of a job in k-blocks for balancing a launch: its reduction plus what its prologue and
-# epilogue cost in the same unit (measured: about 8 us against 0.65 us per k-block for the
-# 128 x 128 class, 12 us against 1.6 us for the 256 x 256 class).
+# Time of a launch by tile class, in microseconds, measured with isolated launches of one class over the same
+# matrices (shapes from 64 x 576 to 4096 x 14336, 1 to 256 of them):
+#   a job alone on its CU      fixed + k-blocks * alone
+#   jobs in turn on a CU       k-blocks * shared + fixed_shared each (their epilogues overlap the neighbour's loop)
+# e.g. 1100 x 1500, X X^T / polynomial / update: 256 x 256 tiles 35 / 27 / 28 us (15 and 30 jobs), 128 x 128
+# tiles 14.5 / 11.8 / 14.4, 64 x 64 tiles 8.3 / 6.8 / 9.9; 768 x 3072: 128 x 128 22 / 9.4 / 11, 64 x 64 12 / 5.6 / 11;
+# 48 x (768 x 3072), where the larger tiles fill the GPU: X X^T 133 us in 128 x 128 tiles, 182 in 64 x 64.
+LAUNCH_COST = {1: dict(fixed=9.5, alone=0.98, shared=1.3, fixed_shared=13.0, base=0.0),
+               0: dict(fixed=5.1, alone=0.36, shared=0.5, fixed_shared=2.2, base=3.0),
+               2: dict(fixed=3.4, alone=0.183, shared=0.235, fixed_shared=0.8, base=2.8)}
+# A job's fixed cost in k-blocks of its class, for balancing the jobs of a launch over the CUs (launch_imbalance).  More than
+# what LAUNCH_COST gives (fixed_shared / shared: 4.4, 10 and 3.4 in classes 0, 1, 2): of 640 plans those figures change only
+# the order of the update jobs of some convolutional networks, base width 106 and 108 993 -> 1005 and 997 -> 1007 us, 114
+# 1150 -> 1141, the others the same.
 JOB_FIXED_KBLOCKS = {0: 12, 1: 8, 2: 12}
 WORKGROUPS_PER_CU = {0: 2, 1: 1, 2: 2}  # must match the kernels' launch bounds
 N_CU = 256
@@ -303,18 +315,6 @@ class Launch:
 NORM_IN_NORMALIZE_BLOCKS = (512, 4096)
 
 LAUNCH_CLASS = os.environ.get("MUON_AMD_LAUNCH_CLASS", "auto")      # measurement knob: "gram,poly,update" classes
-
-
-# Time of a launch by tile class, in microseconds, measured with isolated launches of one class over the same
-# matrices (shapes from 64 x 576 to 4096 x 14336, 1 to 256 of them):
-#   a job alone on its CU      fixed + k-blocks * alone
-#   jobs in turn on a CU       k-blocks * shared + fixed_shared each (their epilogues overlap the neighbour's loop)
-# e.g. 1100 x 1500, X X^T / polynomial / update: 256 x 256 tiles 35 / 27 / 28 us (15 and 30 jobs), 128 x 128
-# tiles 14.5 / 11.8 / 14.4, 64 x 64 tiles 8.3 / 6.8 / 9.9; 768 x 3072: 128 x 128 22 / 9.4 / 11, 64 x 64 12 / 5.6 / 11;
-# 48 x (768 x 3072), where the larger tiles fill the GPU: X X^T 133 us in 128 x 128 tiles, 182 in 64 x 64.
-LAUNCH_COST = {1: dict(fixed=9.5, alone=0.98, shared=1.3, fixed_shared=13.0, base=0.0),
-               0: dict(fixed=5.1, alone=0.36, shared=0.5, fixed_shared=2.2, base=3.0),
-               2: dict(fixed=3.4, alone=0.183, shared=0.235, fixed_shared=0.8, base=2.8)}
 
 
 # ... and what a job of a split reduction adds (it parks its accumulators, and the last one of a tile adds
@@ -731,16 +731,18 @@ def plan_chunks(shapes, steps: int, reference_rounding: bool, workspace_cap: int
 
 
 TAIL_AWARE_CHUNKS = os.environ.get("MUON_AMD_TAIL_AWARE_CHUNKS", "1") != "0"      # measurement knob
-KBLOCK_US = {0: 0.645, 1: 1.58}         # a CU's time per k-block of its tiles (two co-resident 128 x 128 tiles share it)
 CHUNK_FIXED_US = 200.0                  # what one more chunk costs: 18 more launches that fill and drain the GPU
 
 
 def _chunk_time_us(mats, tile_class: int) -> tuple[float, float]:
     """(estimated, ideal) time of the fifteen GEMM launches of one iteration-set of a chunk holding
     `mats` [(rows, cols)], from the busiest CU of every launch (jobs in list order, job j on
-    workgroup j % grid; see launch_imbalance).  The ideal has every CU equally busy."""
+    workgroup j % grid; see launch_imbalance).  The ideal has every CU equally busy.  In the tiles of the
+    chunk's own class: launches that would take smaller ones leave CUs idle, and a chunk is cut only where
+    a workspace is full."""
     unit = pad_unit(tile_class)
     dims = [(_round_up(min(r, c), unit), _round_up(max(r, c), unit)) for r, c in mats]
+    kblocks = [(-(-min(r, c) // GEMM_BK), -(-max(r, c) // GEMM_BK)) for r, c in mats]
     big = (tile_class == 1 or
            (UPDATE_CLASS != "0" and all(mp % 256 == 0 and np_ % 256 == 0 for mp, np_ in dims) and
             (UPDATE_CLASS == "1" or sum((mp // 256) * (np_ // 256) for mp, np_ in dims) >= RESIDENT_BIG_TILE_WORKGROUPS)))
@@ -750,19 +752,19 @@ def _chunk_time_us(mats, tile_class: int) -> tuple[float, float]:
         tc = (1 if big else 0) if kind == "update" else tile_class
         TT = TILE_DIMS[tc][0] if kind == "update" else T
         counts, costs = [], []
-        for mp, np_ in dims:
+        for (mp, np_), (kbm, kbn) in zip(dims, kblocks):
             mt = mp // TT
             if kind == "update":
-                counts.append(mt * (np_ // TT)); costs.append(mp // GEMM_BK)
+                counts.append(mt * (np_ // TT)); costs.append(kbm)
             else:
-                kb = (np_ if kind == "syrk" else mp) // GEMM_BK
                 ns = split_factor(mp, np_) if kind == "syrk" else 1
-                counts.append(mt * (mt + 1) // 2 * ns); costs.append(kb // ns)
-        cost = np.repeat(np.asarray(costs, dtype=np.float64) + JOB_FIXED_KBLOCKS[tc], counts)
+                counts.append(mt * (mt + 1) // 2 * ns); costs.append((kbn if kind == "syrk" else kbm) // ns)
+        us = LAUNCH_COST[tc]
+        cost = np.repeat(np.asarray(costs, dtype=np.float64) * us["shared"] + us["fixed_shared"], counts)
         grid = min(len(cost), N_CU * WORKGROUPS_PER_CU[tc])
         cu = np.bincount((np.arange(len(cost)) % grid) % N_CU, weights=cost, minlength=N_CU)
-        est += cu.max() * KBLOCK_US[tc]
-        ideal += cost.sum() / N_CU * KBLOCK_US[tc]
+        est += cu.max()
+        ideal += cost.sum() / N_CU
     return est, ideal
 
 
