@@ -309,9 +309,13 @@ class Launch:
 
 
 # The normalise launch forms the norms itself (every wave adds up its matrix's partial sums, one per 8192 elements)
-# where no matrix has more than the first number of them and the chunk no more than the second.  One 1500 x 1100
-# Newton-Schulz 163.0 -> 160.9 us, ConvNet step (3300 sums) 355.8 -> 351.3, one 768 x 3072 step 174.9 -> 173.9; GPT-2-124M
-# (5200 in each lane) 2.054 -> 2.062 ms: with many tiles in a launch the reads cost what the launch saved.
+# where no matrix has more than the first number of them and the chunk no more than the second.  That saves a launch and
+# costs every wave the reads.  A step with the norms in a launch of their own -> in the normalise launch, in us, by sums:
+#   768 x 3072 (288) 179.2 -> 176.5, 1500 x 1100 (202) 160.1 -> 157.0, 2500 x 2600 (794) 515.3 -> 511.9, 12 layers of
+#   width 256 (1152) 232.7 -> 230.5, 8 of 512 (3072) 508.8 -> 508.3, 2 of 1024 (3072) 785.9 -> 785.7;
+#   one matrix of 2048, 2198, 4000: 1477.9 -> 1476.5, 1407.2 -> 1412.1, 2372.0 -> 2371.4 (nothing beyond noise);
+#   5 layers of 768 (4320) 945.1 -> 941.4, 3 of 1024 (4608) 1095.0 -> 1098.1, 8 of 640 (4800) 849.8 -> 852.1, 2 of 1280 (4800)
+#   1301.5 -> 1312.0, 4 of 1024 (6144) 1304.9 -> 1318.8, 12 of 640 (7200) 1386.8 -> 1396.3, 4096 x 14336 (7168) 3898 -> 3974.
 NORM_IN_NORMALIZE_BLOCKS = (512, 4096)
 
 LAUNCH_CLASS = os.environ.get("MUON_AMD_LAUNCH_CLASS", "auto")      # measurement knob: "gram,poly,update" classes
