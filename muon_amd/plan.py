@@ -645,7 +645,11 @@ def small_groups(shapes, variant: str = "ns5"):
     """-> [(class, positions in `shapes`)] when every matrix of the group fits one workgroup (its whole step
     is then one launch, see small.hip), else None: beside larger matrices the small ones ride in the
     grouped launches, where a launch of their own would only add its time (bits are the same).  Class 0 stands for
-    matrices of several classes, each of which runs in its own; what takes longest comes first."""
+    matrices of several classes, each of which runs in its own; what takes longest comes first.
+
+    However many there are: Newton-Schulz in the grouped launches -> in one workgroup each, in us: 128 x 320, 1 of them
+    73.9 -> 53.8, 64 98.3 -> 55.9, 300 244 -> 116, 4000 2408 -> 968; 64 x 1088, 1 75.5 -> 60.9, 600 521 -> 197; 128 x 128, 2000
+    727 -> 453; 64 x 64, 1 73.1 -> 24.1, 1000 293 -> 247, 4000 929 -> 867; 20 x 30, 4000 909 -> 858 (the host's part of a call there)."""
     if not SMALL or variant != "ns5" or not shapes:
         return None
     lib = _lib.load()
