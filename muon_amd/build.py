@@ -25,6 +25,8 @@ FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     # hipcc -O3 must not form packed-fp32 instructions on this target
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first kernel arguments arrive in scalar registers with the dispatch instead of through a load of each wave's own
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 
