@@ -120,6 +120,10 @@ typedef struct MuonGemmDesc {
     int32_t q_kmajor;                   /* 0: Q is colsn x K, rows along k; 1: Q is K x colsn   */
 } MuonGemmDesc;
 
+#define MUON_AMD_TILE_ROWS_EMPTY 1   /* the second half of the tile's rows    */
+#define MUON_AMD_TILE_COLS_EMPTY 2   /* the second half of the tile's columns */
+#define MUON_AMD_TILE_EMPTY      3
+
 /* One output tile of one matrix, or one share of its reduction.  A tile whose K is long and
  * whose launch would leave most of the GPU idle (the one 128 x 128 tile of X X^T for a
  * 128 x 16384 matrix) is given to `count` jobs, each reducing k0..k1; each parks its fp32
@@ -134,7 +138,9 @@ typedef struct MuonTileJob {
                           the tile of its mirror image); 0 otherwise                           */
     int32_t k0, k1;    /* reduction range of this job, multiples of 64; 0 and K when unsplit */
     int32_t part_base; /* first slot of the tile's split group (also its counter); unused when unsplit */
-    int32_t split;     /* 0 when unsplit, else index | (count << 16) */
+    int32_t split;     /* 0 when unsplit, else index | (count << 16).  An unsplit job of the 256 x 256 class may carry
+                          MUON_AMD_TILE_*_EMPTY: a half of its tile lies in the padding (whose operand rows are
+                          zero), is not multiplied and comes out as a product of zero              */
 } MuonTileJob;
 
 /* One tensor of the auxiliary Adam group. */

@@ -139,6 +139,15 @@ __device__ __forceinline__ void wait_frags_tr(u32x4 (&a)[TM], u32x2 (&b)[TN2]) {
         static_assert(TM == 2 && TN2 == 4, "wait_frags_tr: add the operand list of this wave tile");
 }
 
+// Column of the wave tile that wave `wave` of a workgroup owns (its row is wave / WGN).  Waves w and w + 4 share a SIMD: in
+// a tile of 2 x 4 wave tiles with an empty half (MUON_AMD_TILE_*_EMPTY) the second row is turned by two, so
+// that whichever half it is every SIMD keeps one wave that multiplies and one that does not.  (Full tiles are not turned:
+// waves of a SIMD that read the same rows of Q are 0.5 % faster, 32 x 4096^2 37.99 against 38.23 ms.)
+template <int WGN>
+__device__ __forceinline__ int wave_column(int wave, int job_split) {
+    return WGN == 4 && (job_split & MUON_AMD_TILE_EMPTY) ? (wave % WGN) ^ ((wave / WGN) * 2) : wave % WGN;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Epilogue helpers
 // ---------------------------------------------------------------------------------------------
@@ -274,7 +283,7 @@ __device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const
     int tid_e = threadIdx.x;
     asm volatile("" : "+v"(tid_e));            // see ns_epilogue_strips
     const int lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wm = wave / WGN, wn = wave_column<WGN>(wave, job.split);
     const int lr = lane & 31, g = lane >> 5;
     const int row0 = job.i0 + wm * WM, col0 = job.j0 + wn * WN;
     const uint32_t stage_lds = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
@@ -327,7 +336,7 @@ __device__ __forceinline__ void ns_epilogue_strips(f32x16 (&acc)[TM][TN], const 
     int tid_e = threadIdx.x;
     asm volatile("" : "+v"(tid_e));
     const int lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wm = wave / WGN, wn = wave_column<WGN>(wave, job.split);
     const int lr = lane & 31, g = lane >> 5;
     const int row0 = job.i0 + wm * WM, col0 = job.j0 + wn * WN;   // origin of this wave's sub-tile
     // X is the parameter itself for a wide parameter and its transpose for a tall one
@@ -491,6 +500,7 @@ struct GemmCfg {
     static constexpr int BM = BT_, BN = BT_, WGM = WGM_, WGN = WGN_, MINB = MINB_, NHALF = NHALF_;
     static constexpr int NW = WGM * WGN, NT = NW * 64;
     static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
+    static constexpr bool SKIP_EMPTY = BT_ >= 256;    // jobs may leave out a half of their tile
     static constexpr bool ROW_SUMS = WN == 64;        // row sums go to slots of 64 columns, one per wave tile
     static constexpr int HALF_BYTES = BT_ * ROW_BYTES;
     static constexpr int DPH = BT_ / 8 / NW;          // DMA instructions (8 rows each) per wave per half
@@ -555,7 +565,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     int tid_l = tid;                                                                           \
     asm volatile("" : "+v"(tid_l));                                                            \
     const int lane = tid_l & 63, wave = __builtin_amdgcn_readfirstlane(tid_l >> 6);            \
-    const int wm = wave / WGN, wn = wave % WGN;                                                \
+    const int wm = wave / WGN, wn = wave_column<WGN>(wave, job.split);                         \
     const int gchunk = (lane & 7) ^ (((wave & 1) << 2) | (lane >> 4));                         \
     const uint32_t dst0 = lds_base + wave * 1024
     // k-major Q: piece (j*NW + wave) of the half-stage is 1024 / ROWQ whole k-rows; lane -> k-row
@@ -792,6 +802,41 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         int sp = 0, sq = 1;                 // ring slots of the P and Q halves of block kb
         int kb = 0;
+        // A tile at the edge of a matrix may have nothing but padding in its second half of rows or columns (1600 rows end
+        // 64 rows into a seventh tile of 256).  The waves there fetch their share of the operands and keep the
+        // barriers, but leave the matrix pipes to the others: such a tile takes about half the time.
+        bool empty = false;
+        if constexpr (Cfg::SKIP_EMPTY)
+            empty = ((job.split & MUON_AMD_TILE_ROWS_EMPTY) && wm * WM >= Cfg::BM / 2) ||
+                    ((job.split & MUON_AMD_TILE_COLS_EMPTY) && wn * WN >= Cfg::BN / 2);
+        if (Cfg::SKIP_EMPTY && empty) {
+#define NS_EMPTY_KBLOCK(MORE_)                                                                  \
+    do {                                                                                       \
+        if (kb > 0) {                                                                          \
+            _Pragma("unroll") for (int jj = DPK; jj < 2 * DPH; ++jj)                           \
+                if ((MORE_) == RING || ((MORE_) == RING - 1 && jj < DPH)) NS_PAIR_DMA(jj);     \
+        }                                                                                      \
+        if ((MORE_) > 0) {                                                                     \
+            NS_WAIT_VMCNT(((MORE_) == RING ? NHALF - 4 : (MORE_) > 0 ? 2 * (MORE_) - 2 : 0) * DPH); \
+            __builtin_amdgcn_s_barrier();                                                      \
+            const int h0 = 2 * kb + NHALF;                                                     \
+            ddst[0] = dst0 + sp * HALF_BYTES;                                                  \
+            ddst[1] = dst0 + sq * HALF_BYTES;                                                  \
+            dk[0] = static_cast<uint32_t>(h0 >> 1) * dstep[0];                                 \
+            dk[1] = static_cast<uint32_t>((h0 + 1) >> 1) * dstep[1];                           \
+        }                                                                                      \
+        if ((MORE_) == RING) {                                                                 \
+            _Pragma("unroll") for (int jj = 0; jj < DPK; ++jj) NS_PAIR_DMA(jj);                \
+        }                                                                                      \
+        sp += 2; sp = sp >= NHALF ? sp - NHALF : sp;                                           \
+        sq += 2; sq = sq >= NHALF ? sq - NHALF : sq;                                           \
+    } while (0)
+            static_assert(!Cfg::SKIP_EMPTY || RING == 2, "one copy of the block for each of the last RING");
+            for (; kb < nk - RING; ++kb) NS_EMPTY_KBLOCK(RING);
+            if (nk - kb == 2) { NS_EMPTY_KBLOCK(1); ++kb; }
+            NS_EMPTY_KBLOCK(0);
+#undef NS_EMPTY_KBLOCK
+        } else {
         for (; kb < nk - RING; ++kb) NS_KBLOCK(RING);
         if constexpr (RING > 3) {
             if (nk - kb == 4) { NS_KBLOCK(3); ++kb; }
@@ -801,6 +846,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
         }
         if (nk - kb == 2) { NS_KBLOCK(1); ++kb; }
         NS_KBLOCK(0);
+        }
         static_assert(RING >= 2 && RING <= 4, "one copy of the block for each of the last RING");
 #undef NS_KBLOCK
 #undef NS_PAIR_DMA
@@ -1215,7 +1261,8 @@ int muon_amd_validate_gemm(const MuonGemmDesc* descs, int ndesc, const MuonTileJ
                      "job %d: K range %d..%d of %d", j, t.k0, t.k1, d.K);
         const int count = t.split >> 16, idx = t.split & 0xffff;
         if (count <= 1) {
-            MUON_REQUIRE(t.split == 0 && t.k0 == 0 && t.k1 == d.K, "job %d: an unsplit job covers all of K", j);
+            MUON_REQUIRE((t.split & ~MUON_AMD_TILE_EMPTY) == 0 && t.k0 == 0 && t.k1 == d.K, "job %d: an unsplit job covers all of K", j);
+            MUON_REQUIRE(t.split == 0 || TR >= 256, "job %d: tile class %d does not leave out halves of a tile", j, tile_class);
         } else {
             MUON_REQUIRE(kTileClasses[tile_class].split_k, "job %d: tile class %d does not split reductions", j, tile_class);
             MUON_REQUIRE(idx < count && t.part_base >= 0 && t.part_base + count <= split_slots,

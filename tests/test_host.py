@@ -812,3 +812,11 @@ def test_build_refuses_store_data_swapped_behind_the_store():
                 check_store_data(f"{store}\t{swap} {args}\n")
         assert check_store_data(f"{store}\ts_nop 1\n\t{swap} v9, v171\n") == 1
         assert check_store_data(f"{store}\t{swap} v9, v174\n") == 1
+
+
+def test_jobs_name_the_empty_halves():
+    chunk = plan.plan_chunks([(1600, 6500)], 5, True, 1 << 33)[0]
+    full = chunk.full_jobs
+    assert chunk.update_class == 1 and len(full) == 7 * 26
+    rows, cols = full["i0"] == 1536, full["j0"] == 6400          # 64 rows and 100 columns of data in the last tiles
+    assert (full["split"] == rows * plan.TILE_ROWS_EMPTY + cols * plan.TILE_COLS_EMPTY).all()
