@@ -271,42 +271,42 @@ __device__ __forceinline__ void apply_chunk8(const ApplyArgs& ap, int prow, int 
 // The addend: the lane that owns row (a*32 + lr) needs columns b*32 + 8q + 4g .. +4 of it.  Fetched
 // that way from global memory, every load instruction would touch 32 different rows for 16 bytes
 // each and the address pipe would take longer than the whole rest of the epilogue.  So the wave's
-// WM x WN piece of D is first streamed into its staging area `stage_d` (WM rows of 2 WN bytes) by
-// the DMA path, one instruction per 1 KiB of full rows (chunks XOR-swizzled as in the operand ring), and
-// the row-owning 8-byte pieces are read from LDS.  All of them are in registers when this returns:
-// before any store of the sub-tile (D may alias C: in-place a*X + B*X).
-template <int WGN, int WM, int WN, int TM, int TN>
-__device__ __forceinline__ void ns_epilogue_addend(u32x2 (&dv)[TM][TN][4], const MuonGemmDesc& d,
-                                                   const MuonTileJob& job, const char* stage_d) {
+// WM x WN piece of D is first streamed into LDS (rows of 2 WN bytes) by the DMA path, one instruction
+// per 1 KiB of full rows (chunks XOR-swizzled as in the operand ring), and the row-owning 8-byte pieces are read
+// from there.  A strip of 32 rows of every wave takes one slot of the operand ring (a half-stage).
+template <int WGN, int WM, int WN>
+__device__ __forceinline__ void ns_addend_fetch(const MuonGemmDesc& d, const MuonTileJob& job, int strip, uint32_t slot_lds) {
     constexpr int CPR = WN / 8, RPI = 64 / CPR;         // chunks per row, rows per instruction
-    static_assert(WM % RPI == 0, "addend staging in whole instructions");
+    static_assert(32 % RPI == 0, "addend staging in whole instructions");
     int tid_e = threadIdx.x;
     asm volatile("" : "+v"(tid_e));            // see ns_epilogue_strips
     const int lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
     const int wm = wave / WGN, wn = wave_column<WGN>(wave, job.split);
-    const int lr = lane & 31, g = lane >> 5;
-    const int row0 = job.i0 + wm * WM, col0 = job.j0 + wn * WN;
-    const uint32_t stage_lds = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
-        reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)stage_d)));
+    const int row0 = job.i0 + wm * WM + strip * 32, col0 = job.j0 + wn * WN;
     const u32x4 rsrc_d = dma_resource(d.D);
 #pragma unroll
-    for (int j = 0; j < WM / RPI; ++j) {
+    for (int j = 0; j < 32 / RPI; ++j) {
         const int rr = j * RPI + lane / CPR;
         const int lc = (lane % CPR) ^ ((rr >> 1) & (CPR - 1));    // logical 16-byte chunk this lane fetches
         dma16(rsrc_d, static_cast<uint32_t>((static_cast<size_t>(row0 + rr) * d.ldd + col0 + lc * 8) * 2), 0u,
-              stage_lds + j * 1024);
+              slot_lds + wave * (32 * WN * 2) + j * 1024);
     }
-    NS_WAIT_VMCNT(0);
+}
+
+template <int WN, int TN>
+__device__ __forceinline__ void ns_addend_read(u32x2 (&dv)[TN][4], const char* slot) {
+    constexpr int CPR = WN / 8;
+    int tid_e = threadIdx.x;
+    asm volatile("" : "+v"(tid_e));
+    const int lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
+    const int lr = lane & 31, g = lane >> 5;
+    const char* const stage_d = slot + wave * (32 * WN * 2);
 #pragma unroll
-    for (int a = 0; a < TM; ++a) {
-        const int rr = a * 32 + lr;
+    for (int b = 0; b < TN; ++b)
 #pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                dv[a][b][q] = *reinterpret_cast<const u32x2*>(
-                    stage_d + rr * WN * 2 + (((b * 4 + q) ^ ((rr >> 1) & (CPR - 1))) * 16) + g * 8);
-    }
+        for (int q = 0; q < 4; ++q)
+            dv[b][q] = *reinterpret_cast<const u32x2*>(
+                stage_d + lr * WN * 2 + (((b * 4 + q) ^ ((lr >> 1) & (CPR - 1))) * 16) + g * 8);
 }
 
 // Wave-private staging bytes of the result strips: 32 rows of WN columns, twice (the scaled copy, or
@@ -506,15 +506,16 @@ struct GemmCfg {
     static constexpr int DPH = BT_ / 8 / NW;          // DMA instructions (8 rows each) per wave per half
     static constexpr size_t RING_BYTES = static_cast<size_t>(NHALF) * HALF_BYTES;
     static constexpr size_t LDS_BYTES = RING_BYTES;
-    // After the main loop the ring is free.  The addend pieces (WM rows of 128 bytes per wave) are
-    // staged at its start; once they are in registers, the first NPRE half-stages of the
+    // While the last k-block is multiplied, and after the main loop, the addend is staged in the slots of the
+    // ring that are free; once it is in registers, the first NPRE half-stages of the
     // workgroup's next job are fetched into slots 0 .. NPRE-1 while the result strips are staged
     // behind them.
     static constexpr int NPRE = 3;
-    static constexpr size_t ADDEND_BYTES = static_cast<size_t>(NW) * WM * WN * 2;
+    static_assert(NW * 32 * WN * 2 == HALF_BYTES, "a strip of the addend takes one slot of the ring");
+    static constexpr int EARLY = TM < NHALF - 2 ? TM : NHALF - 2;    // strips that fit beside the last k-block
     static constexpr size_t STRIP_OFFSET = static_cast<size_t>(NPRE) * HALF_BYTES;
     static constexpr size_t STRIP_BYTES = strip_stage_bytes(WN);
-    static_assert(ADDEND_BYTES <= RING_BYTES, "addend staging");
+    static_assert(TM <= NHALF - 1, "addend staging");
     static_assert(STRIP_OFFSET + NW * STRIP_BYTES <= RING_BYTES, "strip staging behind the prefetched halves");
     static_assert(BT_ % (8 * NW) == 0, "DMA tiling");
     static_assert((NHALF - 2) * DPH < 64 && NHALF >= 5, "vmcnt immediate / ring depth");
@@ -802,6 +803,25 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         int sp = 0, sq = 1;                 // ring slots of the P and Q halves of block kb
         int kb = 0;
+        // The addend is requested ahead of the last k-block, whose two slots are then the only ones in use (the strips of a
+        // 256 x 256 tile need one more, see below).  A tile whose reduction is shared does not know yet whether
+        // it will be written, and its ticket goes through the ring.
+        const bool has_d = APPLY || (!ROWSUM && d.D != nullptr);
+        const bool d_early = has_d && !(Cfg::SPLIT_K && (job.split >> 16) > 1);
+        int last_sq = 0;                    // ring slot of the Q half of the last block: strip a goes to the a+1st after it
+#define NS_ADDEND_SLOT(a_) ((last_sq + 1 + (a_)) >= NHALF ? last_sq + 1 + (a_) - NHALF : last_sq + 1 + (a_))
+#define NS_ADDEND_FETCH(FROM_, TO_)                                                             \
+    do {                                                                                       \
+        _Pragma("unroll") for (int a_ = (FROM_); a_ < (TO_); ++a_)                             \
+            ns_addend_fetch<WGN, WM, WN>(d, job, a_, lds_base + NS_ADDEND_SLOT(a_) * HALF_BYTES); \
+    } while (0)
+#define NS_ADDEND_EARLY()                                                                       \
+    do {                                                                                       \
+        last_sq = sq;                                                                          \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+        if (d_early) NS_ADDEND_FETCH(0, Cfg::EARLY);                                           \
+        __builtin_amdgcn_sched_barrier(0);                                                     \
+    } while (0)
         // A tile at the edge of a matrix may have nothing but padding in its second half of rows or columns (1600 rows end
         // 64 rows into a seventh tile of 256).  The waves there fetch their share of the operands and keep the
         // barriers, but leave the matrix pipes to the others: such a tile takes about half the time.
@@ -834,6 +854,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             static_assert(!Cfg::SKIP_EMPTY || RING == 2, "one copy of the block for each of the last RING");
             for (; kb < nk - RING; ++kb) NS_EMPTY_KBLOCK(RING);
             if (nk - kb == 2) { NS_EMPTY_KBLOCK(1); ++kb; }
+            NS_ADDEND_EARLY();
             NS_EMPTY_KBLOCK(0);
 #undef NS_EMPTY_KBLOCK
         } else {
@@ -845,6 +866,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             if (nk - kb == 3) { NS_KBLOCK(2); ++kb; }
         }
         if (nk - kb == 2) { NS_KBLOCK(1); ++kb; }
+        NS_ADDEND_EARLY();
         NS_KBLOCK(0);
         }
         static_assert(RING >= 2 && RING <= 4, "one copy of the block for each of the last RING");
@@ -929,11 +951,27 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             }
         }
 
-        // ---- epilogue, first part: the addend into registers (staged at the start of the ring) ----
-        const bool has_d = APPLY || (!ROWSUM && d.D != nullptr);
+        // ---- epilogue, first part: the addend into registers.  All of it is there before any store of the sub-tile (D may
+        //      alias C: in-place a*X + B*X).  Requested only here, it kept every wave waiting for 2.5 us of the 29 us of a 256 x 256
+        //      update tile over 12 k-blocks, 1.2 us of the 18 us of a 128 x 128 polynomial tile. ----------------------
         u32x2 dv[TM][TN][4];
         if (write_tile && has_d) {
-            ns_epilogue_addend<WGN, WM, WN, TM, TN>(dv, d, job, reinterpret_cast<const char*>(lds) + wave * (WM * WN * 2));
+            if (!d_early) NS_ADDEND_FETCH(0, Cfg::EARLY);
+            if constexpr (TM > Cfg::EARLY) NS_ADDEND_FETCH(Cfg::EARLY, TM);
+            constexpr int CPR = WN / 8;                     // (32 rows of CPR chunks: CPR / 2 instructions a strip)
+            NS_WAIT_VMCNT((TM - Cfg::EARLY) * (CPR / 2));
+#pragma unroll
+            for (int a = 0; a < Cfg::EARLY; ++a)
+                ns_addend_read<WN, TN>(dv[a], reinterpret_cast<const char*>(lds) + NS_ADDEND_SLOT(a) * HALF_BYTES);
+            if constexpr (TM > Cfg::EARLY) {
+                NS_WAIT_VMCNT(0);
+#pragma unroll
+                for (int a = Cfg::EARLY; a < TM; ++a)
+                    ns_addend_read<WN, TN>(dv[a], reinterpret_cast<const char*>(lds) + NS_ADDEND_SLOT(a) * HALF_BYTES);
+            }
+#undef NS_ADDEND_EARLY
+#undef NS_ADDEND_FETCH
+#undef NS_ADDEND_SLOT
         } else {
             // defined on every path, so that nothing of it is carried around the job loop in registers
 #pragma unroll
