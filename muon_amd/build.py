@@ -25,9 +25,11 @@ FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     # hipcc -O3 must not form packed-fp32 instructions on this target
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # the first kernel arguments arrive in scalar registers with the dispatch instead of through a load of each wave's own
-    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
+# The GEMM kernels' arguments arrive in scalar registers with the dispatch instead of through a load of each wave's own: 0.2 us
+# for each of the 15 dependent launches of a small matrix (768 x 3072: 174.7 -> 170.9 us).  A step of one launch gains nothing
+# (Adam over 50257 x 768 169.0 -> 170.4 us), so the other sources are built without it.
+SOURCE_FLAGS = {"ns_gemm.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
 
 
 _VREG = re.compile(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b")
@@ -133,18 +135,26 @@ def check_store_data(asm_text: str) -> int:
 def build(verbose: bool = True, check: bool = True) -> str:
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     tmp = OUT + ".tmp"
-    cmd = [hipcc, *FLAGS, *[os.path.join(CSRC, s) for s in SOURCES], "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        sys.stderr.write(proc.stdout + proc.stderr)
-        raise RuntimeError("hipcc failed building libmuon_amd.so")
+    with tempfile.TemporaryDirectory() as d:
+        objects = [os.path.join(d, src + ".o") for src in SOURCES]
+        compile_flags = [f for f in FLAGS if f != "-shared"]
+        cmds = [[hipcc, *compile_flags, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
+                for src, obj in zip(SOURCES, objects)]
+        if verbose:
+            print("\n".join(" ".join(c) for c in cmds), flush=True)
+        procs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for c in cmds]
+        outputs = [p.communicate()[0] for p in procs]
+        if not any(p.returncode for p in procs):
+            link = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objects, "-o", tmp], capture_output=True, text=True)
+            procs, outputs = [link], [link.stdout + link.stderr]
+        if any(p.returncode for p in procs):
+            sys.stderr.write("".join(outputs))
+            raise RuntimeError("hipcc failed building libmuon_amd.so")
     if check:
         with tempfile.TemporaryDirectory() as d:
             listing = os.path.join(d, "ns_gemm.s")
             flags = [f for f in FLAGS if f not in ("-shared", "-fPIC")]
-            cmd = [hipcc, *flags, "-S", "--cuda-device-only", os.path.join(CSRC, "ns_gemm.hip"), "-o", listing]
+            cmd = [hipcc, *flags, *SOURCE_FLAGS["ns_gemm.hip"], "-S", "--cuda-device-only", os.path.join(CSRC, "ns_gemm.hip"), "-o", listing]
             proc = subprocess.run(cmd, capture_output=True, text=True)
             if proc.returncode != 0:
                 sys.stderr.write(proc.stdout + proc.stderr)
