@@ -151,7 +151,7 @@ def _symmetric_plan(batch: int, M: int, K: int, addend: bool):
     own = _plan.tile_class_for(M)
     kp = _plan._round_up(K, _plan.GEMM_BK)
     # X X^T of a short, very wide matrix: a few tiles with very long reductions, which are split
-    nsplit = 1 if addend or own != 0 else _plan.split_factor(_plan._round_up(M, 128), kp)
+    nsplit = 1 if addend else _plan.split_factor(_plan._round_up(M, 128), kp, own)
     tile_class = _launch_class("poly" if addend else "gram", own, batch, M, K)
     mp = _plan._round_up(M, _plan.pad_unit(tile_class))
     # X X^T is symmetric bit for bit.  alpha A A^T + beta A is as symmetric as A: for another A, which elements are

@@ -76,13 +76,16 @@ SPLIT_KBLOCKS_PER_JOB = _SPLIT[2]       # ... into jobs of about this many k-blo
 SPLIT_MAX = _SPLIT[3]
 
 
-def split_factor(mp: int, kdim: int) -> int:
+def split_factor(mp: int, kdim: int, own_class: int = 0) -> int:
     """Into how many jobs each tile of X X^T is split along its reduction.  The rule looks at the
     matrix alone, so its result is the same bits whatever else shares the launch: a short, very
     wide matrix has a handful of tiles with thousands of k-blocks each (one tile with 256 for
-    128 x 16384), which one workgroup per tile would grind through while the rest of the GPU idles."""
+    128 x 16384), which one workgroup per tile would grind through while the rest of the GPU idles.
+    Matrices whose own class (tile_class_for) is the 256 x 256 one, which cannot split, are not split
+    in smaller tiles either: which of the two a launch takes depends on what shares it.  (They are longer
+    than SPLIT_MAX_M unless a knob says otherwise.)"""
     kblocks = kdim // GEMM_BK
-    if mp > SPLIT_MAX_M or kblocks < SPLIT_MIN_KBLOCKS:
+    if own_class == 1 or mp > SPLIT_MAX_M or kblocks < SPLIT_MIN_KBLOCKS:
         return 1
     return max(1, min(SPLIT_MAX, kblocks // SPLIT_KBLOCKS_PER_JOB))
 
@@ -176,7 +179,7 @@ def matrix_scratch_bytes(rows: int, cols: int, tile_class: int, aol: bool) -> in
     m, n = min(rows, cols), max(rows, cols)
     mp, np_ = _round_up(m, unit), _round_up(n, unit)
     total = _round_up(-(-rows * cols // EW_BLOCK_ELEMS) * 4, _ALIGN) + _ALIGN
-    nsplit = split_factor(mp, np_)
+    nsplit = split_factor(mp, np_, tile_class)
     if nsplit > 1:
         tiles = (mp // tr) * (mp // tr + 1) // 2 * (tr // tc) if tr != tc else (mp // tr) * (mp // tr + 1) // 2
         total += _round_up(tiles * nsplit * tr * tc * 4, _ALIGN)
@@ -342,9 +345,9 @@ LAUNCH_CLASS = os.environ.get("MUON_AMD_LAUNCH_CLASS", "auto")      # measuremen
 SPLIT_HANDOVER_US = 8.0
 
 
-def launch_time_us(kind: str, tile_class: int, runs) -> float:
-    """Estimated time of a product over `runs` of (layout, matrices of its shape) in tiles of one class (see
-    LAUNCH_COST): one job per CU
+def launch_time_us(kind: str, tile_class: int, runs, own_class: int = 0) -> float:
+    """Estimated time of a product over `runs` of (layout, matrices of its shape), matrices of class `own_class`, in
+    tiles of one class (see LAUNCH_COST): one job per CU
     as long as there are fewer jobs than CUs, whose k-blocks take longer the more CUs are busy; beyond
     that the jobs of a CU in turn, the last partly filled round counted half."""
     T, cost = TILE_DIMS[tile_class][0], LAUNCH_COST[tile_class]
@@ -353,7 +356,7 @@ def launch_time_us(kind: str, tile_class: int, runs) -> float:
         mt, nt = -(-lay.mk // T), -(-lay.nk // T)
         kb, ns = (lay.nk if kind == "gram" else lay.mk) // GEMM_BK, 1
         if kind == "gram":
-            ns = split_factor(lay.mp, lay.np_)
+            ns = split_factor(lay.mp, lay.np_, own_class)
         n = (mt * nt if kind == "update" else mt * (mt + 1) // 2) * ns * count
         split = max(split, ns - 1)
         jobs += n
@@ -374,7 +377,7 @@ def launch_class(kind: str, tile_class: int, runs) -> int:
         want = int(LAUNCH_CLASS.split(",")[("gram", "poly", "update").index(kind)])
         return want if TILE_DIMS[want][0] <= TILE_DIMS[tile_class][0] else tile_class
     classes = [c for c in (1, 0, 2) if TILE_DIMS[c][0] <= TILE_DIMS[tile_class][0]]
-    return min(classes, key=lambda c: launch_time_us(kind, c, runs))
+    return min(classes, key=lambda c: launch_time_us(kind, c, runs, tile_class))
 
 
 class ChunkPlan:
@@ -446,7 +449,7 @@ class ChunkPlan:
         # 128 x 128 class (see update_class_for).
         self.split_slots = sum(count * (lay.mp // self.tile_rows) * (lay.mp // self.tile_rows + 1) // 2 * ns
                                for _, (lay, count) in self._runs
-                               if (ns := split_factor(lay.mp, lay.np_)) > 1)
+                               if (ns := split_factor(lay.mp, lay.np_, tile_class)) > 1)
         self.update_class = update_class_for(tile_class, self.layouts)
         # every tile of the m x m polynomial (no mirrored store): the first iteration of "aol4_rows",
         # whose Gram matrix is not symmetric after the row-only rescaling
@@ -488,7 +491,7 @@ class ChunkPlan:
             nt = -(-(rows if (sym or square) else cols) // TC)
             ti, tj = _tile_order(mt, nt, sym, ratio, si, sj, direct)
             kdim = lay.nk if reduce_over_n else lay.mk
-            nsplit = split_factor(lay.mp, lay.np_) if reduce_over_n else 1
+            nsplit = split_factor(lay.mp, lay.np_, self.tile_class) if reduce_over_n else 1
             n = len(ti) * nsplit
             # the jobs of one matrix, then those of `count` matrices of its shape (columns as in MuonTileJob)
             one = np.zeros((n, 8), dtype=np.int32)
@@ -497,14 +500,14 @@ class ChunkPlan:
                 one[:, 3] = np.repeat(np.where(ti == tj // ratio, 1, np.where(ti // direct == tj // ratio // direct, 2, 0)), nsplit)
             if nsplit == 1:
                 one[:, 5] = kdim
+                if tile_class == 1:
+                    one[:, 7] = empty_halves(one[:, 1], one[:, 2], lay.mk, lay.mk if (sym or square) else lay.nk)
             else:      # k-blocks dealt as evenly as 64-wide blocks allow; one group of slots per tile
                 edges = (np.arange(nsplit + 1) * (kdim // GEMM_BK) // nsplit) * GEMM_BK
                 idx = np.tile(np.arange(nsplit), len(ti))
                 one[:, 4], one[:, 5] = edges[idx], edges[idx + 1]
                 one[:, 6] = np.repeat(np.arange(len(ti)) * nsplit, nsplit)
                 one[:, 7] = idx | (nsplit << 16)
-            if tile_class == 1:
-                one[:, 7] = empty_halves(one[:, 1], one[:, 2], lay.mk, lay.mk if (sym or square) else lay.nk)
             part = np.tile(one, (count, 1))
             part[:, 0] = np.repeat(np.arange(k, k + count), n)
             if nsplit > 1:
@@ -783,7 +786,7 @@ def _chunk_time_us(mats, tile_class: int) -> tuple[float, float]:
             if kind == "update":
                 counts.append(mt * (np_ // TT)); costs.append(kbm)
             else:
-                ns = split_factor(mp, np_) if kind == "syrk" else 1
+                ns = split_factor(mp, np_, tile_class) if kind == "syrk" else 1
                 counts.append(mt * (mt + 1) // 2 * ns); costs.append((kbn if kind == "syrk" else kbm) // ns)
         us = LAUNCH_COST[tc]
         cost = np.repeat(np.asarray(costs, dtype=np.float64) * us["shared"] + us["fixed_shared"], counts)

@@ -820,3 +820,26 @@ def test_jobs_name_the_empty_halves():
     assert chunk.update_class == 1 and len(full) == 7 * 26
     rows, cols = full["i0"] == 1536, full["j0"] == 6400          # 64 rows and 100 columns of data in the last tiles
     assert (full["split"] == rows * plan.TILE_ROWS_EMPTY + cols * plan.TILE_COLS_EMPTY).all()
+
+
+@pytest.mark.parametrize("min_m,launch_class", [(256, "1,1,1"), (256, "auto"), (256, "0,0,0"), (1, "2,2,2")])
+def test_matrices_of_the_256_class_are_never_split(min_m, launch_class, monkeypatch):
+    """The 256 x 256 class does not split reductions.  With the knob that lets shorter matrices into it, a matrix that
+    would be split in the 128 x 128 class is not, whatever tiles its launches take, and every job covers all of K."""
+    lib = _lib.load()
+    monkeypatch.setattr(plan, "BIG_TILE_MIN_M", min_m)
+    monkeypatch.setattr(plan, "LAUNCH_CLASS", launch_class)
+    for shapes in ([(300, 4096)], [(512, 16384), (300, 4096), (290, 2048)]):
+        assert plan.split_factor(plan._round_up(300, 128), 4096) > 1
+        for variant in ("ns5", "aol4"):
+            c, = plan.plan_chunks(shapes, 5, True, 1 << 33, variant)
+            assert c.tile_class == 1 and c.split_slots == 0
+            g = c.gemm_descs(1 << 20)
+            for kind, ph in (("gram", plan.PH_SYRK), ("poly", plan.PH_POLY), ("update", plan.PH_UPD_EVEN)):
+                ln, descs = c.launches[kind], g[ph].copy()
+                descs["rowsum"] = 0
+                rc = lib.muon_amd_validate_gemm(_lib.host_ptr(descs), c.nmat, _lib.host_ptr(ln.jobs), len(ln.jobs),
+                                                ln.tile_class, ln.split_slots)
+                assert rc == 0, (kind, lib.muon_amd_last_error())
+                assert ln.split_slots == 0 and (ln.jobs["split"] >> 16 == 0).all()
+                assert (ln.jobs["k0"] == 0).all() and (ln.jobs["k1"] == descs["K"][ln.jobs["desc"]]).all()
