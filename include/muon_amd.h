@@ -139,8 +139,11 @@ typedef struct MuonTileJob {
     int32_t k0, k1;    /* reduction range of this job, multiples of 64; 0 and K when unsplit */
     int32_t part_base; /* first slot of the tile's split group (also its counter); unused when unsplit */
     int32_t split;     /* 0 when unsplit, else index | (count << 16).  An unsplit job of the 256 x 256 class may carry
-                          MUON_AMD_TILE_*_EMPTY: a half of its tile lies in the padding (whose operand rows are
-                          zero), is not multiplied and comes out as a product of zero              */
+                          MUON_AMD_TILE_*_EMPTY when the second half of its tile's rows (columns) holds no data: that
+                          half is not multiplied, its accumulators are zero whatever the operands hold there
+                          (zero, or what launches of smaller tiles left: rows and columns beyond the last
+                          k-block of data reach no reduction).  How far the data goes is the caller's to say: the library refuses
+                          the flags before the last tile row (column) of the output                 */
 } MuonTileJob;
 
 /* One tensor of the auxiliary Adam group. */

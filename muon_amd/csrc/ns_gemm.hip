@@ -1301,6 +1301,11 @@ int muon_amd_validate_gemm(const MuonGemmDesc* descs, int ndesc, const MuonTileJ
         if (count <= 1) {
             MUON_REQUIRE((t.split & ~MUON_AMD_TILE_EMPTY) == 0 && t.k0 == 0 && t.k1 == d.K, "job %d: an unsplit job covers all of K", j);
             MUON_REQUIRE(t.split == 0 || TR >= 256, "job %d: tile class %d does not leave out halves of a tile", j, tile_class);
+            // (the padding is less than a tile: an empty half before the last tile row or column is a mistake)
+            MUON_REQUIRE((!(t.split & MUON_AMD_TILE_ROWS_EMPTY) || t.i0 + TR == d.rows) &&
+                             (!(t.split & MUON_AMD_TILE_COLS_EMPTY) || t.j0 + TC == d.colsn),
+                         "job %d: tile (%d,%d) of %dx%d cannot have a half in the padding (flags %d)", j, t.i0, t.j0, d.rows, d.colsn,
+                         t.split);
         } else {
             MUON_REQUIRE(kTileClasses[tile_class].split_k, "job %d: tile class %d does not split reductions", j, tile_class);
             MUON_REQUIRE(idx < count && t.part_base >= 0 && t.part_base + count <= split_slots,

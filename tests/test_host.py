@@ -843,3 +843,45 @@ def test_matrices_of_the_256_class_are_never_split(min_m, launch_class, monkeypa
                 assert rc == 0, (kind, lib.muon_amd_last_error())
                 assert ln.split_slots == 0 and (ln.jobs["split"] >> 16 == 0).all()
                 assert (ln.jobs["k0"] == 0).all() and (ln.jobs["k1"] == descs["K"][ln.jobs["desc"]]).all()
+
+
+def test_validator_takes_empty_halves_only_where_padding_can_be():
+    """A wrong MUON_AMD_TILE_*_EMPTY flag leaves half a tile of the result unmultiplied: it is refused but for the last
+    tile row (column) of an output of the 256 x 256 class, the only one that can end in padding."""
+    lib = _lib.load()
+    chunk, = plan.plan_chunks([(1600, 6500)], 5, True, 1 << 33)
+
+    def refused(ph, jobs, tile_class=1, slots=0):
+        d = chunk.gemm_descs(1 << 20)[ph].copy()
+        d["rowsum"] = 0
+        rc = lib.muon_amd_validate_gemm(_lib.host_ptr(d), 1, _lib.host_ptr(jobs), len(jobs), tile_class, slots)
+        assert rc in (0, -1)
+        return rc == -1 and lib.muon_amd_last_error().decode()
+
+    lay, = chunk.layouts
+    for ph, jobs in ((plan.PH_SYRK, chunk.syrk_jobs), (plan.PH_POLY, chunk.sym_jobs), (plan.PH_UPD_EVEN, chunk.full_jobs)):
+        assert (jobs["split"] == plan.TILE_ROWS_EMPTY | plan.TILE_COLS_EMPTY).any() and not refused(ph, jobs)
+        cols = lay.np_ if jobs is chunk.full_jobs else lay.mp
+        last = np.where(jobs["i0"] + 256 == lay.mp, plan.TILE_ROWS_EMPTY, 0) | np.where(jobs["j0"] + 256 == cols, plan.TILE_COLS_EMPTY, 0)
+        for k in range(len(jobs)):
+            for flags in range(-1, 9):
+                one = jobs[k:k + 1].copy()
+                one["split"] = flags
+                ok = 0 <= flags <= 3 and flags & ~last[k] == 0
+                assert bool(refused(ph, one)) != ok, (ph, k, flags)
+        everywhere = jobs.copy()
+        everywhere["split"] = plan.TILE_ROWS_EMPTY | plan.TILE_COLS_EMPTY
+        assert "padding" in refused(ph, everywhere)
+        for flags in (0, 1, 2, 3):                       # no split reductions in this class, flags or not
+            one = jobs[:1].copy()
+            one["split"] = flags | 2 << 16
+            assert "does not split" in refused(ph, one, slots=2)
+    from muon_amd import ops
+    for tile_class in (0, 2):                            # the other classes multiply every tile whole
+        T = plan.TILE_DIMS[tile_class][0]
+        jobs = ops._product_jobs(tile_class, 1, lay.mp, lay.mp, lay.mk, True)
+        assert not refused(plan.PH_POLY, jobs, tile_class)
+        for flags in (1, 2, 3):
+            one = jobs[(jobs["i0"] == lay.mp - T) & (jobs["j0"] == lay.mp - T)].copy()
+            one["split"] = flags
+            assert "does not leave out" in refused(plan.PH_POLY, one, tile_class)
