@@ -27,8 +27,9 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 # The GEMM kernels' arguments arrive in scalar registers with the dispatch instead of through a load of each wave's own: 0.2 us
-# for each of the 15 dependent launches of a small matrix (768 x 3072: 174.7 -> 170.9 us).  A step of one launch gains nothing
-# (Adam over 50257 x 768 169.0 -> 170.4 us), so the other sources are built without it.
+# for each of the 15 dependent launches of a small matrix (768 x 3072: 174.8 -> 171.2 us, runs of one build differ by 0.1 %).  In a
+# step of one launch that does not show in the call (64 x 64 x 3 x 3: the kernel 37.0 -> 36.7 us, the call 47.6-48.3 -> 46.9-48.1 us
+# with runs of one build 0.3-3 % apart; Adam over 50257 x 768 171.9 -> 171.9 us), so the other sources are built without it.
 SOURCE_FLAGS = {"ns_gemm.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
 
 

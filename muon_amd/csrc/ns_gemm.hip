@@ -528,9 +528,8 @@ struct GemmCfg {
 // there are fewer jobs), and workgroup b computes jobs b, b + gridDim.x, b + 2 gridDim.x, ... of the
 // list.  Workgroups are dealt round-robin to the XCDs, so with a grid that is a multiple of 8 job j
 // still runs on XCD j % 8, in list order.  Between two jobs of a workgroup nothing waits for a
-// launch: the descriptors of the next job are read while the addend of the current one is in
-// flight, and its first NPRE half-stages stream into LDS while the epilogue of the current one
-// runs.
+// launch: once the addend of the current job is in registers the descriptors of the next one are read, and
+// its first NPRE half-stages stream into LDS while the result strips of the current one are written.
 // APPLY: the launch is the last update product of the iteration and its epilogue takes the
 // parameter step (mats[job.desc] describes the parameter of the job's matrix; `sc`, when given,
 // holds {lr, wd_factor} in device memory and overrides the by-value arguments).
@@ -824,7 +823,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
     } while (0)
         // A tile at the edge of a matrix may have nothing but padding in its second half of rows or columns (1600 rows end
         // 64 rows into a seventh tile of 256).  The waves there fetch their share of the operands and keep the
-        // barriers, but leave the matrix pipes to the others: such a tile takes about half the time.
+        // barriers, but leave the matrix pipes to the others.  What that gives is measured at plan.empty_halves.
         bool empty = false;
         if constexpr (Cfg::SKIP_EMPTY)
             empty = ((job.split & MUON_AMD_TILE_ROWS_EMPTY) && wm * WM >= Cfg::BM / 2) ||
@@ -858,16 +857,16 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
             NS_EMPTY_KBLOCK(0);
 #undef NS_EMPTY_KBLOCK
         } else {
-        for (; kb < nk - RING; ++kb) NS_KBLOCK(RING);
-        if constexpr (RING > 3) {
-            if (nk - kb == 4) { NS_KBLOCK(3); ++kb; }
-        }
-        if constexpr (RING > 2) {
-            if (nk - kb == 3) { NS_KBLOCK(2); ++kb; }
-        }
-        if (nk - kb == 2) { NS_KBLOCK(1); ++kb; }
-        NS_ADDEND_EARLY();
-        NS_KBLOCK(0);
+            for (; kb < nk - RING; ++kb) NS_KBLOCK(RING);
+            if constexpr (RING > 3) {
+                if (nk - kb == 4) { NS_KBLOCK(3); ++kb; }
+            }
+            if constexpr (RING > 2) {
+                if (nk - kb == 3) { NS_KBLOCK(2); ++kb; }
+            }
+            if (nk - kb == 2) { NS_KBLOCK(1); ++kb; }
+            NS_ADDEND_EARLY();
+            NS_KBLOCK(0);
         }
         static_assert(RING >= 2 && RING <= 4, "one copy of the block for each of the last RING");
 #undef NS_KBLOCK
@@ -953,7 +952,10 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         // ---- epilogue, first part: the addend into registers.  All of it is there before any store of the sub-tile (D may
         //      alias C: in-place a*X + B*X).  Requested only here, it kept every wave waiting for 2.5 us of the 29 us of a 256 x 256
-        //      update tile over 12 k-blocks, 1.2 us of the 18 us of a 128 x 128 polynomial tile. ----------------------
+        //      update tile over 12 k-blocks.  Part of that is gained:
+        //      update launches of 256 x 256 tiles, requested here -> ahead of the last block, two profiles each: 12 layers
+        //      of width 1024 324.7, 323.4 -> 318.8, 318.0 us, 6 of 1600 607, 610 -> 601, 598, GPT-2 145.6, 147.5 -> 142.4, 143.1.
+        //      Polynomials and tiles of 128 x 128 and 64 x 64 measure the same either way. ---------------------------------
         u32x2 dv[TM][TN][4];
         if (write_tile && has_d) {
             if (!d_early) NS_ADDEND_FETCH(0, Cfg::EARLY);
@@ -969,9 +971,6 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
                 for (int a = Cfg::EARLY; a < TM; ++a)
                     ns_addend_read<WN, TN>(dv[a], reinterpret_cast<const char*>(lds) + NS_ADDEND_SLOT(a) * HALF_BYTES);
             }
-#undef NS_ADDEND_EARLY
-#undef NS_ADDEND_FETCH
-#undef NS_ADDEND_SLOT
         } else {
             // defined on every path, so that nothing of it is carried around the job loop in registers
 #pragma unroll
@@ -982,9 +981,12 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
                     for (int q = 0; q < 4; ++q) dv[a][b][q] = u32x2{0u, 0u};
         }
 
-        // ---- the next job's first half-stages stream in while the result strips are written -----
-        // every wave holds its addend: the start of the ring is free for the next job's halves, and
-        // the part of it under the strip staging of other waves may be overwritten
+#undef NS_ADDEND_EARLY
+#undef NS_ADDEND_FETCH
+#undef NS_ADDEND_SLOT
+
+        // every wave holds its addend: the whole ring is free again, its start for the next job's halves and
+        // the rest for the strip staging
         if (write_tile && has_d) __syncthreads();
 
         // ---- the workgroup's next job: its first half-stages stream in while the result strips

@@ -39,3 +39,27 @@ def test_empty_halves_are_products_of_zero(shape, variant, monkeypatch):
     muon_amd.clear_engine_cache()
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(*outs)
+
+
+# the rows-only rescaling multiplies the polynomial over every tile, stored in one orientation; the long shapes would be split
+# (their X X^T) in the class that their sizes ask for
+ROWS_SHAPES = [s for s in SHAPES if min(s[1:]) >= 32] + [(1, 300, 4096), (2, 4160, 260)]
+
+
+@pytest.mark.parametrize("shape", ROWS_SHAPES)
+def test_empty_halves_of_the_unmirrored_polynomial(shape, monkeypatch):
+    import muon_amd
+    from muon_amd import plan
+    monkeypatch.setattr(plan, "SMALL", False)
+    monkeypatch.setattr(plan, "BIG_TILE_MIN_M", 1)
+    monkeypatch.setattr(plan, "LAUNCH_CLASS", "1,1,1")
+    torch.manual_seed(sum(shape))
+    G = torch.randn(*shape, device="cuda")
+    outs = []
+    for skip in (False, True):
+        monkeypatch.setattr(plan, "SKIP_EMPTY", skip)
+        muon_amd.clear_engine_cache()
+        outs.append(muon_amd.zeropower_via_aol4(G, rescale="rows"))
+    muon_amd.clear_engine_cache()
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(*outs)
