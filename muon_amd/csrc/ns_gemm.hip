@@ -952,10 +952,12 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void ns_gemm_kernel(
 
         // ---- epilogue, first part: the addend into registers.  All of it is there before any store of the sub-tile (D may
         //      alias C: in-place a*X + B*X).  Requested only here, it kept every wave waiting for 2.5 us of the 29 us of a 256 x 256
-        //      update tile over 12 k-blocks.  Part of that is gained:
-        //      update launches of 256 x 256 tiles, requested here -> ahead of the last block, two profiles each: 12 layers
-        //      of width 1024 324.7, 323.4 -> 318.8, 318.0 us, 6 of 1600 607, 610 -> 601, 598, GPT-2 145.6, 147.5 -> 142.4, 143.1.
-        //      Polynomials and tiles of 128 x 128 and 64 x 64 measure the same either way. ---------------------------------
+        //      update tile over 12 k-blocks.  Part of that is gained.  Requested here -> ahead of the last block:
+        //      update launches of 256 x 256 tiles, two profiles each on two GPUs: 12 layers of width 1024 324.7, 323.4 ->
+        //      318.8, 318.0 us and 317.5, 318.3 -> 313.8, 314.6; 6 of 1600 607, 610 -> 601, 598 and 608, 611 -> 598, 598;
+        //      polynomials of 64 x 64 tiles, ten matrices: 5.8, 5.8 -> 5.5, 5.5 us (1500 x 1100, whole call: 158.7 -> 156.6).
+        //      Polynomials of 256 x 256 tiles and everything in 128 x 128 measure the same either way (24 products of 768^2:
+        //      20.5, 21.4 -> 21.0, 20.1 us; updates of ten matrices 22.3, 22.2 -> 22.0, 22.0). ---------------------
         u32x2 dv[TM][TN][4];
         if (write_tile && has_d) {
             if (!d_early) NS_ADDEND_FETCH(0, Cfg::EARLY);
