@@ -312,7 +312,7 @@ def empty_halves(i0: np.ndarray, j0: np.ndarray, rows: int, cols: int) -> np.nda
     """MUON_AMD_TILE_*_EMPTY of 256 x 256 tiles at (i0, j0) of a product with `rows` x `cols` of data: the halves that
     the kernel need not multiply.  (Whole halves only: a half is what one of the two waves that share a SIMD owns.)
     Six layers of width 1600, X X^T / polynomial / update with every tile multiplied -> without the empty halves: 394 -> 369,
-    164 -> 159, 630 -> 615 us, for 12.5, 12.5 and 7.7 % fewer multiplications (the busiest CU keeps a full tile in every
+    164 -> 159, 630 -> 615 us, for 13.4, 13.4 and 7.8 % fewer multiplications (the busiest CU keeps a full tile in every
     round, and its 225, 75 and 325 k-blocks).  The list keeps its order: with the short jobs at its end, in the last, partly
     filled round, where they balance the CUs best, the launches lose their operands in L2 (366, 166 and 641 us).
     The estimates of the planner (launch_imbalance, launch_time_us) count every tile in full."""
